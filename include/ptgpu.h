@@ -118,11 +118,12 @@ int ptgpu_ctx_set_max_depth(ptgpu_ctx *ctx, int max_depth);
  * nodes).  All give the same bits. */
 int ptgpu_ctx_set_engine(ptgpu_ctx *ctx, int engine);
 /* Launch tuning, no effect on results: "regroup" (1..64, ready lanes that start a shading pass in
- * engine 3, default 16), "blocks_per_cu" (1..64, persistent workgroups per CU, default 2), "wide"
+ * engine 3, default 24), "blocks_per_cu" (1..64, persistent workgroups per CU; until it is set, the
+ * launch picks the workgroups and the pixels per wave from the frame's size), "wide"
  * (engine 3's node format: 0 binary, 1 four-wide fp32, 2 four-wide with binary16 boxes rounded
  * outward, half the bytes per node, where the tree's leaves allow it; default 2), "quad" (0..16,
- * with wide 2: when at most this many lanes of a wave are traversing, four lanes share each query,
- * one child box and leaf each; default 16, 0 off); "stack" (0..64, the smallest traversal stack
+ * with wide 2: when at most this many lanes of a wave are traversing, four or more lanes share each
+ * query, one child box each and several stack entries at a time; default 16, 0 off); "stack" (0..64, the smallest traversal stack
  * class a launch uses: the launch takes the first class (24 or 64 entries for binary nodes, 32, 48 or 64
  * for four-wide nodes) that holds both this many entries and the tree's height; default 0, the height
  * alone decides; a larger class only costs LDS, so this is a test knob for every kernel instance);

@@ -189,10 +189,11 @@ struct ptgpu_ctx {
     int cu_count = 0;
     int max_depth = 6;   // MAX_DEPTH (geom.h:32) for ptgpu_radiance_gpu
     int engine = 0;      // 0 auto, 1 megakernel (lockstep queries), 2 wavefront, 3 megakernel (per-lane states)
-    int regroup = 16;   // per-lane-state megakernel: ready lanes that trigger a shading pass
+    int regroup = 24;   // per-lane-state megakernel: ready lanes that trigger a shading pass
     int quad = 16;      // per-lane-state megakernel, binary16 nodes: traversing lanes at or below which four lanes share a query
     int batch_regroup = 32;
-    int blocks_per_cu = 2;        // single-frame renders: few waves shorten each pixel's chain
+    int blocks_per_cu = 2;        // single-frame renders
+    bool blocks_auto = true;      // until "blocks_per_cu" is set, the launch picks (launch_shape, render.hip)
     int batch_blocks_per_cu = 3;  // batched renders: throughput-bound, more waves per SIMD
     int wide = 2;        // per-lane-state megakernel: 0 binary nodes, 1 four-wide, 2 four-wide binary16 (when they exist)
     int stack_min = 0;

@@ -194,6 +194,7 @@ int ptgpu_ctx_set_tuning(ptgpu_ctx *ctx, const char *name, int value) {
     } else if (!strcmp(name, "blocks_per_cu")) {
         PT_CHECK(value >= 1 && value <= 64, PTGPU_ERR_INVALID, "blocks_per_cu %d not in [1, 64]", value);
         ctx->blocks_per_cu = value;
+        ctx->blocks_auto = false;
     } else if (!strcmp(name, "batch_blocks_per_cu")) {
         PT_CHECK(value >= 1 && value <= 64, PTGPU_ERR_INVALID, "batch_blocks_per_cu %d not in [1, 64]", value);
         ctx->batch_blocks_per_cu = value;

@@ -21,7 +21,7 @@
 #include <vector>
 
 #include "lbvh.hpp"
-#include "render_device.hpp"
+#include "walk_half.hpp"
 
 namespace ptgpu {
 
@@ -60,33 +60,12 @@ struct RenderParams {
     int njobs;
     const int2 *tiles;            // tiled launches (RadianceBoxGPU): tile origins; NULL renders the whole frame
     int tile_w, tile_h;
-    float one;                    // 1.0f, opaque to the compiler (slab_hn's mixed-precision differences)
+    int slack;                    // binary16 walk: stack entries above a depth-first walk's need (half_sparse)
+    int blocks_open;              // workgroups that stay when the camera is outside the scene's box
+    int lanes;                    // lanes of a wave that take pixels; the others help in the sparse phase
     int depth_cap;                // deepest tree the launch's stack holds (checked when acc.height_check is set)
     unsigned *status;             // the context's check words: [0] flags, [1] deepest height seen
 };
-
-// The short traversal-stack class of the binary16 walk: 36 entries per lane, so a workgroup's stack
-// takes 36 KB of LDS and four workgroups fit on a CU (three with the 48-entry class).  A walk that
-// would push past it marks kOverflow in its visit count and is finished against every primitive.
-constexpr int kStackShort = 36;
-constexpr int kStackTiny = 8;   // a test class: nearly every walk outgrows it (tuning short_stack 2)
-constexpr unsigned kOverflow = 1u << 31;
-
-// A pointer read from device memory (a batch's job table) or moved between lanes is a generic
-// pointer to the compiler, and loads through it become flat loads, which count against both memory
-// wait counters and make every wait cover all outstanding LDS and scalar accesses too.  Every buffer
-// the render kernels read or write lives in device (global) memory, so the per-lane pointers of
-// the render loop are held as global-address-space pointers (gmem): loads and stores through them
-// are global ones, also after a generic-pointer helper is inlined on from_gmem's result.  to_gmem
-// goes through the address bits: a cast would fold with from_gmem's back into the generic pointer.
-template <class T>
-using gmem = __attribute__((address_space(1))) T;
-template <class T>
-__device__ __forceinline__ gmem<T> *to_gmem(T *p) {
-    return reinterpret_cast<gmem<T> *>(reinterpret_cast<unsigned long long>(p));
-}
-template <class T>
-__device__ __forceinline__ T *from_gmem(gmem<T> *p) { return (T *)p; }
 
 // A launch recorded right after a build sized its stack for a height bound (acc.height_check set).
 // The built tree is checked before any work: a build error (flag 1) or a tree deeper than the stack
@@ -123,6 +102,22 @@ __device__ bool recorded_jobs_unfit(const RenderParams &P) {
     }
     __syncthreads();
     return s_unfit != 0;
+}
+
+// Whether the camera lies outside the scene's box (the union of the root node's child boxes).  Every thread
+// reads the same words, so whole workgroups decide alike.
+__device__ __forceinline__ bool camera_outside(const RenderParams &P) {
+    const TNode4H &r = P.acc.nodes4h[P.acc.root];
+    const float inf = __builtin_inff();
+    f3 lo = mk(inf, inf, inf), hi = mk(-inf, -inf, -inf);
+    for (int k = 0; k < 4; k++) {
+        const uint4 c = r.c[k];
+        if ((int)c.w == kEmptyRef) continue;
+        lo = mk(fminf(lo.x, half_lo(c.x)), fminf(lo.y, half_lo(c.y)), fminf(lo.z, half_lo(c.z)));
+        hi = mk(fmaxf(hi.x, half_hi(c.x)), fmaxf(hi.y, half_hi(c.y)), fmaxf(hi.z, half_hi(c.z)));
+    }
+    const f3 o = ldvec(&P.camera->orig);
+    return !(o.x >= lo.x && o.x <= hi.x && o.y >= lo.y && o.y <= hi.y && o.z >= lo.z && o.z <= hi.z);
 }
 
 // The frame pixel of claimed work item m: pixel m of the frame, or, in a tiled launch, pixel
@@ -282,28 +277,41 @@ __global__ __launch_bounds__(256) void k_render(RenderParams P) {
 // leaves it with its next query (or its pixel done).  The random numbers are drawn in the same
 // order as in k_render (shadow-ray outcomes never draw), so the bits are the same.  Needs a tree
 // whose root is an internal node (brute force and single-leaf trees run in k_render).
+//
+// What bounds it: on four workgroups per CU the instructions of the traversal step and of the shading
+// pass (a timing copy counted 4,700 and 9,000 cycles a wave for them on a closed mesh, 45% and 33% of
+// its time, before the pass was changed); on two, the latency of the longest pixels' steps (3,500 cycles
+// beside one neighbour, 2,400 alone).  Hence:
+//   * the step has no branch but the one around the triangle test: one fma per box plane (slab_hn) and the
+//     children pushed by counted places (half_step); 265 -> 200 vector instructions;
+//   * the traversal loop holds the step alone, so its back edge copies no path state;
+//   * one shading pass serves a bounce: both lights and the next direction are drawn in it, and a finished
+//     shadow ray starts the next query between passes;
+//   * divisions and roots are correctly rounded in three and five instructions (rcp_exact, sqrt_exact);
+//   * a wave with few queries left shares them among its lanes (half_sparse).
+// Times before and after, one frame: 512x512x8 spp of the 65,538-shape soup 7.6 -> 5.3 ms; 1024x768x16 of the
+// 327,692-shape mesh 36.2 -> 18.3 ms; 640x480x4 of a 20,492-shape SAH KD tree 5.1 -> 3.2 ms; 97x61x1 of a
+// 332-shape mesh 0.57 -> 0.25 ms.
 enum : int {
     kNeed = 0,    // wants a pixel
     kTrav = 1,    // traversing
-    kCDone = 2,   // closest-hit query finished: tb / bid hold the result
-    kADone = 3,   // any-hit query finished: bid >= 0 means occluded
-    kLight = 4,   // next light of SampleLights (index li)
+    kADone = 2,   // any-hit query finished: bid >= 0 means occluded
+    kCDone = 3,   // closest-hit query finished: tb / bid hold the result
+    kLight = 4,   // next lights of SampleLights (from index li)
     kSeg = 5,     // start of a path segment (depth checked here)
     kEnded = 6,   // sample finished
     kIdle = 7,    // no work left
 };
+constexpr unsigned kShadowMin = 8;   // finished shadow rays that a full wave leaves the traversal loop for
 
 template <int STACK, bool STATS, bool WIDE, bool MULTI, bool HALF>
-__global__ __launch_bounds__(256, STACK == kStackShort || STACK == kStackTiny ? 4 : 1) void k_render_lanes(RenderParams P) {
+__global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && STACK <= 48 ? 3 : 1) void k_render_lanes(RenderParams P) {
     if (!MULTI && recorded_tree_unfit(P)) return;
     if (MULTI && P.status && recorded_jobs_unfit(P)) return;
+    if (HALF && !MULTI && (int)blockIdx.x >= P.blocks_open && camera_outside(P)) return;
     __shared__ int s_stack[STACK * 256];
     int *stk = s_stack + threadIdx.x;
-    // The short class (binary16 walk only) holds fewer entries than the tree's height could need: a
-    // push that does not fit sets kOverflow in the lane's visit count, which ends the walk at its next
-    // step, and the query is then finished against every primitive (see kTrav below).
-    constexpr bool kShort = STACK == kStackShort || STACK == kStackTiny;
-    static_assert(!kShort || (WIDE && HALF), "the short stack class serves the binary16 walk");
+    static_assert(!kIsShort<STACK> || (WIDE && HALF), "the short stack class serves the binary16 walk");
     const unsigned long long lt = lanemask_lt();
     // A single frame's first kLdsLights lights, 16 words each (words 0-12 of the light's Shape, then
     // its area), copied once per workgroup: SampleLights then reads LDS instead of two dependent
@@ -351,34 +359,50 @@ __global__ __launch_bounds__(256, STACK == kStackShort || STACK == kStackTiny ? 
     // the tree of the lane's current query (uniform for a single frame)
     const gmem<const TNode> *t_nodes = to_gmem(P.acc.nodes);
     const gmem<const TNode4> *t_nodes4 = to_gmem(P.acc.nodes4);
-    const gmem<const TNode4H> *t_nodes4h = to_gmem(P.acc.nodes4h);
-    const gmem<const Prim> *t_prims = to_gmem(P.acc.prims);
-    int t_nnodes = P.acc.nnodes, t_nprims = P.acc.nprims, t_nshapes = P.acc.nshapes, t_root = P.acc.root;
+    HalfTree T;
+    T.nodes = to_gmem(P.acc.nodes4h);
+    T.prims = to_gmem(P.acc.prims);
+    T.nprims = P.acc.nprims;
+    T.skip = P.acc.nshapes - 1;
+    int t_nnodes = P.acc.nnodes, t_root = P.acc.root, t_slack = P.slack;
 
-    int st = kNeed;
+    int st = (int)__lane_id() < P.lanes ? kNeed : kIdle;
     bool drained = false;
     int gid = 0, k = 0, depth = 0, li = 0;
-    bool spec = true, qany = false;
+    bool spec = true;
     unsigned s0 = 0, s1 = 0;
-    f3 col = mk(0.f, 0.f, 0.f), ro = col, rd = mk(0.f, 0.f, 1.f), rad = col, thr = mk(1.f, 1.f, 1.f);
+    f3 col = mk(0.f, 0.f, 0.f), rad = col, thr = mk(1.f, 1.f, 1.f);
     f3 nl = col, Ld = col, contrib = col, inv = col;
-    RaySlab rsl = ray_slab(mk(1.f, 1.f, 1.f));
-    float tb = kInf;
-    int bid = -1, node = 0, sp = 0;
-    int pl = -1;   // binary16 walk: first primitive of a leaf run waiting to be tested (-1 none)
-    unsigned nv = 0;
+    f3 rd2 = col, contrib2 = col;   // the bounce's second shadow ray, if `more`
+    float maxt2 = 0.f;
+    bool more = false;
+    // the lane's query: HalfWalk's fields serve every node format (leaf and rs the binary16 one only)
+    HalfWalk Q;
+    Q.o = col;
+    Q.d = mk(0.f, 0.f, 1.f);
+    Q.tb = kInf;
+    Q.bid = -1;
+    Q.node = Q.sp = 0;
+    Q.leaf = 0;
+    Q.any = false;
+    Q.rs = ray_slab(Q.o, mk(1.f, 1.f, 1.f));
+    f3 &ro = Q.o, &rd = Q.d;
+    float &tb = Q.tb;
+    int &bid = Q.bid, &node = Q.node, &sp = Q.sp;
+    bool &qany = Q.any;
+    unsigned nv = 0;   // node visits (fp32 and binary nodes: a caller's tree may be malformed)
     unsigned long long n_closest = 0, n_any = 0;
     unsigned st_nodes = 0, st_prims = 0;
 
     // the primitives of one leaf for the lane's current query; true when an any-hit query is decided
     auto leaf = [&](int first, int cnt) -> bool {
-        if (first < 0 || cnt > t_nprims - first) return false;   // malformed caller tree
+        if (first < 0 || cnt > T.nprims - first) return false;   // malformed caller tree
         for (int q = 0; q < cnt; q++) {
             int id;
-            const float t = prim_isect(from_gmem(t_prims), first + q, ro, rd, &id);
+            const float t = prim_isect(from_gmem(T.prims), first + q, ro, rd, &id);
             if (STATS) st_prims++;
             if (qany) {
-                if (t != 0.f && t < tb && id != t_nshapes - 1) { bid = 1; return true; }
+                if (t != 0.f && t < tb && id != T.skip) { bid = 1; return true; }
             } else if (t != 0.f && (t < tb || (t == tb && id > bid))) {
                 tb = t;
                 bid = id;
@@ -386,252 +410,61 @@ __global__ __launch_bounds__(256, STACK == kStackShort || STACK == kStackTiny ? 
         }
         return false;
     };
-    // the primitive run of one leaf (binary16 nodes carry no counts: a run ends at kLastInLeaf)
-    auto leaf_run = [&](int first) -> bool {
-        if (first < 0 || first >= t_nprims) return false;   // malformed caller tree
-        for (int q = first; q < t_nprims; q++) {
-            int id;
-            bool last;
-            const float t = prim_isect_run(from_gmem(t_prims), q, ro, rd, &id, &last);
-            if (STATS) st_prims++;
-            if (qany) {
-                if (t != 0.f && t < tb && id != t_nshapes - 1) { bid = 1; return true; }
-            } else if (t != 0.f && (t < tb || (t == tb && id > bid))) {
-                tb = t;
-                bid = id;
-            }
-            if (last) break;
-        }
-        return false;
-    };
-    // A walk that outgrew the short stack is finished against every primitive, from the best hit found
-    // so far.  The closest hit is the least (t, then the higher id) whatever the order of the tests,
-    // and an occluder ends an any-hit query, so the result is the walk's.
-    auto finish_overflowed = [&]() {
-        for (int q = 0; q < t_nprims && !(qany && bid >= 0); q++) {
-            const Prim *tq = from_gmem(t_prims) + q;
-            int id;
-            bool last;
-            const float t = prim_isect_vals(tq->p0, tq->p1, tq->p2, ro, rd, &id, &last);
-            if (STATS) st_prims++;
-            if (qany) {
-                if (t != 0.f && t < tb && id != t_nshapes - 1) bid = 1;
-            } else if (t != 0.f && (t < tb || (t == tb && id > bid))) {
-                tb = t;
-                bid = id;
-            }
-        }
-    };
-    // start the lane's query along (ro, rd); tb = maxt for any-hit
+    // the lane's next query, along (ro, rd) as they stand at the end of the shading pass (tb = maxt for
+    // any-hit): all lanes that leave the pass with one set it up together there
+    bool fresh = false;
     auto start = [&](bool any, float maxt) {
         qany = any;
         tb = any ? maxt : kInf;
-        bid = -1;
-        inv = mk(1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z);
-        if (HALF) rsl = ray_slab(inv);
-        node = t_root;
-        pl = -1;
-        sp = 0;
-        nv = 0;
         st = kTrav;
+        fresh = true;
+    };
+    auto set_up = [&]() {
+        if (HALF) {
+            half_start(Q, t_root);
+        } else {
+            bid = -1;
+            inv = mk(1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z);
+            node = t_root;
+            sp = 0;
+            nv = 0;
+        }
+        fresh = false;
     };
 
+    // the light term joins the radiance and the path goes on along the direction drawn with it (nl holds it)
+    auto end_bounce = [&]() {
+        Ld = mul3(thr, Ld);
+        rad = add3(rad, Ld);
+        rd = nl;
+        depth++;
+        if (depth > JFR(max_depth)) {
+            st = kEnded;
+        } else {
+            n_closest++;
+            start(false, 0.f);
+        }
+    };
+
+    // The wave's schedule.  The traversal loop changes the queries' state only and is left for everything
+    // else, so that its back edge carries (and copies) nothing but that state.
     for (;;) {
-        // ---- traversal: one node of every traversing lane per iteration, until `regroup` lanes
-        // (or all that are left) have finished their queries ----
         const unsigned long long live = __ballot(st != kIdle);
         if (!live) break;
         // a sparse wave (the end of the frame) shades sooner, so no lane's path waits long on others
         const unsigned nlive = (unsigned)__popcll(live);
         const unsigned quarter = (nlive + 3u) >> 2;
-        const unsigned regroup = (unsigned)P.regroup < quarter ? (unsigned)P.regroup : quarter;
+        unsigned regroup = (unsigned)P.regroup < quarter ? (unsigned)P.regroup : quarter;
+        if (nlive >= 48u) regroup = (unsigned)P.regroup;
+        const unsigned shadow_min = kShadowMin < regroup ? kShadowMin : regroup;
+        const unsigned dense_min = HALF ? (unsigned)P.quad : 0u;
+        // ---- traversal: one node of every traversing lane per iteration, until `regroup` lanes wait for
+        // shading, `shadow_min` shadow rays have finished, or the wave is sparse ----
         for (;;) {
             const unsigned long long trav = __ballot(st == kTrav);
-            if (!trav || (unsigned)__popcll(live & ~trav) >= regroup) break;
-            if (HALF && (unsigned)__popcll(trav) <= (unsigned)P.quad) {
-                // ---- quad phase: a sparse wave lends its idle lanes to the queries in flight.  The
-                // k-th traversing lane's query is walked by lanes 4k..4k+3, lane c of the quad taking
-                // child c of each node: one 16-byte load, one box test and (for a leaf child) one
-                // primitive run per lane, then the quad agrees on the hit, the next node and the
-                // pushes through DPP.  Same nodes, same hits, shorter steps. ----
-                const int qk = (int)(__lane_id() >> 2), qc = (int)(__lane_id() & 3);
-                const int nq = __popcll(trav);
-                int owner = 0;
-                {
-                    unsigned long long m = trav;
-                    for (int j = 0; j < nq; j++) {
-                        const int b = __ffsll((long long)m) - 1;
-                        if (j == qk) owner = b;
-                        m &= m - 1;
-                    }
-                }
-                const bool inq = qk < nq;
-                // the owner's query (every lane runs the shuffles; lanes beyond nq read lane 0)
-                f3 q_o, q_d, q_inv;
-                q_o.x = __shfl(ro.x, owner); q_o.y = __shfl(ro.y, owner); q_o.z = __shfl(ro.z, owner);
-                q_d.x = __shfl(rd.x, owner); q_d.y = __shfl(rd.y, owner); q_d.z = __shfl(rd.z, owner);
-                q_inv.x = __shfl(inv.x, owner); q_inv.y = __shfl(inv.y, owner); q_inv.z = __shfl(inv.z, owner);
-                const RaySlab q_rs = ray_slab(q_inv);
-                float q_tb = __shfl(tb, owner);
-                int q_bid = __shfl(bid, owner), q_node = __shfl(node, owner), q_sp = __shfl(sp, owner);
-                int q_pl = __shfl(pl, owner);
-                unsigned q_nv = (unsigned)__shfl((int)nv, owner);
-                const bool q_any = __shfl((int)qany, owner) != 0;
-                const gmem<const TNode4H> *q_nodes = t_nodes4h;
-                const gmem<const Prim> *q_prims = t_prims;
-                int q_nnodes = t_nnodes, q_nprims = t_nprims, q_nshapes = t_nshapes;
-                if (MULTI) {
-                    auto shp = [&](const void *ptr) -> const void * {
-                        const unsigned long long v = reinterpret_cast<unsigned long long>(ptr);
-                        const unsigned lo = (unsigned)__shfl((int)(unsigned)v, owner);
-                        const unsigned hi = (unsigned)__shfl((int)(unsigned)(v >> 32), owner);
-                        return reinterpret_cast<const void *>(((unsigned long long)hi << 32) | lo);
-                    };
-                    q_nodes = to_gmem(static_cast<const TNode4H *>(shp(from_gmem(t_nodes4h))));
-                    q_prims = to_gmem(static_cast<const Prim *>(shp(from_gmem(t_prims))));
-                    q_nnodes = __shfl(t_nnodes, owner);
-                    q_nprims = __shfl(t_nprims, owner);
-                    q_nshapes = __shfl(t_nshapes, owner);
-                }
-                int *q_stk = s_stack + (threadIdx.x & ~63u) + owner;   // the owner's stack column
-                bool q_done = !inq;
-                bool q_end = false;   // the query finished (as opposed to the phase ending)
-                constexpr float inf = __builtin_inff();
-                const unsigned ready0 = (unsigned)__popcll(live & ~trav);
-                for (;;) {
-                    const unsigned long long fin = __ballot(inq && q_end && qc == 0);
-                    if (ready0 + (unsigned)__popcll(fin) >= regroup || (unsigned)__popcll(fin) >= (unsigned)nq) break;
-                    if (!q_done) {
-                        const bool qhn = q_node >= 0;
-                        if ((qhn && q_node >= q_nnodes) || ++q_nv > kMaxVisits) {
-                            q_done = q_end = true;   // malformed caller tree
-                        } else {
-                            // On lane 0 the owner's pending run, then on every lane its leaf child, against
-                            // the step's tb.  The run's first primitive is loaded before the child (every
-                            // lane issues both loads; the others read primitive 0 and ignore it), so its
-                            // test overlaps the child's latency.
-                            const bool qhl = qc == 0 && q_pl >= 0 && q_pl < q_nprims;
-                            const Prim *qpp = from_gmem(q_prims) + (qhl ? q_pl : 0);
-                            const float4 m0 = qpp->p0, m1 = qpp->p1, m2 = qpp->p2;
-                            asm volatile("" ::: "memory");   // compiler-only: keeps the order above
-                            const uint4 w = from_gmem(q_nodes)[qhn ? q_node : 0].c[qc];   // ignored with no node
-                            float bt = q_tb;
-                            int bb = q_bid;
-                            bool occl = false;
-                            auto take = [&](float t, int id) -> bool {   // true: occluded, stop
-                                if (STATS) st_prims++;
-                                if (q_any) {
-                                    if (t != 0.f && t < q_tb && id != q_nshapes - 1) { occl = true; return true; }
-                                } else if (t != 0.f && (t < bt || (t == bt && id > bb))) {
-                                    bt = t;
-                                    bb = id;
-                                }
-                                return false;
-                            };
-                            if (qhl) {
-                                int id;
-                                bool last;
-                                const float t = prim_isect_vals(m0, m1, m2, q_o, q_d, &id, &last);
-                                if (!take(t, id) && !last) {
-                                    for (int q = q_pl + 1; q < q_nprims; q++) {
-                                        const float t2 = prim_isect_run(from_gmem(q_prims), q, q_o, q_d, &id, &last);
-                                        if (take(t2, id) || last) break;
-                                    }
-                                }
-                            }
-                            const int ref = qhn ? (int)w.w : kEmptyRef;
-                            float tc = slab_hn(w.x, w.y, w.z, q_o, q_inv, q_rs, q_tb * kSlack, P.one);
-                            if (!qhn) tc = inf;
-                            if (STATS) st_nodes += ref != kEmptyRef;
-                            if (!occl && ref < 0 && tc != inf && ~ref < q_nprims) {
-                                for (int q = ~ref; q < q_nprims; q++) {
-                                    int id;
-                                    bool last;
-                                    const float t = prim_isect_run(from_gmem(q_prims), q, q_o, q_d, &id, &last);
-                                    if (take(t, id) || last) break;
-                                }
-                            }
-                            q_pl = -1;
-                            if (ref < 0) tc = inf;   // only internal children from here on
-                            // the quad's hit: occlusion by any lane; closest by (t, then higher id)
-                            occl = (qxor<1>((int)occl) | qxor<2>((int)occl) | qxor<1>(qxor<2>((int)occl)) |
-                                    (int)occl) != 0;
-                            {
-                                float ot = qxorf<1>(bt);
-                                int oi = qxor<1>(bb);
-                                if (ot < bt || (ot == bt && oi > bb)) { bt = ot; bb = oi; }
-                                ot = qxorf<2>(bt);
-                                oi = qxor<2>(bb);
-                                if (ot < bt || (ot == bt && oi > bb)) { bt = ot; bb = oi; }
-                            }
-                            if (q_any) {
-                                if (occl) {
-                                    q_bid = 1;
-                                    q_done = q_end = true;
-                                }
-                            } else {
-                                q_tb = bt;
-                                q_bid = bb;
-                            }
-                            if (!q_done) {
-                                // internal children: nearest next, the rest pushed farthest first; order
-                                // by (t, slot), which every lane of the quad evaluates alike
-                                const float t1 = qrotf<1>(tc), t2 = qrotf<2>(tc), t3 = qrotf<3>(tc);
-                                const int r1 = qrot<1>(ref), r2 = qrot<2>(ref), r3 = qrot<3>(ref);
-                                const int s1 = (qc + 1) & 3, s2 = (qc + 2) & 3, s3 = (qc + 3) & 3;
-                                const int nh = (tc != inf) + (t1 != inf) + (t2 != inf) + (t3 != inf);
-                                auto before = [](float ta, int sa, float tb_, int sb) {
-                                    return ta < tb_ || (ta == tb_ && sa < sb);
-                                };
-                                const int rank = before(t1, s1, tc, qc) + before(t2, s2, tc, qc) + before(t3, s3, tc, qc);
-                                float nt = tc;
-                                int nr = ref, ns = qc;
-                                if (before(t1, s1, nt, ns)) { nt = t1; nr = r1; ns = s1; }
-                                if (before(t2, s2, nt, ns)) { nt = t2; nr = r2; ns = s2; }
-                                if (before(t3, s3, nt, ns)) { nt = t3; nr = r3; ns = s3; }
-                                if (nh > 0) {
-                                    if (tc != inf && rank > 0) {
-                                        const int pos = q_sp + nh - 1 - rank;
-                                        if (pos < STACK) q_stk[pos * 256] = ref;
-                                    }
-                                    q_sp += nh - 1;
-                                    // a push past the stack (the same test on every lane of the quad)
-                                    if (kShort && q_sp > STACK) q_nv |= kOverflow;
-                                    if (q_sp > STACK) q_sp = STACK;
-                                    q_node = nr;
-                                } else if (q_sp == 0) {
-                                    q_done = q_end = true;
-                                } else {
-                                    const int r = q_stk[(--q_sp) * 256];   // a node, or a leaf to test next
-                                    q_node = r >= 0 ? r : -1;
-                                    q_pl = r >= 0 ? -1 : ~r;
-                                }
-                            }
-                        }
-                    }
-                }
-                // hand each query back to its owner: the owner of quad k reads lane 4k
-                const int src = 4 * (int)__popcll(trav & lt);
-                const int b_node = __shfl(q_node, src), b_sp = __shfl(q_sp, src), b_bid = __shfl(q_bid, src);
-                const float b_tb = __shfl(q_tb, src);
-                const unsigned b_nv = (unsigned)__shfl((int)q_nv, src);
-                const bool b_end = __shfl((int)q_end, src) != 0;
-                const int b_pl = __shfl(q_pl, src);
-                if (st == kTrav) {
-                    node = b_node;
-                    pl = b_pl;
-                    sp = b_sp;
-                    bid = b_bid;
-                    tb = b_tb;
-                    nv = b_nv;
-                    if (b_end) {
-                        // a walk that overflowed ends at its next quad step and is finished here
-                        if (kShort && (b_nv & kOverflow)) finish_overflowed();
-                        st = qany ? kADone : kCDone;
-                    }
-                }
-                continue;
-            }
+            if ((unsigned)__popcll(trav) <= dense_min || (unsigned)__popcll(live & ~trav) >= regroup ||
+                (unsigned)__popcll(__ballot(st == kADone)) >= shadow_min)
+                break;
             if (!WIDE && st == kTrav) {
                 bool done = false;
                 if ((unsigned)node >= (unsigned)t_nnodes || ++nv > kMaxVisits) {
@@ -671,124 +504,7 @@ __global__ __launch_bounds__(256, STACK == kStackShort || STACK == kStackTiny ? 
                 if (done) st = qany ? kADone : kCDone;
             }
             if (HALF && st == kTrav) {
-                // One step = the current node (if any) and the pending leaf run (if any), loaded
-                // together: a hit leaf is not tested in the step that finds it but in the next one,
-                // beside the next node's loads, so a step costs one memory round trip, not two.
-                bool done = false;
-                constexpr float inf = __builtin_inff();
-                const bool hn = node >= 0;
-                if ((hn && node >= t_nnodes) || ++nv > kMaxVisits) {
-                    done = true;   // malformed caller tree
-                } else {
-                    // Every lane issues both loads, the run's primitive first: a lane with no run reads
-                    // primitive 0 and one with no node reads node 0 (both exist in a tree with binary16
-                    // nodes), and ignores them.  With no branch around the loads the wait for the
-                    // primitive leaves the node's four loads in flight, so the triangle test overlaps
-                    // the node's latency.
-                    const bool hl = pl >= 0 && pl < t_nprims;
-                    const Prim *pp = from_gmem(t_prims) + (hl ? pl : 0);
-                    float4 a0 = pp->p0, a1 = pp->p1, a2 = pp->p2;
-                    // compiler-only barrier (no operands, no instruction): the primitive's loads stay
-                    // here, ahead of the node's, instead of sinking into the branch that tests them
-                    asm volatile("" ::: "memory");
-                    const TNode4H *np = from_gmem(t_nodes4h) + (hn ? node : 0);
-                    const uint4 q0 = np->c[0], q1 = np->c[1], q2 = np->c[2], q3 = np->c[3];
-                    // the pending run (one primitive per LBVH leaf), before the boxes so tb is tight
-                    if (hl) {
-                        // true: the run ends here (an occluder found, or its last primitive)
-                        auto test_prim = [&](const float4 &b0, const float4 &b1, const float4 &b2, int q) -> bool {
-                            const int id = __float_as_int(b0.w);
-                            const float t = (__float_as_int(b2.w) & 0xff) == SPHERE ? sph_isect(b0, b1.x, ro, rd)
-                                                                                     : tri_isect(b0, b1, b2, ro, rd);
-                            if (STATS) st_prims++;
-                            if (qany) {
-                                if (t != 0.f && t < tb && id != t_nshapes - 1) { bid = 1; done = true; return true; }
-                            } else if (t != 0.f && (t < tb || (t == tb && id > bid))) {
-                                tb = t;
-                                bid = id;
-                            }
-                            return (__float_as_int(b1.w) & kLastInLeaf) || q + 1 >= t_nprims;
-                        };
-                        // the first primitive outside the loop: the loop's own loads issue in another
-                        // order, and a shared loop head would make this test wait for the node too
-                        if (!test_prim(a0, a1, a2, pl)) {
-                            for (int q = pl + 1;; q++) {
-                                const Prim *tq = from_gmem(t_prims) + q;
-                                const float4 b0 = tq->p0, b1 = tq->p1, b2 = tq->p2;
-                                if (test_prim(b0, b1, b2, q)) break;
-                            }
-                        }
-                    }
-                    pl = -1;
-                    int nn = -1;
-                    if (!done && hn) {
-                        int r0 = (int)q0.w, r1 = (int)q1.w, r2 = (int)q2.w, r3 = (int)q3.w;
-                        const float tbs = tb * kSlack;
-                        float t0 = slab_hn(q0.x, q0.y, q0.z, ro, inv, rsl, tbs, P.one);
-                        float t1 = slab_hn(q1.x, q1.y, q1.z, ro, inv, rsl, tbs, P.one);
-                        float t2 = slab_hn(q2.x, q2.y, q2.z, ro, inv, rsl, tbs, P.one);
-                        float t3 = slab_hn(q3.x, q3.y, q3.z, ro, inv, rsl, tbs, P.one);
-                        if (STATS) st_nodes += (r0 != kEmptyRef) + (r1 != kEmptyRef) + (r2 != kEmptyRef) + (r3 != kEmptyRef);
-                        auto cswap = [](float &ta, int &ra, float &tb_, int &rb) {
-                            const bool sw = tb_ < ta;
-                            const float tt = sw ? tb_ : ta;
-                            tb_ = sw ? ta : tb_;
-                            ta = tt;
-                            const int rr = sw ? rb : ra;
-                            rb = sw ? ra : rb;
-                            ra = rr;
-                        };
-                        cswap(t0, r0, t1, r1);
-                        cswap(t2, r2, t3, r3);
-                        cswap(t0, r0, t2, r2);
-                        cswap(t1, r1, t3, r3);
-                        cswap(t1, r1, t2, r2);
-                        // nearest internal child next, nearest leaf pending, the rest pushed farthest first
-                        bool c0 = false, c1 = false, c2 = false, c3 = false;
-                        auto choose = [&](float t, int r, bool &c) {
-                            if (t == inf) return;
-                            if (r >= 0) {
-                                if (nn < 0) { nn = r; c = true; }
-                            } else if (pl < 0) {
-                                pl = ~r;
-                                c = true;
-                            }
-                        };
-                        choose(t0, r0, c0);
-                        choose(t1, r1, c1);
-                        choose(t2, r2, c2);
-                        choose(t3, r3, c3);
-                        auto push = [&](float t, bool c, int r) {
-                            if (t == inf || c) return;
-                            if (sp < STACK) stk[(sp++) * 256] = r;
-                            else if (kShort) nv |= kOverflow;
-                        };
-                        push(t3, c3, r3);
-                        push(t2, c2, r2);
-                        push(t1, c1, r1);
-                        push(t0, c0, r0);
-                    }
-                    node = nn;
-                    if (!done) {
-                        // refill from the stack: a node for the next step, and a leaf to load beside it.
-                        // The top two entries are read together (one LDS round trip, not two).
-                        const int e1 = sp > 0 ? stk[(sp - 1) * 256] : 0;
-                        const int e2 = sp > 1 ? stk[(sp - 2) * 256] : 0;
-                        int top = e1;
-                        if (node < 0 && sp > 0 && e1 >= 0) {
-                            node = e1;
-                            --sp;
-                            top = e2;
-                        }
-                        if (pl < 0 && sp > 0 && top < 0) {
-                            pl = ~top;
-                            --sp;
-                        }
-                        if (node < 0 && pl < 0) done = true;   // the stack is empty
-                    }
-                }
-                if (kShort && done && (nv & kOverflow)) finish_overflowed();
-                if (done) st = qany ? kADone : kCDone;
+                if (half_step<STACK, STATS>(Q, T, stk, &st_nodes, &st_prims)) st = qany ? kADone : kCDone;
             }
             if (WIDE && !HALF && st == kTrav) {
                 bool done = false;
@@ -797,18 +513,7 @@ __global__ __launch_bounds__(256, STACK == kStackShort || STACK == kStackTiny ? 
                 } else {
                     float4 lx, ly, lz, hx, hy, hz;
                     int4 rf, cn;
-                    if (HALF) {
-                        const TNode4H *np = from_gmem(t_nodes4h) + node;
-                        const uint4 q0 = np->c[0], q1 = np->c[1], q2 = np->c[2], q3 = np->c[3];
-                        rf = make_int4((int)q0.w, (int)q1.w, (int)q2.w, (int)q3.w);
-                        cn = make_int4(0, 0, 0, 0);
-                        lx = make_float4(half_lo(q0.x), half_lo(q1.x), half_lo(q2.x), half_lo(q3.x));
-                        hx = make_float4(half_hi(q0.x), half_hi(q1.x), half_hi(q2.x), half_hi(q3.x));
-                        ly = make_float4(half_lo(q0.y), half_lo(q1.y), half_lo(q2.y), half_lo(q3.y));
-                        hy = make_float4(half_hi(q0.y), half_hi(q1.y), half_hi(q2.y), half_hi(q3.y));
-                        lz = make_float4(half_lo(q0.z), half_lo(q1.z), half_lo(q2.z), half_lo(q3.z));
-                        hz = make_float4(half_hi(q0.z), half_hi(q1.z), half_hi(q2.z), half_hi(q3.z));
-                    } else {
+                    {
                         const TNode4 *np = from_gmem(t_nodes4) + node;
                         lx = np->lox; ly = np->loy; lz = np->loz;
                         hx = np->hix; hy = np->hiy; hz = np->hiz;
@@ -834,12 +539,8 @@ __global__ __launch_bounds__(256, STACK == kStackShort || STACK == kStackTiny ? 
                         const unsigned k = (unsigned)__builtin_ctz(lm);
                         lm &= lm - 1u;
                         const int lr = k == 0 ? rf.x : k == 1 ? rf.y : k == 2 ? rf.z : rf.w;
-                        if (HALF) {
-                            done = leaf_run(~lr);
-                        } else {
-                            const int lc = k == 0 ? cn.x : k == 1 ? cn.y : k == 2 ? cn.z : cn.w;
-                            done = leaf(~lr, lc);
-                        }
+                        const int lc = k == 0 ? cn.x : k == 1 ? cn.y : k == 2 ? cn.z : cn.w;
+                        done = leaf(~lr, lc);
                     }
                     if (!done) {
                         // inner children: nearest first (order only changes the visit count)
@@ -867,6 +568,35 @@ __global__ __launch_bounds__(256, STACK == kStackShort || STACK == kStackTiny ? 
                     }
                 }
                 if (done) st = qany ? kADone : kCDone;
+            }
+        }
+        // ---- finished shadow rays: the bounce's other shadow ray, or its next segment, both drawn when the
+        // bounce was shaded, start here without a shading pass ----
+        if (st == kADone) {
+            if (bid < 0) Ld = add3(Ld, contrib);
+            if (more) {
+                more = false;
+                contrib = contrib2;
+                rd = rd2;
+                n_any++;
+                start(true, maxt2);
+            } else if (li < JFR(nlights)) {
+                st = kLight;
+            } else {
+                end_bounce();
+            }
+            if (fresh) set_up();
+        }
+        {
+            const unsigned long long trav = __ballot(st == kTrav);
+            const unsigned ready = (unsigned)__popcll(live & ~trav);
+            if (trav && ready < regroup) {
+                // a sparse wave lends its idle lanes to the queries in flight
+                if (HALF && (unsigned)__popcll(trav) <= (unsigned)P.quad &&
+                    half_sparse<STACK, STATS, MULTI>(Q, T, t_slack, st == kTrav, trav, ready, regroup, s_stack,
+                                                     &st_nodes, &st_prims))
+                    st = qany ? kADone : kCDone;
+                continue;
             }
         }
         // ---- shading pass: pixels for lanes that need one (one atomic per wave) ----
@@ -906,12 +636,13 @@ __global__ __launch_bounds__(256, STACK == kStackShort || STACK == kStackTiny ? 
                         const DevAccel &A = P.jobs[jb].acc;
                         t_nodes = to_gmem(A.nodes);
                         t_nodes4 = to_gmem(A.nodes4);
-                        t_nodes4h = to_gmem(A.nodes4h);
-                        t_prims = to_gmem(A.prims);
+                        T.nodes = to_gmem(A.nodes4h);
+                        T.prims = to_gmem(A.prims);
                         t_nnodes = A.nnodes;
-                        t_nprims = A.nprims;
-                        t_nshapes = A.nshapes;
+                        T.nprims = A.nprims;
+                        T.skip = A.nshapes - 1;
                         t_root = A.root;
+                        t_slack = half_slack(STACK, A);
                         j_shapes = to_gmem(P.jobs[jb].shapes);
                         j_lights = to_gmem(P.jobs[jb].lights);
                         j_nlights = P.jobs[jb].nlights;
@@ -974,39 +705,44 @@ __global__ __launch_bounds__(256, STACK == kStackShort || STACK == kStackTiny ? 
                     }
                 }
             }
-            if (st == kADone) {
-                if (bid < 0) Ld = add3(Ld, contrib);
-                li++;
-                st = kLight;
-            }
             if (st == kLight) {
-                // lights whose sample needs no shadow ray only draw their random numbers
+                // The next two lights whose sample needs a shadow ray (the others only draw their random
+                // numbers) and, once every light is drawn, the direction the path goes on in: shadow rays
+                // never draw, so the numbers come in the reference's order, and one pass serves the whole
+                // bounce.
                 float len = 0.f;
                 bool shoot = false;
-                const int nlights = MULTI ? j_nlights : P.nlights;
-                for (; li < nlights; li++) {
+                const int nlights = JFR(nlights);
+                while (li < nlights && !more) {
+                    f3 sd, con;
                     const bool sh = !MULTI && li < n_lds_lights
                                         ? sample_light_words(s_lights + 16 * li, s_lights[16 * li + 13], s0, s1, ro,
-                                                             nl, &rd, &len, &contrib)
-                                        : sample_light(JSHAPES + (MULTI ? from_gmem(j_lights) : P.lights)[li], s0, s1, ro, nl, &rd, &len,
-                                                       &contrib);
-                    if (sh) {
+                                                             nl, &sd, &len, &con)
+                                        : sample_light(JSHAPES + (MULTI ? from_gmem(j_lights) : P.lights)[li], s0, s1, ro, nl, &sd, &len,
+                                                       &con);
+                    li++;
+                    if (!sh) continue;
+                    if (shoot) {
+                        more = true;
+                        rd2 = sd;
+                        contrib2 = con;
+                        maxt2 = len - kEpsilon;
+                    } else {
                         shoot = true;
-                        break;
+                        rd = sd;
+                        contrib = con;
+                        tb = len - kEpsilon;
                     }
                 }
+                if (li >= nlights) nl = diffuse_dir(nl, s0, s1);
                 if (shoot) {
                     n_any++;
-                    start(true, len - kEpsilon);
+                    start(true, tb);
                     continue;
                 }
-                Ld = mul3(thr, Ld);
-                rad = add3(rad, Ld);
-                rd = diffuse_dir(nl, s0, s1);
-                depth++;
-                st = kSeg;
+                end_bounce();
             }
-            if (st == kSeg && depth > (MULTI ? j_max_depth : P.max_depth)) st = kEnded;
+            if (st == kSeg && depth > JFR(max_depth)) st = kEnded;
             if (st == kEnded) {
                 col = running_mean(col, rad, JFR(currentSample) + k);
                 k++;
@@ -1032,6 +768,7 @@ __global__ __launch_bounds__(256, STACK == kStackShort || STACK == kStackTiny ? 
                 start(false, 0.f);
             }
         }
+        if (fresh) set_up();
     }
     if (P.ray_counter) {
         unsigned long long a = n_closest, b = n_any;
@@ -1511,6 +1248,40 @@ static int stack_for(const DevAccel &acc, int least) {
     return -1;
 }
 
+// Workgroups of a single-frame launch and the wave's share of pixels, for `total` work items.
+//
+// Set by the caller ("blocks_per_cu"): that many persistent workgroups per CU, never more than needed.
+// By default, for the binary16 walk:
+//   * Up to 8 pixels per wave slot (16 slots per CU: 32,768 pixels on 256 CUs) only the first 1, 2, 4 or 8
+//     lanes of a wave take pixels and the others help their queries (half_sparse): such a frame ends with
+//     its longest path whatever else runs, and shared queries take fewer steps.  97x61x1 spp of the
+//     332-shape mesh: 380 us with 64 pixels a wave, 230 us with two; 200x150 of the 5,132-shape mesh:
+//     428 us, with eight 397 us; at 320x240 sharing loses (510 us, with eight 855 us), so the line lies there.
+//   * Larger frames get four workgroups per CU (what the registers and the stack leave room for), but a
+//     frame of fewer than two pixels a lane whose camera is outside the scene's box keeps two (the kernel
+//     decides: the camera is device memory).  Seen from inside, every pixel's path is long and more waves
+//     keep the SIMDs busy: 1024x768x16 of the 327,692-shape mesh, two / four a CU: 28.8 / 18.5 ms.  From
+//     outside, much of the frame is background and the few long paths decide: on two a CU they run with
+//     fewer neighbours and lanes whose pixel was background take another (512x512x8 of the 65,538-shape
+//     soup, two / four: 5.1 / 5.7 ms; at 1024x1024x4, 6.9 / 5.0 ms).
+static int launch_shape(const ptgpu_ctx *ctx, int total, bool half, RenderParams &P) {
+    const int cus = ctx->cu_count;
+    int per_cu = ctx->blocks_per_cu;
+    if (ctx->blocks_auto && half) {
+        per_cu = 4;
+        if (ctx->quad > 0 && !P.trav_stats) {   // (counting launches keep one walk order for every shape)
+            int lanes = 1;
+            while (lanes < kWave && total > lanes * 16 * cus) lanes *= 2;
+            P.lanes = lanes <= 8 ? lanes : kWave;
+        }
+        if (total < 2 * 4 * 256 * cus) P.blocks_open = 2 * cus;
+    }
+    int blocks = cus * per_cu;
+    const int need = (total + 4 * P.lanes - 1) / (4 * P.lanes);
+    if (blocks > need) blocks = need;
+    return blocks < 1 ? 1 : blocks;
+}
+
 int launch_render(ptgpu_ctx *ctx, const DevAccel &acc, const RenderLaunch &L) {
     // work items: every pixel, or every pixel slot of the listed tiles (slots past the frame's edge are skipped)
     const int total = L.tiles ? L.ntiles * L.tile_w * L.tile_h : L.width * L.height;
@@ -1557,23 +1328,22 @@ int launch_render(ptgpu_ctx *ctx, const DevAccel &acc, const RenderLaunch &L) {
     P.tiles = L.tiles;
     P.tile_w = L.tile_w;
     P.tile_h = L.tile_h;
-    P.one = 1.0f;
+    P.slack = 0;
+    P.lanes = kWave;
+    P.blocks_open = 0x7fffffff;
     P.depth_cap = binary_depth_cap(st);
     P.status = nullptr;
     if (acc.height_check) {
         PT_TRY(ctx->rec_status.ensure(16));   // allocated at context creation; kept here for safety
         P.status = ctx->rec_status.as<unsigned>();
     }
-    // persistent waves: enough workgroups to fill every CU several times, never more than needed
-    int blocks = ctx->cu_count * ctx->blocks_per_cu;
-    const int need = (total + 255) / 256;
-    if (blocks > need) blocks = need;
-    if (blocks < 1) blocks = 1;
+    const bool lanes_engine = (ctx->engine == 0 || ctx->engine == 3) && acc.mode != PTGPU_ACCEL_NONE && acc.root >= 0;
+    const bool half = lanes_engine && ctx->wide == 2 && acc.nodes4h && stack_for_wide(acc, ctx->stack_min) > 0;
+    const int blocks = launch_shape(ctx, total, half, P);
     // auto and engine 3: per-lane states whenever there is a tree to walk (measured fastest at every
     // size tried); brute force and single-leaf scenes keep the lockstep megakernel
-    if ((ctx->engine == 0 || ctx->engine == 3) && acc.mode != PTGPU_ACCEL_NONE && acc.root >= 0) {
+    if (lanes_engine) {
         const int sw = acc.nodes4 && ctx->wide ? stack_for_wide(acc, ctx->stack_min) : -1;
-        const bool half = ctx->wide == 2 && acc.nodes4h;
         if (sw > 0) P.depth_cap = wide_depth_cap(sw);
         // the binary16 walk of a tree in the 48-entry class runs on the short stack, four workgroups
         // per CU (short_stack 2, a test setting, runs every binary16 walk on the 8-entry class).  Held
@@ -1581,6 +1351,7 @@ int launch_render(ptgpu_ctx *ctx, const DevAccel &acc, const RenderLaunch &L) {
         // entry does not ask the runtime for.
         const bool tiny = half && sw > 0 && ctx->short_stack == 2 && !L.no_alloc;
         const bool shortst = half && sw == 48 && ctx->short_stack == 1 && !L.no_alloc;
+        if (half && sw > 0) P.slack = half_slack(tiny ? kStackTiny : shortst ? kStackShort : sw, acc);
 #define PT_LANES(ST, STATS_, WIDE_, HALF_)                                                                      \
     hipLaunchKernelGGL((k_render_lanes<ST, STATS_, WIDE_, false, HALF_>), dim3(blocks), dim3(256), 0, ctx->stream, P)
 #define PT_LANES_W(ST, STATS_) \
@@ -2146,7 +1917,9 @@ int launch_batch(ptgpu_ctx *ctx, BatchChannel &ch, const ptgpu_render_job *jobs,
         P.jobs = reinterpret_cast<const RenderJob *>(static_cast<char *>(d_table) + K.jo);
         P.job_begin = reinterpret_cast<const unsigned *>(static_cast<char *>(d_table) + K.bo);
         P.njobs = (int)K.jobs.size();
-        P.one = 1.0f;
+        P.slack = 0;
+        P.lanes = kWave;
+    P.blocks_open = 0x7fffffff;
         P.depth_cap = wide_depth_cap(K.st);
         P.status = K.checks ? ctx->rec_status.as<unsigned>() : nullptr;
         long long blocks = (long long)ctx->cu_count * ctx->batch_blocks_per_cu;

@@ -27,7 +27,35 @@ PT_HD float dot3(f3 a, f3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 PT_HD f3 cross3(f3 a, f3 b) {
     return mk(a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x);
 }
-PT_HD f3 norm3(f3 v) { float l = 1.f / sqrtf(dot3(v, v)); return smul(l, v); }
+
+// 1/x and sqrt(x), correctly rounded, in three and five instructions where the compiler's forms take eleven
+// and sixteen (they scale every operand for the ends of the exponent range).  The hardware's reciprocal
+// and reciprocal square root are within one ulp, and one fma correction makes the result the IEEE
+// one for every binary32 x of the stated range: all 4.19e9 values of 2^-125 <= |x| <= 2^125 (1/x) and all
+// of 2^-96 <= x <= 2^126 (sqrt) were compared on gfx950.  A wave with any other x takes the compiler's
+// form (a branch of the whole wave: no lane mask to save and restore).
+PT_HD float rcp_exact(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const float a = fabsf(x);
+    if (__builtin_expect(__ballot(!(a >= 0x1p-125f && a <= 0x1p125f)) != 0ull, 0)) return 1.0f / x;
+    const float r = __builtin_amdgcn_rcpf(x);
+    return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+#else
+    return 1.0f / x;
+#endif
+}
+PT_HD float sqrt_exact(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if (__builtin_expect(__ballot(!(x >= 0x1p-96f && x <= 0x1p126f)) != 0ull, 0)) return sqrtf(x);
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float g = x * y;
+    return __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * y, g);
+#else
+    return sqrtf(x);
+#endif
+}
+
+PT_HD f3 norm3(f3 v) { float l = rcp_exact(sqrt_exact(dot3(v, v))); return smul(l, v); }
 PT_HD bool iszero3(f3 v) { return v.x == 0.f && v.y == 0.f && v.z == 0.f; }
 PT_HD f3 ldvec(const Vec *p) {
     const float *f = reinterpret_cast<const float *>(p);
@@ -96,7 +124,7 @@ PT_HD float tri_isect(const float4 &p0, const float4 &p1, const float4 &p2, f3 o
     const f3 pvec = cross3(d, e2);
     const float det = dot3(e1, pvec);
     if (det == 0.f) return 0.f;
-    const float inv = 1.0f / det;
+    const float inv = rcp_exact(det);
     const f3 tvec = sub3(o, v0);
     const float u = dot3(tvec, pvec) * inv;
     if (u < 0.0f || u > 1.0f) return 0.f;
@@ -111,7 +139,7 @@ PT_HD float sph_isect(const float4 &p0, float rad, f3 o, f3 d) {
     const float b = dot3(op, d);
     float det = b * b - dot3(op, op) + rad * rad;
     if (det < 0.f) return 0.f;
-    det = sqrtf(det);
+    det = sqrt_exact(det);
     float t = b - det;
     if (t > kEpsilon) return t;
     t = b + det;
@@ -175,48 +203,61 @@ PT_HD float slab(float lx, float ly, float lz, float hx, float hy, float hz, f3 
 }
 
 // The same test on a binary16 box: each word holds a bound pair, lo in its low half and hi in its
-// high half.  Each difference `bound - o` is one mixed-precision fma, fma(bound, one, -o) with the
-// binary16 bound read from its half of the word: the bound converts to binary32 exactly and the
-// product by one is exact, so the result is the rounded difference, bit for bit what a conversion
-// and a subtraction give.  `one` is 1.0f held where the compiler cannot see it (a literal would be
-// folded into that conversion and subtraction, two instructions instead of one).
+// high half.  The distance to a bound plane is one mixed-precision fma, bound * (1/d) + (-o * (1/d)), with
+// the binary16 bound read from its half of the word (v_fma_mix_f32).
 //
 // A ray's side of the test, set once per query (RaySlab): per axis, the rotation that brings the
 // near bound of a bound word into its low half (0 when the reciprocal direction is >= 0, where lo is
-// nearer; 16 otherwise), and the reciprocal for the far bound scaled by the slack.  Choosing near and
-// far by the direction's sign gives the values a min and a max of the two distances would (rounding
-// is monotone), with no min/max pair per axis.  The slack applied to the far reciprocal and to the
-// limit, rather than to the exit distance as slab() does, differs by rounding far below the slack
-// itself, so the test stays conservative.  Where a distance is NaN (a ray in a bound's plane with an
-// infinite reciprocal) the test ignores that axis's bound, which only accepts more boxes.
+// nearer; 16 otherwise), the reciprocal, and the offset -o/d once lowered (near) and once raised (far)
+// by 2^-21 of itself.  Choosing near and far by the direction's sign gives the values a min and a max
+// of the two distances would (rounding is monotone), with no min/max pair per axis.
+//
+// Against slab()'s (bound - o) * (1/d) the rounded product o * (1/d) brings an error of at most 2^-24
+// of itself, and the fma's own rounding the relative error that slab() has too; the widened offsets
+// cover the first eight times over, and the slack on the exit distance is slab()'s.  So the test accepts
+// every box slab() accepts and a few more.  The reciprocal is held to +-2^100: a larger one (a ray
+// in an axis plane) would make bound * (1/d) + (-o/d) infinity minus infinity.  At that size a plane at
+// any distance a binary32 coordinate shows is beyond every query's limit (1e20), so the clamp changes no
+// answer.  Where a distance is NaN all the same (an origin beyond 1e8 on such a ray) the test ignores
+// that axis's bound, which only accepts more boxes.
 struct RaySlab {
     unsigned rx, ry, rz;
-    f3 inv_far;
+    f3 inv, on, of;
 };
-__device__ __forceinline__ RaySlab ray_slab(f3 inv) {
+__device__ __forceinline__ RaySlab ray_slab_inv(f3 o, f3 inv) {
     RaySlab r;
+    r.inv = inv;
     r.rx = inv.x >= 0.f ? 0u : 16u;
     r.ry = inv.y >= 0.f ? 0u : 16u;
     r.rz = inv.z >= 0.f ? 0u : 16u;
-    r.inv_far = mk(inv.x * kSlack, inv.y * kSlack, inv.z * kSlack);
+    constexpr float kWiden = 4.76837158e-7f;   // 2^-21
+    const f3 p = mk(-o.x * inv.x, -o.y * inv.y, -o.z * inv.z);
+    r.on = mk(p.x - fabsf(p.x) * kWiden, p.y - fabsf(p.y) * kWiden, p.z - fabsf(p.z) * kWiden);
+    r.of = mk(p.x + fabsf(p.x) * kWiden, p.y + fabsf(p.y) * kWiden, p.z + fabsf(p.z) * kWiden);
     return r;
 }
+__device__ __forceinline__ RaySlab ray_slab(f3 o, f3 d) {
+    // the hardware's reciprocal (one ulp): it scales both of an axis's distances alike, far within the slack
+    constexpr float kMost = 0x1p100f;
+    auto inv = [](float x) { return fminf(fmaxf(__builtin_amdgcn_rcpf(x), -kMost), kMost); };
+    return ray_slab_inv(o, mk(inv(d.x), inv(d.y), inv(d.z)));
+}
 
-// tlimit_s: the query's limit times kSlack
-__device__ __forceinline__ float slab_hn(unsigned wx, unsigned wy, unsigned wz, f3 o, f3 inv, const RaySlab &rs,
-                                         float tlimit_s, float one) {
+// The entry distance's bits (as an unsigned number they order as the distances do), at least 4, or 0 on a miss.
+constexpr float kLeastEntry = 0x1p-147f;   // bits 4: the low two bits of a hit's key are free for a child's slot
+__device__ __forceinline__ unsigned slab_hn(unsigned wx, unsigned wy, unsigned wz, const RaySlab &rs, float tlimit) {
     const unsigned nx = __builtin_amdgcn_alignbit(wx, wx, rs.rx);
     const unsigned ny = __builtin_amdgcn_alignbit(wy, wy, rs.ry);
     const unsigned nz = __builtin_amdgcn_alignbit(wz, wz, rs.rz);
-    const float tnx = __builtin_fmaf(half_lo(nx), one, -o.x) * inv.x;
-    const float tfx = __builtin_fmaf(half_hi(nx), one, -o.x) * rs.inv_far.x;
-    const float tny = __builtin_fmaf(half_lo(ny), one, -o.y) * inv.y;
-    const float tfy = __builtin_fmaf(half_hi(ny), one, -o.y) * rs.inv_far.y;
-    const float tnz = __builtin_fmaf(half_lo(nz), one, -o.z) * inv.z;
-    const float tfz = __builtin_fmaf(half_hi(nz), one, -o.z) * rs.inv_far.z;
-    const float tn = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, 0.f));
-    const float tf = fminf(fminf(tfx, tfy), fminf(tfz, tlimit_s));
-    return tn <= tf ? tn : __builtin_inff();
+    const float tnx = __builtin_fmaf(half_lo(nx), rs.inv.x, rs.on.x);
+    const float tfx = __builtin_fmaf(half_hi(nx), rs.inv.x, rs.of.x);
+    const float tny = __builtin_fmaf(half_lo(ny), rs.inv.y, rs.on.y);
+    const float tfy = __builtin_fmaf(half_hi(ny), rs.inv.y, rs.of.y);
+    const float tnz = __builtin_fmaf(half_lo(nz), rs.inv.z, rs.on.z);
+    const float tfz = __builtin_fmaf(half_hi(nz), rs.inv.z, rs.of.z);
+    const float tn = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, kLeastEntry));
+    const float tf = fminf(fminf(tfx, tfy), fminf(tfz, tlimit));
+    return tn <= tf * kSlack ? __float_as_uint(tn) : 0u;
 }
 
 // Closest hit over a prepared structure.  Returns the hit shape index or -1; t in *tout.
@@ -350,7 +391,7 @@ __device__ __forceinline__ bool anyhit(const DevAccel &A, f3 o, f3 d, float maxt
 // ---- camera ray, rendering_kernel.cl:1042-1070 ----
 PT_HD void camera_ray(const Camera *cam, unsigned &s0, unsigned &s1, int width, int height,
                                            int x, int y, f3 &ro, f3 &rd) {
-    const float invW = 1.f / (float)width, invH = 1.f / (float)height;
+    const float invW = rcp_exact((float)width), invH = rcp_exact((float)height);
     const float r1 = get_random(s0, s1) - .5f;
     const float r2 = get_random(s0, s1) - .5f;
     const float kcx = ((float)x + r1) * invW - .5f;
@@ -410,7 +451,7 @@ PT_HD bool sample_light_words(const float *lw, float area, unsigned &s0, unsigne
     if (ltype == TRIANGLE) {
         const float u1 = get_random(s0, s1);
         const float u2 = get_random(s0, s1);
-        const float su1 = sqrtf(u1);
+        const float su1 = sqrt_exact(u1);
         const float bu = 1.0f - su1, bv = u2 * su1;
         const f3 p1 = mk(lw[1], lw[2], lw[3]);
         f3 e1 = sub3(mk(lw[4], lw[5], lw[6]), p1), e2 = sub3(mk(lw[7], lw[8], lw[9]), p1);
@@ -423,7 +464,7 @@ PT_HD bool sample_light_words(const float *lw, float area, unsigned &s0, unsigne
         const float u2 = get_random(s0, s1);
         const float zz = 1.f - 2.f * u1;
         const float q = 1.f - zz * zz;
-        const float rr = sqrtf(0.f < q ? q : 0.f);
+        const float rr = sqrt_exact(0.f < q ? q : 0.f);
         const float phi = 2.f * kPi * u2;
         float sphi, cphi;
         sincos_f32(phi, &sphi, &cphi);
@@ -432,8 +473,8 @@ PT_HD bool sample_light_words(const float *lw, float area, unsigned &s0, unsigne
         ln = usp;
     }
     f3 sd = sub3(lp, hp);
-    const float len = sqrtf(dot3(sd, sd));
-    sd = smul(1.f / len, sd);
+    const float len = sqrt_exact(dot3(sd, sd));
+    sd = smul(rcp_exact(len), sd);
     float wo = dot3(sd, ln);
     if (wo > 0.f) return false;
     wo = -wo;
@@ -463,7 +504,7 @@ PT_HD bool sample_light(const Shape *L, unsigned &s0, unsigned &s1, f3 hp, f3 nl
 PT_HD f3 diffuse_dir(f3 nl, unsigned &s0, unsigned &s1) {
     const float r1 = 2.f * kPi * get_random(s0, s1);
     const float r2 = get_random(s0, s1);
-    const float r2s = sqrtf(r2);
+    const float r2s = sqrt_exact(r2);
     f3 ww = nl;
     const f3 aa = fabsf(ww.x) > .1f ? mk(0.f, 1.f, 0.f) : mk(1.f, 0.f, 0.f);
     f3 u = norm3(cross3(aa, ww));
@@ -473,7 +514,7 @@ PT_HD f3 diffuse_dir(f3 nl, unsigned &s0, unsigned &s1) {
     u = smul(cr1 * r2s, u);
     v = smul(sr1 * r2s, v);
     f3 nd = add3(u, v);
-    ww = smul(sqrtf(1 - r2), ww);
+    ww = smul(sqrt_exact(1 - r2), ww);
     return add3(nd, ww);
 }
 
@@ -496,7 +537,7 @@ PT_HD void specular_or_refract(const Surface &S, f3 &rd, f3 &thr, unsigned &s0, 
         rd = nd;
         return;
     }
-    const float kk = (float)(into ? 1 : -1) * (ddn * nnt + sqrtf(cos2t));
+    const float kk = (float)(into ? 1 : -1) * (ddn * nnt + sqrt_exact(cos2t));
     const f3 nkk = smul(kk, S.nrm);
     f3 td = smul(nnt, rd);
     td = sub3(td, nkk);
@@ -524,7 +565,7 @@ PT_HD void specular_or_refract(const Surface &S, f3 &rd, f3 &thr, unsigned &s0, 
 PT_HD f3 running_mean(f3 col, f3 rad, int cs) {
     if (cs == 0) return rad;
     const float k1 = (float)cs;
-    const float k2 = 1.f / ((float)cs + 1.f);
+    const float k2 = rcp_exact((float)cs + 1.f);
     return mk((col.x * k1 + rad.x) * k2, (col.y * k1 + rad.y) * k2, (col.z * k1 + rad.z) * k2);
 }
 

@@ -103,11 +103,13 @@ struct Frame {
 
 struct SavedTuning {
     int bpc, regroup, wide, bbpc, bregroup;
+    bool bauto;
     explicit SavedTuning(const ptgpu_ctx *c)
         : bpc(c->blocks_per_cu), regroup(c->regroup), wide(c->wide), bbpc(c->batch_blocks_per_cu),
-          bregroup(c->batch_regroup) {}
+          bregroup(c->batch_regroup), bauto(c->blocks_auto) {}
     void restore(ptgpu_ctx *c) const {
         c->blocks_per_cu = bpc;
+        c->blocks_auto = bauto;
         c->regroup = regroup;
         c->wide = wide;
         c->batch_blocks_per_cu = bbpc;
@@ -148,6 +150,7 @@ int autotune_frame(ptgpu_ctx *ctx, ptgpu_clbvh *h, const ptgpu_render_args *a, i
     // a launch that asks for more than half of a CU's workgroups leaves it no room (measured: three or
     // four per CU render one frame alone as fast, but frames in flight 2-5% slower at C2).
     const int bpc_max = frames_per_build == 0 ? 2 : 4;
+    ctx->blocks_auto = false;
     for (int wide : {2, 1, 0})
         for (int bpc = 1; bpc <= bpc_max; bpc++)
             for (int rg : {8, 16, 32}) {
