@@ -132,7 +132,7 @@ int ptgpu_ctx_set_engine(ptgpu_ctx *ctx, int engine);
  * every primitive, with the same result; 1 the default, 0 off: about 2.6% less time for one frame
  * alone, 4% less throughput with frames in flight at C2; 2 walks every binary16 tree on an 8-entry
  * stack, a test setting);
- * "batch_regroup" and "batch_blocks_per_cu" (the same for ptgpu_render_batch, defaults 32 and 3). */
+ * "batch_regroup" and "batch_blocks_per_cu" (the same for ptgpu_render_batch, defaults 40 and 3). */
 int ptgpu_ctx_set_tuning(ptgpu_ctx *ctx, const char *name, int value);
 int ptgpu_malloc(ptgpu_ctx *ctx, size_t bytes, void **d_out);
 int ptgpu_free(ptgpu_ctx *ctx, void *d_ptr);

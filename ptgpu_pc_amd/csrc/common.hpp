@@ -191,7 +191,7 @@ struct ptgpu_ctx {
     int engine = 0;      // 0 auto, 1 megakernel (lockstep queries), 2 wavefront, 3 megakernel (per-lane states)
     int regroup = 24;   // per-lane-state megakernel: ready lanes that trigger a shading pass
     int quad = 16;      // per-lane-state megakernel, binary16 nodes: traversing lanes at or below which four lanes share a query
-    int batch_regroup = 32;
+    int batch_regroup = 40;
     int blocks_per_cu = 2;        // single-frame renders
     bool blocks_auto = true;      // until "blocks_per_cu" is set, the launch picks (launch_shape, render.hip)
     int batch_blocks_per_cu = 3;  // batched renders: throughput-bound, more waves per SIMD
@@ -203,6 +203,7 @@ struct ptgpu_ctx {
     ptgpu::DevBuf tmp_nodes, tmp_nodes4, tmp_prims, tmp_lights, tmp_scan, tmp_counter;
     ptgpu::DevBuf tmp_parents;           // parent map and height of a caller's BVH (ptgpu_radiance_gpu)
     ptgpu::DevBuf tmp_tiles;             // tile origins of RadianceBoxGPU launches
+    ptgpu::DevBuf pack_tab;              // thresholds of the RGBA8 pack, filled when the context is made
     ptgpu::DevBuf rec_status;            // recorded renders' device-side checks: flags, height seen
     ptgpu::BatchChannel batch;            // ptgpu_render_batch launches (on the context's stream)
     ptgpu::BuildStaging build_staging;    // batched LBVH builds
@@ -225,6 +226,7 @@ namespace ptgpu {
 // (the scan order of SampleLights, rendering_kernel.cl:415-423).  Writes *found on the host.
 int build_light_list(ptgpu_ctx *ctx, const Shape *d_shapes, int n, int light_cnt, DevBuf &out_lights,
                      DevBuf &scan_tmp, int *found);
+int build_pack_table(ptgpu_ctx *ctx);
 // brute-force layout: prims in shape-index order
 int build_index_prims(ptgpu_ctx *ctx, const Shape *d_shapes, int n, DevBuf &out_prims);
 // four-wide nodes for a prepared binary structure (no-op without internal nodes); sets acc->nodes4

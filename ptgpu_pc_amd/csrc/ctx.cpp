@@ -126,6 +126,7 @@ int ptgpu_ctx_create(int device, void *stream, ptgpu_ctx **out) {
     // status words of recorded renders (allocated here: a recording must not be the first to allocate)
     int s = c->rec_status.ensure(16);
     if (s == PTGPU_OK) s = ptgpu::fill_u32(c->stream, c->rec_status.p, 0u, 4);
+    if (s == PTGPU_OK) s = ptgpu::build_pack_table(c);
     if (s != PTGPU_OK) {
         ptgpu_ctx_destroy(c);
         return s;
@@ -147,6 +148,7 @@ int ptgpu_ctx_destroy(ptgpu_ctx *ctx) {
     ctx->tmp_parents.release();
     ctx->tmp_tiles.release();
     ctx->rec_status.release();
+    ctx->pack_tab.release();
     ptgpu::release_stages(ctx->rec_stages);
     ctx->batch.release();
     ctx->build_staging.release();

@@ -407,6 +407,28 @@ PT_HD int to_int(float x) {   // vec.h:60 with the OpenCL clamp builtin
 }
 
 
+// The same byte from a table: entry k (1..255) is the least x whose to_int is at least k, entry 0 is -infinity and
+// entry 256 infinity.  The kernel's own to_int fills it (k_pack_table), a hardware log2 / exp2 guesses the byte and
+// the table settles it, in about 20 instructions instead of the 150 of powf, which every shading pass that
+// finished a pixel ran three times.  powf is not monotone in its last bits (of all binary32 x two lie one and two
+// places beyond a threshold on the wrong side), so a wave with an x within four places of one calls to_int:
+// the result is to_int's (compared for every binary32 x).
+constexpr int kPackEntries = 257;
+__device__ __forceinline__ int to_int_tab(float x, const float *tab) {
+    x = fminf(fmaxf(x, 0.f), 1.f);
+    int g = (int)(__builtin_amdgcn_exp2f(__builtin_amdgcn_logf(x) * (1.f / 2.2f)) * 255.f + .5f);
+    g = g < 255 ? g : 255;
+    const float lo = tab[g], hi = tab[g + 1];
+    const int b = __float_as_int(x);
+    const bool near = (unsigned)(b - __float_as_int(lo) + 4) <= 8u || (unsigned)(b - __float_as_int(hi) + 4) <= 8u;
+    if (__builtin_expect(__ballot(near) != 0ull, 0)) return to_int(x);
+    return g + (x >= hi) - (x < lo);
+}
+__device__ __forceinline__ unsigned pack_rgba_tab(f3 col, const float *tab) {
+    return (unsigned)to_int_tab(col.x, tab) | ((unsigned)to_int_tab(col.y, tab) << 8) |
+           ((unsigned)to_int_tab(col.z, tab) << 16) | 0xff000000u;
+}
+
 // ---- surface at a hit (rendering_kernel.cl:550-598) ----
 struct Surface {
     f3 nrm, nl, e, c;
