@@ -63,8 +63,12 @@ constexpr float kFarBox = 1e30f;   // coordinates of an unused TNode4 slot
 // and every ray that hits the fp32 box hits it too; the walk may visit a few more nodes, never
 // fewer, and the hits are the same.  One 16-byte word per child k: (x, y, z, ref), each axis as
 // lo in the low half and hi in the high half, so one lane can fetch one child in one load.  Leaves
-// are runs of primitives ending in kLastInLeaf (trees with leaf_runs only).  An unused slot holds
-// +inf bounds, which no ray hits.
+// are runs of primitives ending in kLastInLeaf (trees with leaf_runs only).  An unused slot holds the
+// inverted bounds kEmptyHalf (lo = +inf, hi = -inf): near is +inf and far -inf on an axis where the ray's
+// origin and reciprocal direction are ordinary numbers, whatever the limit.  A ray with infinite or NaN
+// components on all three can pass any box test, so the slot's reference is the run of primitive 0, which
+// every tree has: testing it again changes no result.
+constexpr unsigned kEmptyHalf = 0xFC007C00u;
 struct alignas(16) TNode4H {
     uint4 c[4];
 };

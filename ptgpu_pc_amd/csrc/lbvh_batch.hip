@@ -382,7 +382,8 @@ int build_batch(ptgpu_ctx *ctx, ptgpu_clbvh *const *hs, int ns) {
         h->sorted = h->valsA.as<unsigned>();
         for (bool &t : h->timed) t = false;
         clbvh_mark_built(h);
-        if (h->height_pending) {
+        // a tree whose build failed keeps its height pending: every use reads its error word and is refused
+        if (h->height_pending && h_out[ns + s] == 0) {
             h->acc.depth = (int)h_out[s];
             h->known_height[0] = (int)h_out[s];
             h->height_pending = false;

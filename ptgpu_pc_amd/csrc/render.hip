@@ -113,8 +113,7 @@ __device__ __forceinline__ bool camera_outside(const RenderParams &P) {
     const float inf = __builtin_inff();
     f3 lo = mk(inf, inf, inf), hi = mk(-inf, -inf, -inf);
     for (int k = 0; k < 4; k++) {
-        const uint4 c = r.c[k];
-        if ((int)c.w == kEmptyRef) continue;
+        const uint4 c = r.c[k];   // an unused slot's inverted bounds change neither
         lo = mk(fminf(lo.x, half_lo(c.x)), fminf(lo.y, half_lo(c.y)), fminf(lo.z, half_lo(c.z)));
         hi = mk(fmaxf(hi.x, half_hi(c.x)), fmaxf(hi.y, half_hi(c.y)), fmaxf(hi.z, half_hi(c.z)));
     }
@@ -984,13 +983,15 @@ __global__ __launch_bounds__(256) void k_half4(const TNode4 *__restrict__ in, in
     const float hi[3][4] = {{t.hix.x, t.hix.y, t.hix.z, t.hix.w}, {t.hiy.x, t.hiy.y, t.hiy.z, t.hiy.w},
                             {t.hiz.x, t.hiz.y, t.hiz.z, t.hiz.w}};
     const int ref[4] = {t.ref.x, t.ref.y, t.ref.z, t.ref.w};
-    unsigned w[3][4];
-    for (int a = 0; a < 3; a++)
-        for (int k = 0; k < 4; k++)
-            w[a][k] = ref[k] == kEmptyRef ? 0x7C007C00u
-                                          : (unsigned)half_down(lo[a][k]) | ((unsigned)half_up(hi[a][k]) << 16);
+    const int cnt[4] = {t.cnt.x, t.cnt.y, t.cnt.z, t.cnt.w};
     TNode4H o;
-    for (int k = 0; k < 4; k++) o.c[k] = make_uint4(w[0][k], w[1][k], w[2][k], (unsigned)ref[k]);
+    for (int k = 0; k < 4; k++) {
+        unsigned w[3];
+        const bool empty = ref[k] == kEmptyRef || (ref[k] < 0 && cnt[k] <= 0);   // a leaf without primitives has no run
+        for (int a = 0; a < 3; a++)
+            w[a] = empty ? kEmptyHalf : (unsigned)half_down(lo[a][k]) | ((unsigned)half_up(hi[a][k]) << 16);
+        o.c[k] = make_uint4(w[0], w[1], w[2], empty ? ~0u : (unsigned)ref[k]);
+    }
     out[i] = o;
 }
 

@@ -162,8 +162,7 @@ __device__ __forceinline__ bool half_step(HalfWalk &W, const HalfTree &T, int *s
         const unsigned t0 = slab_hn(q0.x, q0.y, q0.z, W.rs, W.tb), t1 = slab_hn(q1.x, q1.y, q1.z, W.rs, W.tb);
         const unsigned t2 = slab_hn(q2.x, q2.y, q2.z, W.rs, W.tb), t3 = slab_hn(q3.x, q3.y, q3.z, W.rs, W.tb);
         if (STATS)
-            *st_nodes += ((int)q0.w != kEmptyRef) + ((int)q1.w != kEmptyRef) + ((int)q2.w != kEmptyRef) +
-                         ((int)q3.w != kEmptyRef);
+            *st_nodes += (q0.x != kEmptyHalf) + (q1.x != kEmptyHalf) + (q2.x != kEmptyHalf) + (q3.x != kEmptyHalf);
         const unsigned k0 = t0 & ~3u, k1 = (t1 & ~3u) | 1u, k2 = (t2 & ~3u) | 2u, k3 = t3 | 3u;
         const int c01 = k0 < k1, c02 = k0 < k2, c03 = k0 < k3, c12 = k1 < k2, c13 = k1 < k3, c23 = k2 < k3;
         const int p0 = c01 + c02 + c03, p1 = 1 - c01 + c12 + c13, p2 = 2 - c02 - c12 + c23, p3 = 3 - c03 - c13 - c23;
@@ -324,7 +323,7 @@ __device__ __forceinline__ bool half_sparse(HalfWalk &W, const HalfTree &T, int 
         if (inner) {
             cref = (int)w.w;
             key = slab_hn(w.x, w.y, w.z, rs, tb);
-            if (STATS) *st_nodes += cref != kEmptyRef;
+            if (STATS) *st_nodes += w.x != kEmptyHalf;
         }
         const bool hit = key != 0u;
         key = (key & ~3u) | (unsigned)qc;

@@ -121,3 +121,26 @@ def test_axis_rays_and_far_origins(ctx):
     for a, b in ((out[0], out[1]), (out[2], out[3])):
         for x, y in zip(a, b):
             assert x.tobytes() == y.tobytes()
+
+
+@pytest.mark.parametrize("orig", [(np.nan,) * 3, (np.inf, np.inf, np.inf), (-np.inf, np.inf, 0.5), (np.nan, 0.5, 0.5)])
+def test_camera_not_finite(orig):
+    """Rays that pass every box test reach the unused slots of nodes too: they end, and the image is the binary
+    walk's."""
+    say("case camera not finite", orig)
+    s, lc, cam = _scene("soup", 65, 33)
+    cam["orig"][0] = orig
+    out = []
+    with pt.Context(0) as ctx:
+        d_sh, d_cam = ctx.to_device(s), ctx.to_device(cam)
+        bvh = pt.CLBVH(ctx, d_sh)
+        bvh.buildRadixTree()
+        bvh.buildBVHTree()
+        for quad, wide in ((8, 2), (0, 2), (0, 0)):
+            ctx.set_tuning("quad", quad)
+            ctx.set_tuning("wide", wide)
+            out.append(_frame(ctx, bvh, d_sh, len(s), lc, d_cam, 65, 33, 1, 3))
+        bvh.close()
+    for a, b, c in zip(*out):
+        assert a.tobytes() == b.tobytes()
+        assert a.tobytes() == c.tobytes()
