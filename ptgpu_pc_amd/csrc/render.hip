@@ -842,6 +842,157 @@ __global__ __launch_bounds__(256) void k_trace(DevAccel A, const Ray *rays, cons
     }
 }
 
+// binary16 bounds rounded outward: the nearest binary16 (round to nearest even), stepped one
+// binary16 ulp down (lo) or up (hi) when it lies on the wrong side of x.  A NaN bound becomes the
+// infinity on its own side; values beyond the binary16 range round to +-65504 or the infinity.
+__device__ __forceinline__ unsigned short half_down(float x) {
+    if (x != x) return 0xFC00u;   // -inf
+    const _Float16 h = (_Float16)x;
+    unsigned short b = __builtin_bit_cast(unsigned short, h);
+    if ((float)h > x) {
+        if (b == 0x0000u || b == 0x8000u) b = 0x8001u;   // +-0 -> the largest negative subnormal
+        else if (b & 0x8000u) b = (unsigned short)(b + 1u);   // negative: away from zero
+        else b = (unsigned short)(b - 1u);                    // positive: toward zero
+    }
+    return b;
+}
+__device__ __forceinline__ unsigned short half_up(float x) {
+    if (x != x) return 0x7C00u;   // +inf
+    const _Float16 h = (_Float16)x;
+    unsigned short b = __builtin_bit_cast(unsigned short, h);
+    if ((float)h < x) {
+        if (b == 0x0000u || b == 0x8000u) b = 0x0001u;   // +-0 -> the smallest positive subnormal
+        else if (b & 0x8000u) b = (unsigned short)(b - 1u);   // negative: toward zero
+        else b = (unsigned short)(b + 1u);                    // positive: away from zero
+    }
+    return b;
+}
+
+// Do binary16 bounds blur this tree?  They are absolute, so a scene far from the origin (or past 65,504) has
+// boxes a binary16 step wide, whatever its shapes' size, and a walk of them visits much of the tree.  Each lane
+// widens the leaf boxes of one node, spread evenly over the tree, and the wave compares the areas' sums:
+// one answer for all waves of a launch.  At a sum over four times the exact one the two walks cost alike (100,000
+// rays; the scene moved by 16: 1,002-shape soup 67 us here against 71 over binary nodes, 327,692-shape mesh 413
+// against 236; by 256: 256 against 73 us, 146 against 0.24 ms).
+__device__ __forceinline__ bool half_blurs(const DevAccel &A) {
+    const int at = (int)((long long)__lane_id() * A.nnodes / kWave);
+    const TNode t = A.nodes[at];
+    float exact = 0.f, wide = 0.f;
+    auto add = [&](int r, float x0, float y0, float z0, float x1, float y1, float z1) {
+        auto area = [](float dx, float dy, float dz) { return dx * dy + dy * dz + dz * dx; };
+        auto lo = [](float v) { return (float)__builtin_bit_cast(_Float16, half_down(v)); };
+        auto hi = [](float v) { return (float)__builtin_bit_cast(_Float16, half_up(v)); };
+        if (r >= 0 || r == kEmptyRef) return;
+        exact += area(x1 - x0, y1 - y0, z1 - z0);
+        wide += area(hi(x1) - lo(x0), hi(y1) - lo(y0), hi(z1) - lo(z0));
+    };
+    add(t.r.x, t.a.x, t.a.y, t.a.z, t.a.w, t.b.x, t.b.y);
+    add(t.r.y, t.b.z, t.b.w, t.c.x, t.c.y, t.c.z, t.c.w);
+    for (int x = 1; x < kWave; x <<= 1) {
+        exact += __shfl_xor(exact, x);
+        wide += __shfl_xor(wide, x);
+    }
+    return __builtin_amdgcn_readfirstlane((int)(wide > 4.f * exact)) != 0;
+}
+
+// The same queries over binary16 four-wide nodes.  A lane whose query ends takes the wave's next ray once eight
+// lanes (or a quarter of those that still have work) have ended, so the wave's steps stay full, where one ray per
+// thread over binary nodes let the longest of 64 hold the others; few rays are spread over all waves, whose idle
+// lanes share them (half_sparse), and so is the end of a larger batch.  A wave's rays are fixed by its number, in
+// runs of sixteen from all over the batch: neighbours in the batch often cost alike, and a counter that all waves
+// take rays from cost more than it evened out (0.74 ms with one stretch a wave, 2 ms with the counter).  Bound by
+// the step's instructions and its loads.  One million closest-hit and as many any-hit queries of a 65,538-shape
+// soup, half of them from inside it in any direction: 1.42 -> 0.65 ms; 30,000: 0.53 -> 0.12; 1,000: 0.43 -> 0.063.
+template <int STACK>
+__global__ __launch_bounds__(256, STACK <= 36 ? 4 : 2) void k_trace_half(DevAccel A, const Ray *rays, const float *maxt,
+                                                                         int n, float *tout, int *idout, int *hitout,
+                                                                         int any, int lanes, int regroup_max, int quad,
+                                                                         int slack) {
+    __shared__ int s_stack[STACK * 256];
+    int *const stk = s_stack + threadIdx.x;
+    if (half_blurs(A)) {
+        // one ray per thread over the binary nodes; every four-wide stack class holds their walk
+        for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
+            const float *rf = reinterpret_cast<const float *>(rays + i);
+            const f3 o = mk(rf[0], rf[1], rf[2]), d = mk(rf[3], rf[4], rf[5]);
+            if (any) {
+                hitout[i] = anyhit<STACK>(A, o, d, maxt[i], stk, nullptr, nullptr) ? 1 : 0;
+            } else {
+                float t;
+                const int id = closest<STACK>(A, o, d, &t, stk, nullptr, nullptr);
+                tout[i] = id >= 0 ? t : 0.f;
+                idout[i] = id;
+            }
+        }
+        return;
+    }
+    HalfTree T;
+    T.nodes = to_gmem(A.nodes4h);
+    T.prims = to_gmem(A.prims);
+    T.nprims = A.nprims;
+    T.skip = A.nshapes - 1;
+    const unsigned long long lt = lanemask_lt();
+    // the wave's own share of the rays: every waves-th run of sixteen (of lanes, where fewer work)
+    const long long wave = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int run = lanes < 16 ? lanes : 16;
+    const long long stride = (long long)gridDim.x * 4 * run;
+    const int shift = __ffs(run) - 1;
+    int next = 0;
+    enum : int { kWant, kWalk, kDone, kOut };
+    int st = (int)__lane_id() < lanes ? kWant : kOut;
+    int cur = 0;
+    HalfWalk W;
+    W.o = W.d = mk(0.f, 0.f, 1.f);
+    W.rs = ray_slab(W.o, W.d);
+    W.tb = 0.f;
+    W.bid = -1;
+    W.node = W.leaf = W.sp = 0;
+    W.any = any != 0;
+    for (;;) {
+        // results of the finished queries, then the next rays
+        if (st == kDone) {
+            if (any) {
+                hitout[cur] = W.bid >= 0 ? 1 : 0;
+            } else {
+                tout[cur] = W.bid >= 0 ? W.tb : 0.f;
+                idout[cur] = W.bid;
+            }
+            st = kWant;
+        }
+        const unsigned long long want = __ballot(st == kWant);
+        if (st == kWant) {
+            const int p = next + (int)__popcll(want & lt);
+            const long long at = (p >> shift) * stride + wave * run + (p & (run - 1));
+            if (at < n) {
+                cur = (int)at;
+                const float *rf = reinterpret_cast<const float *>(rays + cur);
+                W.o = mk(rf[0], rf[1], rf[2]);
+                W.d = mk(rf[3], rf[4], rf[5]);
+                W.tb = any ? maxt[cur] : kInf;
+                half_start(W, A.root);
+                st = kWalk;
+            } else {
+                st = kOut;
+            }
+        }
+        next += (int)__popcll(want);
+        const unsigned long long live = __ballot(st != kOut);
+        if (!live) break;
+        const unsigned quarter = ((unsigned)__popcll(live) + 3u) >> 2;
+        const unsigned regroup = (unsigned)regroup_max < quarter ? (unsigned)regroup_max : quarter;
+        unsigned long long walk;
+        for (;;) {
+            walk = __ballot(st == kWalk);
+            if (__popcll(walk) <= quad || (unsigned)__popcll(live & ~walk) >= regroup) break;
+            if (st == kWalk && half_step<STACK, false>(W, T, stk, nullptr, nullptr)) st = kDone;
+        }
+        const unsigned ready = (unsigned)__popcll(live & ~walk);
+        if (walk && ready < regroup &&
+            half_sparse<STACK, false, false>(W, T, slack, st == kWalk, walk, ready, regroup, s_stack, nullptr, nullptr))
+            st = kDone;
+    }
+}
+
 // ---- scene preparation kernels ----
 __global__ void k_index_prims(const Shape *shapes, int n, Prim *prims) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -945,32 +1096,6 @@ __global__ __launch_bounds__(256) void k_collapse4(const TNode *__restrict__ bn,
     o.ref = make_int4(ref[0], ref[1], ref[2], ref[3]);
     o.cnt = make_int4(cnt[0], cnt[1], cnt[2], cnt[3]);
     out[i] = o;
-}
-
-// binary16 bounds rounded outward: the nearest binary16 (round to nearest even), stepped one
-// binary16 ulp down (lo) or up (hi) when it lies on the wrong side of x.  A NaN bound becomes the
-// infinity on its own side; values beyond the binary16 range round to +-65504 or the infinity.
-__device__ __forceinline__ unsigned short half_down(float x) {
-    if (x != x) return 0xFC00u;   // -inf
-    const _Float16 h = (_Float16)x;
-    unsigned short b = __builtin_bit_cast(unsigned short, h);
-    if ((float)h > x) {
-        if (b == 0x0000u || b == 0x8000u) b = 0x8001u;   // +-0 -> the largest negative subnormal
-        else if (b & 0x8000u) b = (unsigned short)(b + 1u);   // negative: away from zero
-        else b = (unsigned short)(b - 1u);                    // positive: toward zero
-    }
-    return b;
-}
-__device__ __forceinline__ unsigned short half_up(float x) {
-    if (x != x) return 0x7C00u;   // +inf
-    const _Float16 h = (_Float16)x;
-    unsigned short b = __builtin_bit_cast(unsigned short, h);
-    if ((float)h < x) {
-        if (b == 0x0000u || b == 0x8000u) b = 0x0001u;   // +-0 -> the smallest positive subnormal
-        else if (b & 0x8000u) b = (unsigned short)(b - 1u);   // negative: toward zero
-        else b = (unsigned short)(b + 1u);                    // positive: away from zero
-    }
-    return b;
 }
 
 // TNode4 -> TNode4H (leaf counts dropped: leaves are runs ending in kLastInLeaf)
@@ -1428,6 +1553,31 @@ int launch_trace(ptgpu_ctx *ctx, const DevAccel &acc, unsigned int shapeCnt, con
     if (n <= 0) return PTGPU_OK;
     PT_CHECK(!acc.height_check, PTGPU_ERR_UNSUPPORTED,
              "batch queries cannot be recorded before the tree height was read back");
+    const int sw = acc.nodes4h && acc.root >= 0 && ctx->wide == 2 ? stack_for_wide(acc, ctx->stack_min) : -1;
+    if (sw > 0) {
+        // Few rays are spread as launch_shape spreads few pixels.  Four workgroups of the 32-entry stack on a CU
+        // (five would fit: 0.80 against 0.71 ms for 20,000 shapes and a million rays); under the short stack, which
+        // trees past 32 entries take, three for a batch that fills all lanes (0.64 against 0.72 ms for 65,538
+        // shapes) and four for one that is spread (30,000 rays: 111 against 137 us).
+        const int cus = ctx->cu_count;
+        int lanes = 1;
+        while (lanes < kWave && n > lanes * 16 * cus) lanes *= 2;
+        if (lanes > 8 || ctx->quad == 0) lanes = kWave;
+        const bool shortst = sw == 48 && ctx->short_stack != 0;
+        const int per_cu = sw == 32 ? 4 : shortst ? (lanes == kWave ? 3 : 4) : sw == 48 ? 3 : 2;
+        long long blocks = ((long long)n + 4 * lanes - 1) / (4 * lanes);
+        if (blocks > (long long)cus * per_cu) blocks = (long long)cus * per_cu;
+#define PT_TRACE(ST)                                                                                                  \
+    hipLaunchKernelGGL(k_trace_half<ST>, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, acc, d_rays, d_maxt, n, d_t, d_id, \
+                       d_hit, any ? 1 : 0, lanes, 8, ctx->quad, half_slack(ST, acc))
+        if (sw == 32) PT_TRACE(32);
+        else if (shortst) PT_TRACE(kStackShort);
+        else if (sw == 48) PT_TRACE(48);
+        else PT_TRACE(64);
+#undef PT_TRACE
+        PT_HIP(hipGetLastError());
+        return PTGPU_OK;
+    }
     const int st = stack_for(acc, ctx->stack_min);
     PT_CHECK(st > 0, PTGPU_ERR_UNSUPPORTED, "tree depth %d exceeds the 62-level traversal stack", acc.depth);
     if (st == 24)
