@@ -22,6 +22,15 @@ __global__ void k_fill_u32(unsigned *p, unsigned v, size_t n) {
     for (; i < n; i += stride) p[i] = v;
 }
 
+__global__ void k_clear3(unsigned *p, size_t np, unsigned *q, int nq, unsigned *r, int nr) {
+    const size_t stride = (size_t)gridDim.x * blockDim.x;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < np + nq + nr; i += stride) {
+        if (i < np) p[i] = 0u;
+        else if (i < np + nq) q[i - np] = 0u;
+        else r[i - np - nq] = 0u;
+    }
+}
+
 __global__ void k_fill_u8(unsigned char *p, unsigned char v, size_t n) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     size_t stride = (size_t)gridDim.x * blockDim.x;
@@ -106,32 +115,11 @@ __global__ __launch_bounds__(256) void k_refit_levels(const ShapeBox *boxes, con
                             blockIdx.x);
 }
 
-__global__ __launch_bounds__(256) void k_karras_morton(const unsigned *keys, int n, int4 *mnode, int *mpar_int,
-                                                       int *mpar_leaf) {
-    karras_morton_body(keys, n, mnode, mpar_int, mpar_leaf, blockIdx.x);
-}
-
-__global__ __launch_bounds__(kMChunk) void k_mrefit_chunk(int n, const int4 *mnode, const int *mpar_int,
-                                                      const int *mpar_leaf, const BVHNodeGPU *btl, TNode *tnodes,
-                                                      float *gbi, int *gh, int2 *xlist, unsigned *xcnt,
-                                                      unsigned *root_height, unsigned *err) {
-    mrefit_chunk_body(n, mnode, mpar_int, mpar_leaf, btl, tnodes, gbi, gh, xlist, xcnt, root_height, err, blockIdx.x);
-}
-
-__global__ __launch_bounds__(1024) void k_mrefit_mid(const int4 *mnode, const int *mpar_int, const BVHNodeGPU *btl,
-                                                     TNode *tnodes, float *gbi, int *gh, const int2 *xlist,
-                                                     const unsigned *xcnt, unsigned *gcnt, int2 *xtop,
-                                                     unsigned *xtop_count, unsigned xtop_cap, unsigned *root_height,
-                                                     unsigned *err) {
-    mrefit_mid_body(mnode, mpar_int, btl, tnodes, gbi, gh, xlist, xcnt, gcnt, xtop, xtop_count, xtop_cap, root_height,
-                    err, blockIdx.x);
-}
-
-__global__ __launch_bounds__(1024) void k_mrefit_top(const int4 *mnode, const int *mpar_int, const BVHNodeGPU *btl,
-                                                     TNode *tnodes, float *gbi, int *gh, const int2 *xtop,
-                                                     const unsigned *xtop_count, unsigned xtop_cap, unsigned *gcnt,
-                                                     unsigned *root_height, unsigned *err) {
-    mrefit_top_body(mnode, mpar_int, btl, tnodes, gbi, gh, xtop, xtop_count, xtop_cap, gcnt, root_height, err);
+template <bool LEAVES>
+__global__ __launch_bounds__(kWave) void k_mtree(int n, const unsigned *keys, const BVHNodeGPU *btl, const MItem *in,
+                                                 const int *in_cnt, int lists_in, MItem *out, int *out_cnt,
+                                                 TNode *tnodes, unsigned *root_height, unsigned *err) {
+    mtree_body<LEAVES>(n, keys, btl, in, in_cnt, lists_in, out, out_cnt, tnodes, root_height, err, blockIdx.x);
 }
 
 }  // namespace ptgpu
@@ -173,24 +161,13 @@ int clbvh_level_scratch(ptgpu_clbvh *h, float **halves, size_t *per) {
 }
 
 int clbvh_morton_scratch(ptgpu_clbvh *h, MortonScratch *m) {
-    const size_t N = (size_t)h->n;
-    PT_TRY(h->mnode.ensure((N > 1 ? N - 1 : 1) * sizeof(int4)));
-    PT_TRY(h->mpar.ensure((2 * N + 2) * sizeof(int)));
-    PT_TRY(h->gbi.ensure((N > 1 ? N - 1 : 1) * 6 * sizeof(float) + (N + 2) * sizeof(int)));
-    const size_t nsuper = (N + kMSuper - 1) / kMSuper;
-    const size_t xcap = nsuper * kXCap, tcap = mtop_cap((unsigned)nsuper);
-    PT_TRY(h->xlist.ensure((xcap + tcap) * sizeof(int2) + (nsuper + N + 2) * sizeof(unsigned)));
-    m->mnode = h->mnode.as<int4>();
-    m->mpar_int = h->mpar.as<int>();
-    m->mpar_leaf = h->mpar.as<int>() + N;
-    m->gbi = h->gbi.as<float>();
-    m->gh = reinterpret_cast<int *>(m->gbi + (N > 1 ? N - 1 : 1) * 6);
-    m->xlist = h->xlist.as<int2>();
-    m->xtop = m->xlist + xcap;
-    m->xtop_cap = (unsigned)tcap;
-    m->xcnt = reinterpret_cast<unsigned *>(m->xtop + tcap);
-    m->gcnt = m->xcnt + nsuper;
-    m->nsuper = (unsigned)nsuper;
+    m->levels = mtree_levels(h->n, m->lists);
+    const size_t n0 = (size_t)m->lists[0], n1 = (n0 + kMFan - 1) / kMFan;
+    PT_TRY(h->mitems.ensure((n0 + n1) * (kMItems * sizeof(MItem) + sizeof(int))));
+    m->items[0] = h->mitems.as<MItem>();
+    m->items[1] = m->items[0] + n0 * kMItems;
+    m->counts[0] = reinterpret_cast<int *>(m->items[1] + n1 * kMItems);
+    m->counts[1] = m->counts[0] + n0;
     return PTGPU_OK;
 }
 }  // namespace ptgpu
@@ -261,39 +238,26 @@ static int clbvh_refit_levels(ptgpu_clbvh *h) {
     return PTGPU_OK;
 }
 
-// Morton-keyed traversal tree (topology + two-pass refit); also records the tree height.
+// Morton-keyed traversal tree, level by level; also records the tree height.
 static int clbvh_traversal_morton(ptgpu_clbvh *h) {
     hipStream_t st = h->ctx->stream;
     const int n = h->n;
-    const size_t N = (size_t)n;
+    if (n < 2) return PTGPU_OK;
     MortonScratch ms;
     PT_TRY(clbvh_morton_scratch(h, &ms));
-    int *mpar_int = ms.mpar_int, *mpar_leaf = ms.mpar_leaf;
-    float *gbi = ms.gbi;
-    int *gh = ms.gh;
-    int2 *xlist = ms.xlist;
-    unsigned *gcnt = ms.gcnt;
-    unsigned *ctr = misc_counters(h);   // [9] error word, [10] arrivals for pass 3, [11] root height
-    PT_TRY(fill_u32(st, ctr + 10, 0u, 2));
-    if (n > 1) {
-        PT_TRY(fill_u32(st, ms.xcnt, 0u, ms.nsuper + N - 1));   // per-super-chunk counts, then gcnt
-        hipLaunchKernelGGL(k_karras_morton, dim3((n - 1 + 255) / 256), dim3(256), 0, st, h->keysA.as<unsigned>(), n,
-                           h->mnode.as<int4>(), mpar_int, mpar_leaf);
+    unsigned *ctr = misc_counters(h);   // [9] error word, [11] root height
+    for (int k = 0; k < ms.levels; k++) {
+        MItem *out = k + 1 < ms.levels ? ms.items[k & 1] : nullptr;
+        const MItem *in = k > 0 ? ms.items[(k - 1) & 1] : nullptr;
+        const int *in_cnt = k > 0 ? ms.counts[(k - 1) & 1] : nullptr;
+        const dim3 grid((unsigned)ms.lists[k]), block(kWave);
+        if (k == 0)
+            hipLaunchKernelGGL(k_mtree<true>, grid, block, 0, st, n, h->keysA.as<unsigned>(), h->btl.as<BVHNodeGPU>(), in,
+                               in_cnt, 0, out, ms.counts[0], h->tnodes.as<TNode>(), ctr + 11, ctr + 9);
+        else
+            hipLaunchKernelGGL(k_mtree<false>, grid, block, 0, st, n, h->keysA.as<unsigned>(), h->btl.as<BVHNodeGPU>(), in,
+                               in_cnt, ms.lists[k - 1], out, ms.counts[k & 1], h->tnodes.as<TNode>(), ctr + 11, ctr + 9);
         PT_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_mrefit_chunk, dim3((n + kMChunk - 1) / kMChunk), dim3(kMChunk), 0, st, n,
-                           h->mnode.as<int4>(), mpar_int, mpar_leaf, h->btl.as<BVHNodeGPU>(), h->tnodes.as<TNode>(),
-                           gbi, gh, xlist, ms.xcnt, ctr + 11, ctr + 9);
-        PT_HIP(hipGetLastError());
-        if (n > kMChunk) {
-            hipLaunchKernelGGL(k_mrefit_mid, dim3(ms.nsuper), dim3(1024), 0, st, h->mnode.as<int4>(), mpar_int,
-                               h->btl.as<BVHNodeGPU>(), h->tnodes.as<TNode>(), gbi, gh, (const int2 *)xlist,
-                               (const unsigned *)ms.xcnt, gcnt, ms.xtop, ctr + 10, ms.xtop_cap, ctr + 11, ctr + 9);
-            PT_HIP(hipGetLastError());
-            hipLaunchKernelGGL(k_mrefit_top, dim3(1), dim3(1024), 0, st, h->mnode.as<int4>(), mpar_int,
-                               h->btl.as<BVHNodeGPU>(), h->tnodes.as<TNode>(), gbi, gh, (const int2 *)ms.xtop,
-                               (const unsigned *)(ctr + 10), ms.xtop_cap, gcnt, ctr + 11, ctr + 9);
-            PT_HIP(hipGetLastError());
-        }
     }
     return PTGPU_OK;
 }
@@ -307,9 +271,14 @@ static int clbvh_sort(ptgpu_clbvh *h) {
     unsigned *hist = h->hist.as<unsigned>();
     unsigned *status = h->status.as<unsigned>();
     unsigned *ctr = misc_counters(h);
-    PT_TRY(fill_u32(st, hist, 0u, (size_t)C::kPasses * C::kRadix));
-    PT_TRY(fill_u32(st, status, 0u, (size_t)C::kPasses * tiles * C::kRadix));
-    PT_TRY(fill_u32(st, ctr + 1, 0u, 9));
+    // the histogram, the look-back words, and counters 1..11 (tile counters, error word, height) in one launch
+    {
+        const size_t nh = (size_t)C::kPasses * C::kRadix, ns = nh * tiles, words = nh + ns + 11;
+        const size_t blocks = (words + 255) / 256;
+        hipLaunchKernelGGL(k_clear3, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, st, status, ns, hist,
+                           (int)nh, ctr + 1, 11);
+        PT_HIP(hipGetLastError());
+    }
     int hblocks = (int)((n + kSortThreads * 8 - 1) / (kSortThreads * 8));
     if (hblocks > 2048) hblocks = 2048;
     if (hblocks < 1) hblocks = 1;
@@ -364,11 +333,11 @@ int clbvh_prepare_traversal(ptgpu_clbvh *h, bool recording, bool exact) {
         h->acc.depth = bound;
         h->acc.height_check = misc_counters(h) + 9;
     } else if (h->height_pending) {
-        unsigned w[3] = {0, 0, 0};   // error word, pass-3 arrivals, height
+        unsigned w[3] = {0, 0, 0};   // error word, -, height
         PT_HIP(hipMemcpyAsync(w, misc_counters(h) + 9, 12, hipMemcpyDeviceToHost, h->ctx->stream));
         PT_HIP(hipStreamSynchronize(h->ctx->stream));
         PT_CHECK(w[0] == 0, PTGPU_ERR_HIP, "LBVH build failed (error word %u: 1 sort look-back spin limit, 2 "
-                 "traversal-tree list overflow, 4 climb beyond the height bound)", w[0]);
+                 "traversal-tree list overflow)", w[0]);
         h->acc.depth = (int)w[2];
         h->acc.height_check = nullptr;
         h->known_height[h->optimized ? 1 : 0] = (int)w[2];
@@ -458,11 +427,6 @@ int ptgpu_clbvh_export_traversal(ptgpu_clbvh *h, int *h_refs4, float *h_boxes12,
     }
     std::vector<TNode> tn((size_t)m);
     PT_HIP(hipMemcpyAsync(tn.data(), h->tnodes.p, (size_t)m * sizeof(TNode), hipMemcpyDeviceToHost, h->ctx->stream));
-    std::vector<int4> mn;
-    if (h->trav_topology == 1 && !h->optimized) {
-        mn.resize((size_t)m);
-        PT_HIP(hipMemcpyAsync(mn.data(), h->mnode.p, (size_t)m * sizeof(int4), hipMemcpyDeviceToHost, h->ctx->stream));
-    }
     std::vector<BVHNodeGPU> bt;
     if (h->trav_topology == 0 && !h->optimized) {
         bt.resize((size_t)m);
@@ -470,13 +434,29 @@ int ptgpu_clbvh_export_traversal(ptgpu_clbvh *h, int *h_refs4, float *h_boxes12,
                               h->ctx->stream));
     }
     PT_HIP(hipStreamSynchronize(h->ctx->stream));
+    // leaf ranges of the Morton-keyed tree: a node's index is one end of its range (the last leaf of a left
+    // child, the first of any other), and the other end is its outer child's; children before parents
+    std::vector<int2> range;
+    if (h->trav_topology == 1 && !h->optimized) {
+        range.resize((size_t)m);
+        std::vector<int> order{0};
+        for (size_t k = 0; k < order.size(); k++) {
+            const int4 r = tn[order[k]].r;
+            if (r.x >= 0) order.push_back(r.x);
+            if (r.y >= 0) order.push_back(r.y);
+        }
+        for (size_t k = order.size(); k-- > 0;) {
+            const int4 r = tn[order[k]].r;
+            range[order[k]] = make_int2(r.x < 0 ? ~r.x : range[r.x].x, r.y < 0 ? ~r.y : range[r.y].y);
+        }
+    }
     for (int i = 0; i < m; i++) {
         const TNode &t = tn[i];
         h_refs4[i * 4 + 0] = t.r.x;
         h_refs4[i * 4 + 1] = t.r.y;
         // leaf ranges [lo, hi] of the build's tree; an optimised tree has none (-1)
-        h_refs4[i * 4 + 2] = h->optimized ? -1 : h->trav_topology == 1 ? mn[i].z : bt[i].min;
-        h_refs4[i * 4 + 3] = h->optimized ? -1 : h->trav_topology == 1 ? mn[i].w : bt[i].max;
+        h_refs4[i * 4 + 2] = h->optimized ? -1 : h->trav_topology == 1 ? range[i].x : bt[i].min;
+        h_refs4[i * 4 + 3] = h->optimized ? -1 : h->trav_topology == 1 ? range[i].y : bt[i].max;
         const float v[12] = {t.a.x, t.a.w, t.a.y, t.b.x, t.a.z, t.b.y, t.b.z, t.c.y, t.b.w, t.c.z, t.c.x, t.c.w};
         for (int f = 0; f < 12; f++) h_boxes12[i * 12 + f] = v[f];   // two Bounds in reference order
     }
@@ -631,7 +611,7 @@ int ptgpu_clbvh_get_trees(ptgpu_clbvh *h, BVHNodeGPU **h_btn, BVHNodeGPU **h_btl
     PT_HIP(hipMemcpyAsync(&err, misc_counters(h) + 9, 4, hipMemcpyDeviceToHost, h->ctx->stream));
     PT_HIP(hipStreamSynchronize(h->ctx->stream));
     PT_CHECK(err == 0, PTGPU_ERR_HIP, "LBVH build failed (error word %u: 1 sort look-back spin limit, 2 "
-             "traversal-tree list overflow, 4 climb beyond the height bound)", err);
+             "traversal-tree list overflow)", err);
     *h_btn = h->h_btn.data();
     *h_btl = h->h_btl.data();
     return PTGPU_OK;
@@ -651,7 +631,7 @@ int ptgpu_clbvh_device_bytes(ptgpu_clbvh *h, size_t *bytes) {
     PT_CHECK(h && bytes, PTGPU_ERR_INVALID, "null argument");
     const DevBuf *bufs[] = {&h->own_shapes, &h->keysA, &h->pairs, &h->valsA, &h->btn, &h->btl,
                             &h->tnodes, &h->prims, &h->hist, &h->status, &h->misc, &h->lights, &h->scan,
-                            &h->opt_tmp, &h->mnode, &h->mpar, &h->gbi, &h->xlist, &h->tnodes4, &h->treelet,
+                            &h->opt_tmp, &h->mitems, &h->tnodes4, &h->treelet,
                             &h->boxes};
     size_t t = 0;
     for (const DevBuf *b : bufs) t += b->bytes;
@@ -701,7 +681,7 @@ int ptgpu_clbvh_destroy(ptgpu_clbvh *h) {
     h->btn.release(); h->btl.release(); h->tnodes.release(); h->prims.release();
     h->hist.release(); h->status.release(); h->misc.release(); h->own_shapes.release();
     h->lights.release(); h->scan.release(); h->opt_tmp.release();
-    h->mnode.release(); h->mpar.release(); h->gbi.release(); h->xlist.release(); h->tnodes4.release();
+    h->mitems.release(); h->tnodes4.release();
     h->boxes.release();
     h->treelet.release();
     for (auto &e : h->ev)

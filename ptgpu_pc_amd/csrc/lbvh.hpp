@@ -16,18 +16,13 @@ constexpr int kRecordedHeightMargin = 4;
 constexpr int kRecordedHeightDefault = 41;   // the deepest tree the 64-entry four-wide stack walks
 int clbvh_export_optimized(ptgpu_clbvh *h);
 
-// Scratch of the Morton-keyed traversal tree: topology, parents, and the refit's crossing queue.
+struct MItem;
+// Scratch of the Morton-keyed traversal tree: each level's lists of leftover items, in two buffers by turns.
 struct MortonScratch {
-    int4 *mnode;
-    int *mpar_int, *mpar_leaf;
-    float *gbi;      // bounds of internal nodes whose subtree spans 1024-leaf chunks
-    int *gh;         // their heights
-    int2 *xlist;     // (node, child) arrivals at chunk-spanning nodes, kXCap per super-chunk
-    unsigned *xcnt;  // their count per super-chunk
-    int2 *xtop;      // arrivals at nodes spanning super-chunks
-    unsigned xtop_cap;
-    unsigned *gcnt;  // visit counters of the passes over chunk-spanning nodes
-    unsigned nsuper; // super-chunks (kMSuper leaves each)
+    int levels;
+    int lists[8];      // lists of each level (kMMaxLevels)
+    MItem *items[2];
+    int *counts[2];
 };
 int clbvh_morton_scratch(ptgpu_clbvh *h, MortonScratch *m);
 // Bound buffers handed between the level passes of the index-keyed refit (two halves of `per` floats).
@@ -51,7 +46,7 @@ struct ptgpu_clbvh {
     ptgpu::DevBuf btn, btl, tnodes, prims;
     ptgpu::DevBuf hist, status, misc;
     ptgpu::DevBuf lights, scan, opt_tmp;
-    ptgpu::DevBuf mnode, mpar, gbi, xlist;   // Morton-keyed traversal tree: topology, parents, refit scratch
+    ptgpu::DevBuf mitems;                    // Morton-keyed traversal tree: leftover items of its levels
     ptgpu::DevBuf tnodes4;                   // four-wide view of tnodes, rebuilt after each refit
     bool wide_pending = false;
     ptgpu::DevBuf treelet;                   // treelet optimiser state (kept for the lazy export)
@@ -65,7 +60,7 @@ struct ptgpu_clbvh {
     ptgpu::DevAccel acc;
     std::vector<BVHNodeGPU> h_btn, h_btl;
     // misc: [0..5] scene centroid bounds, words 8.. counters ([0] unused, [1..8] sort
-    // tile counters, [9] sort look-back error, [10] chunk crossings, [11] traversal-tree height),
+    // tile counters, [9] build error word, [10] unused, [11] traversal-tree height),
     // floats 64.. per-block bound partials
     float *scene6() const { return misc.as<float>(); }
     unsigned *counters() const { return misc.as<unsigned>() + 8; }

@@ -8,8 +8,8 @@
 // alone.  The sort passes take tile ids from one atomic counter for the whole batch; a tile's
 // decoupled look-back only waits on earlier tiles of its own scene, which hold smaller ids and have
 // therefore already started.  Small scenes fill the chip together instead of leaving it idle
-// behind a launch each, and the single-workgroup top pass of the traversal-tree refit runs for all
-// scenes at once.  One 8-byte-per-scene readback at the end carries tree heights and sort errors.
+// behind a launch each, and the last levels of the traversal trees, a few waves each, run for all scenes
+// at once.  One 8-byte-per-scene readback at the end carries tree heights and sort errors.
 #include <cstring>
 #include <unordered_set>
 #include <vector>
@@ -34,14 +34,8 @@ struct BuildSeg {
     TNode *tnodes;
     Prim *prims;
     float *lvl;             // level-refit hand-off: two halves of lvl_per floats
-    int4 *mnode;
-    int *mpar_int, *mpar_leaf;
-    float *gbi;
-    int *gh;
-    int2 *xlist, *xtop;
-    unsigned *xcnt, *gcnt;
-    unsigned xtop_cap, pad;
     long long lvl_per;
+    MortonScratch ms;
     int n, tiles, levels_total, topo;
 };
 
@@ -51,8 +45,8 @@ struct FillSeg {
     unsigned value, pad;
 };
 
-enum Stage { kStBounds, kStMorton, kStKarras, kStHist, kStTiles, kStRefit0, kStRefit1, kStRefit2, kStKMorton,
-             kStMChunk, kStMSuper, kStages };
+enum Stage { kStBounds, kStMorton, kStKarras, kStHist, kStTiles, kStRefit0, kStRefit1, kStRefit2, kStMtree,
+             kStages = kStMtree + kMMaxLevels };
 constexpr int kMaxRefitPasses = 3;   // ceil(30 / kRefitLog) levels for N < 2^30
 constexpr int kFillWords = 4096;     // words cleared per block of the fill launch
 
@@ -146,32 +140,15 @@ __global__ __launch_bounds__(256) void kb_refit(const BuildSeg *g, const int *st
                             blockIdx.x - starts[s]);
 }
 
-__global__ __launch_bounds__(256) void kb_karras_morton(const BuildSeg *g, const int *starts, int ns) {
+// Level k of every scene's Morton-keyed tree.
+template <bool LEAVES>
+__global__ __launch_bounds__(kWave) void kb_mtree(const BuildSeg *g, const int *starts, int ns, int k) {
     const int s = seg_find(starts, ns, blockIdx.x);
     const BuildSeg &S = g[s];
-    karras_morton_body(S.keysA, S.n, S.mnode, S.mpar_int, S.mpar_leaf, blockIdx.x - starts[s]);
-}
-
-__global__ __launch_bounds__(kMChunk) void kb_mrefit_chunk(const BuildSeg *g, const int *starts, int ns) {
-    const int s = seg_find(starts, ns, blockIdx.x);
-    const BuildSeg &S = g[s];
-    mrefit_chunk_body(S.n, S.mnode, S.mpar_int, S.mpar_leaf, S.btl, S.tnodes, S.gbi, S.gh, S.xlist, S.xcnt,
-                      S.ctr + 11, S.ctr + 9, blockIdx.x - starts[s]);
-}
-
-__global__ __launch_bounds__(1024) void kb_mrefit_mid(const BuildSeg *g, const int *starts, int ns) {
-    const int s = seg_find(starts, ns, blockIdx.x);
-    const BuildSeg &S = g[s];
-    mrefit_mid_body(S.mnode, S.mpar_int, S.btl, S.tnodes, S.gbi, S.gh, S.xlist, S.xcnt, S.gcnt, S.xtop, S.ctr + 10,
-                    S.xtop_cap, S.ctr + 11, S.ctr + 9, (unsigned)(blockIdx.x - starts[s]));
-}
-
-// One workgroup per scene: the chunk-spanning nodes of every scene are refitted concurrently.
-__global__ __launch_bounds__(1024) void kb_mrefit_top(const BuildSeg *g) {
-    const BuildSeg &S = g[blockIdx.x];
-    if (S.topo != 1 || S.n <= kMChunk) return;
-    mrefit_top_body(S.mnode, S.mpar_int, S.btl, S.tnodes, S.gbi, S.gh, S.xtop, S.ctr + 10, S.xtop_cap, S.gcnt,
-                    S.ctr + 11, S.ctr + 9);
+    MItem *out = k + 1 < S.ms.levels ? S.ms.items[k & 1] : nullptr;
+    mtree_body<LEAVES>(S.n, S.keysA, S.btl, LEAVES ? nullptr : S.ms.items[(k - 1) & 1],
+                       LEAVES ? nullptr : S.ms.counts[(k - 1) & 1], LEAVES ? 0 : S.ms.lists[k - 1], out,
+                       S.ms.counts[k & 1], S.tnodes, S.ctr + 11, S.ctr + 9, blockIdx.x - starts[s]);
 }
 
 // heights[s] = traversal-tree height, errs[s] = build error word
@@ -223,20 +200,7 @@ int build_batch(ptgpu_ctx *ctx, ptgpu_clbvh *const *hs, int ns) {
         S.levels_total = L;
         S.topo = h->trav_topology;
         const bool mtree = S.topo == 1 && n > 1;
-        if (mtree) {
-            MortonScratch ms;
-            PT_TRY(clbvh_morton_scratch(h, &ms));
-            S.mnode = ms.mnode;
-            S.mpar_int = ms.mpar_int;
-            S.mpar_leaf = ms.mpar_leaf;
-            S.gbi = ms.gbi;
-            S.gh = ms.gh;
-            S.xlist = ms.xlist;
-            S.xtop = ms.xtop;
-            S.xcnt = ms.xcnt;
-            S.xtop_cap = ms.xtop_cap;
-            S.gcnt = ms.gcnt;
-        }
+        if (mtree) PT_TRY(clbvh_morton_scratch(h, &S.ms));
         // block counts: the single-scene launches' grids
         int bb = (n + kBoundsThreads - 1) / kBoundsThreads;
         blocks(kStBounds, s) = bb > 4096 ? 4096 : bb < 1 ? 1 : bb;
@@ -251,16 +215,13 @@ int build_batch(ptgpu_ctx *ctx, ptgpu_clbvh *const *hs, int ns) {
             const long long m = ((long long)n + (1ll << s0) - 1) >> s0;
             blocks(kStRefit0 + p, s) = (int)((m + kRefitItems - 1) / kRefitItems);
         }
-        blocks(kStKMorton, s) = mtree ? (n - 1 + 255) / 256 : 0;
-        blocks(kStMChunk, s) = mtree ? (n + kMChunk - 1) / kMChunk : 0;
-        blocks(kStMSuper, s) = mtree && n > kMChunk ? (int)((n + kMSuper - 1) / kMSuper) : 0;
+        for (int k = 0; mtree && k < S.ms.levels; k++) blocks(kStMtree + k, s) = S.ms.lists[k];
         // clears done by the single-scene path (CLBVH.cpp:83-88 for btn/btl: kb_karras writes them,
         // except the lone leaf of a one-shape scene)
         if (n == 1) fills.push_back({(unsigned *)S.btl, (unsigned long long)sizeof(BVHNodeGPU) / 4, 0xFFFFFFFFu, 0u});
         fills.push_back({S.hist, (unsigned long long)C::kPasses * C::kRadix, 0u, 0u});
         fills.push_back({S.status, (unsigned long long)C::kPasses * S.tiles * C::kRadix, 0u, 0u});
         fills.push_back({S.ctr + 9, 3ull, 0u, 0u});
-        if (mtree) fills.push_back({S.xcnt, (unsigned long long)(S.gcnt - S.xcnt) + (n - 1), 0u, 0u});
     }
     for (int k = 0; k < kStages; k++)
         for (int s = 0; s < ns; s++) starts[(size_t)k * (ns + 1) + s + 1] += starts[(size_t)k * (ns + 1) + s];
@@ -351,14 +312,11 @@ int build_batch(ptgpu_ctx *ctx, ptgpu_clbvh *const *hs, int ns) {
     for (int p = 1; p < kMaxRefitPasses; p++) {
         PT_BATCH_LAUNCH(kb_refit<false>, kStRefit0 + p, 256, p);
     }
-    PT_BATCH_LAUNCH(kb_karras_morton, kStKMorton, 256);
-    PT_BATCH_LAUNCH(kb_mrefit_chunk, kStMChunk, kMChunk);
-    PT_BATCH_LAUNCH(kb_mrefit_mid, kStMSuper, 1024);
-#undef PT_BATCH_LAUNCH
-    if (total(kStMChunk) > 0) {
-        hipLaunchKernelGGL(kb_mrefit_top, dim3(ns), dim3(1024), 0, st, d_segs);
-        PT_HIP(hipGetLastError());
+    PT_BATCH_LAUNCH(kb_mtree<true>, kStMtree, kWave, 0);
+    for (int k = 1; k < kMMaxLevels; k++) {
+        PT_BATCH_LAUNCH(kb_mtree<false>, kStMtree + k, kWave, k);
     }
+#undef PT_BATCH_LAUNCH
     if (recording) {
         // nothing is read back: each handle's height stays pending, and a recorded traversal checks
         // it (with the build's error word, both in the handle's counters) on the device

@@ -723,263 +723,225 @@ __device__ __forceinline__ int delta_key(const unsigned *keys, int i, int j, int
     return x ? __clz(x) : 32 + __clz(i ^ j);
 }
 
-__device__ __forceinline__ void karras_morton_body(const unsigned *keys, int n, int4 *mnode, int *mpar_int,
-                                                   int *mpar_leaf, int bid) {
-    const int i = bid * blockDim.x + threadIdx.x;
-    if (i >= n - 1) return;
-    const int d = (delta_key(keys, i, i + 1, n) - delta_key(keys, i, i - 1, n)) > 0 ? 1 : -1;
-    const int dmin = delta_key(keys, i, i - d, n);
-    long long lmax = 2;
-    while (delta_key(keys, i, (int)(i + lmax * d), n) > dmin) lmax <<= 1;
-    long long l = 0;
-    for (long long t = lmax >> 1; t >= 1; t >>= 1)
-        if (delta_key(keys, i, (int)(i + (l + t) * d), n) > dmin) l += t;
-    const int j = (int)(i + l * d);
-    const int dnode = delta_key(keys, i, j, n);
-    long long s = 0, t = l;
-    do {
-        t = (t + 1) >> 1;
-        if (delta_key(keys, i, (int)(i + (s + t) * d), n) > dnode) s += t;
-    } while (t > 1);
-    const int gamma = (int)(i + s * d + (d < 0 ? d : 0));
-    const int lo = i < j ? i : j, hi = i < j ? j : i;
-    const int lref = (lo == gamma) ? ~gamma : gamma;
-    const int rref = (hi == gamma + 1) ? ~(gamma + 1) : gamma + 1;
-    mnode[i] = make_int4(lref, rref, lo, hi);
-    if (lref < 0) mpar_leaf[gamma] = i; else mpar_int[gamma] = i;
-    if (rref < 0) mpar_leaf[gamma + 1] = i; else mpar_int[gamma + 1] = i;
-    if (i == 0) mpar_int[0] = -1;
-}
-
-// Pass 1: one workgroup per 512 consecutive leaves.  Every node whose leaf range lies inside the
-// chunk has its Karras index inside the chunk too, so visit counters and bounds live in LDS and the
-// bottom-up climb synchronises through workgroup-scope LDS atomics only.  A climb that reaches a
-// node spanning chunks publishes its child's bound and height and queues the (node, child) arrival
-// in the list of the 64-chunk super-chunk that holds the node's first leaf.  512-leaf chunks keep
-// the pass at 40 KB of LDS per workgroup, so it runs beside a render's persistent workgroups (two
-// per CU hold about 100 KB of the 160 KB) instead of waiting for them to retire.
+// Topology and bounds bottom-up, in one pass per level of lists.  An item is a finished subtree: a leaf, or
+// what an earlier level left over.  Items stand in leaf order, and between neighbours stands their prefix
+// length D.  An item [a, b] belongs under the split with the longer prefix of its two sides: the left child
+// of the split after b, or the right child of the split before a (the tree over the adjacent prefixes is
+// the radix tree).  The first child to reach a split waits in the split's slot; the second merges both,
+// writes the traversal node and goes on with it.  A node's index is the radix tree's: its last leaf where it
+// is a left child, its first leaf otherwise.  No topology pass, parent links or counters in memory, and a
+// node's children, range and side are known from the items alone.
 //
-// List capacities follow from the tree height h <= 62 (30-bit codes, ties split by a 32-bit index):
-// at most h nodes cross any boundary and each node receives two arrivals, so a super-chunk's list
-// holds at most 2 * 62 * 64 entries and the list of nodes spanning super-chunks 2 * 62 per boundary.
-// An overflow (a malformed tree) sets the build's error word instead of writing out of bounds.
-constexpr int kMChunk = 512;
-constexpr unsigned kMSuper = 64u * kMChunk;    // leaves per super-chunk (64 chunks)
-constexpr unsigned kXCap = 8192;               // arrivals per super-chunk list
-// Climb steps of one thread: a tree over 30-bit codes with ties split by a 32-bit index is at most 62
-// levels high, so a climb longer than this follows a malformed parent chain (a cycle): it stops and
-// sets bit 4 of the build's error word instead of spinning.
-constexpr int kMaxClimb = 64;
-__host__ __device__ constexpr unsigned mtop_cap(unsigned nsuper) { return 128u * (nsuper + 1u); }
+// One wave works a list: 128 leaves, or the leftovers of kMFan lists.  Its lanes hold one item each, and a
+// lane whose item waits takes the next one, so the wave's steps stay full until its items run out; one
+// thread per leaf climbing its parents left most lanes of each wave idle after two steps, and read the
+// topology from memory.  What bounds it: the step's instructions and its LDS round trips.  4,000,003 shapes:
+// topology, chunk climb and the two climbs above it 907 us; this pass and its upper levels 250 us (512 leaves a list:
+// 244 us, but 1,003 shapes 9 us longer: their waves' chains are what counts there).
+//
+// Leftovers: items whose split is not inside the list, and those that wait for one that is not.  They are
+// cut by nodes that span an end of the list, whose prefixes differ: at most one per prefix length and end, so
+// 2 * 62 + 1 (30-bit codes, ties split by the index).  More come only of unsorted keys (a failed sort): the
+// surplus is dropped and the build's error word set.
+constexpr int kMChunk = 128;      // leaves per list of the first level
+constexpr int kMFan = 16;         // lists per list of the next level
+constexpr int kMItems = 128;      // room for a list's leftovers (at most 125)
+constexpr int kMMaxLevels = 8;    // lists of 2^30 leaves: 2^21, then a sixteenth at each level
+struct alignas(16) MItem {
+    float4 q0;   // bound: min_x, max_x, min_y, max_y
+    float2 q1;   // min_z, max_z
+    int first;   // first leaf
+    int dh;      // bits 0-7: prefix length with the leaf before it, plus one (0 at the tree's start); bits 8-: height
+};
+static_assert(sizeof(MItem) == 32, "MItem");
 
-__device__ __forceinline__ void mrefit_chunk_body(int n, const int4 *mnode, const int *mpar_int, const int *mpar_leaf,
-                                                  const BVHNodeGPU *btl, TNode *tnodes, float *gbi, int *gh,
-                                                  int2 *xlist, unsigned *xcnt, unsigned *root_height, unsigned *err,
-                                                  int bid) {
-    __shared__ float lb[6][kMChunk];
-    __shared__ float nb[6][kMChunk];
-    __shared__ int nh[kMChunk];
-    __shared__ unsigned cnt[kMChunk];
-    // The chunk's internal nodes, their parents and the leaves' parents, loaded once with coalesced
-    // reads: the climbs below then touch global memory only for their tnodes stores and, at their
-    // end, for a parent spanning chunks.  (On gfx950 a wait for a global load also waits for every
-    // earlier store of the thread, so a load inside the climb would serialise it on those stores.)
-    __shared__ int4 smn[kMChunk];
-    __shared__ int spar[kMChunk];
-    __shared__ int slp[kMChunk];
+template <bool LEAVES>
+struct MTreeList {
+    static constexpr int kCap = LEAVES ? kMChunk : kMFan * (kMItems - 3);
+    float2 b[3][kCap + 1];            // slot s: the bound waiting at the split before item s; item s-1 until it is taken
+    unsigned tag[kCap + 1];           // bit 31: an item waits, bit 30: the left child, bits 16-29: height, 0-15: its far end
+    int first[LEAVES ? 1 : kCap + 1];
+    unsigned char d[kCap + 4];        // d[s]: prefix length across split s, plus one
+    unsigned char h[LEAVES ? 4 : kCap + 4];
+    unsigned starts[(kCap + 31) / 32];
+    int offs[kMFan + 1];
+};
+
+// `lists_in`: lists of the level below (upper levels).  out / out_cnt: this level's leftovers.
+template <bool LEAVES>
+__device__ __forceinline__ void mtree_body(int n, const unsigned *keys, const BVHNodeGPU *btl, const MItem *in,
+                                           const int *in_cnt, int lists_in, MItem *out, int *out_cnt, TNode *tnodes,
+                                           unsigned *root_height, unsigned *err, int bid) {
+    __shared__ MTreeList<LEAVES> S;
+    constexpr int kCap = MTreeList<LEAVES>::kCap;
+    const int lane = threadIdx.x;
+    const unsigned long long lt = lanemask_lt();
     const int base = bid * kMChunk;
-    const int cend = (n - base) < kMChunk ? n : base + kMChunk;
-    for (int q = threadIdx.x; q < kMChunk; q += (int)blockDim.x) {
-        cnt[q] = 0;
-        const int k = base + q;
-        if (k < cend) {
-            const Bound b = load_bound(&btl[k].bound);
-            lb[0][q] = b.min_x; lb[1][q] = b.max_x; lb[2][q] = b.min_y;
-            lb[3][q] = b.max_y; lb[4][q] = b.min_z; lb[5][q] = b.max_z;
-            slp[q] = n > 1 ? mpar_leaf[k] : -1;
+    int count;
+    auto stage = [&](int item, float2 x, float2 y, float2 z) {
+        S.b[0][item + 1] = x;
+        S.b[1][item + 1] = y;
+        S.b[2][item + 1] = z;
+    };
+    if (LEAVES) {
+        count = n - base < kMChunk ? n - base : kMChunk;
+#pragma unroll 4
+        for (int i = lane; i < count; i += kWave) {
+            const float *f = reinterpret_cast<const float *>(&btl[base + i].bound);
+            stage(i, make_float2(f[0], f[1]), make_float2(f[2], f[3]), make_float2(f[4], f[5]));
         }
-        if (k < n - 1) {
-            smn[q] = mnode[k];
-            spar[q] = mpar_int[k];
+#pragma unroll 4
+        for (int i = lane; i <= count; i += kWave) {
+            const int k = base + i;
+            S.d[i] = (unsigned char)(k < n ? delta_key(keys, k, k - 1, n) + 1 : 0);
         }
+    } else {
+        const int l0 = bid * kMFan;
+        const int lists = lists_in - l0 < kMFan ? lists_in - l0 : kMFan;
+        int c = lane < lists ? in_cnt[l0 + lane] : 0;
+        c = c < kMItems - 3 ? c : kMItems - 3;
+        int run = c;
+        for (int x = 1; x < kMFan; x <<= 1) {
+            const int o = __shfl_up(run, x);
+            if (lane >= x) run += o;
+        }
+        if (lane < kMFan) S.offs[lane + 1] = run;
+        if (lane == 0) S.offs[0] = 0;
+        __syncthreads();
+        count = S.offs[kMFan];
+#pragma unroll 4
+        for (int i = lane; i < count; i += kWave) {
+            int q = 0;
+            for (int x = kMFan >> 1; x > 0; x >>= 1)
+                if (S.offs[q + x] <= i) q += x;
+            const MItem m = in[(size_t)(l0 + q) * kMItems + (i - S.offs[q])];
+            stage(i, make_float2(m.q0.x, m.q0.y), make_float2(m.q0.z, m.q0.w), m.q1);
+            S.first[i] = m.first;
+            S.d[i] = (unsigned char)(m.dh & 0xff);
+            S.h[i] = (unsigned char)(m.dh >> 8);
+        }
+        if (lane == 0) {
+            const bool more = l0 + kMFan < lists_in;
+            const MItem *nx = in + (size_t)(l0 + kMFan) * kMItems;
+            S.first[count] = more ? nx->first : n;
+            S.d[count] = (unsigned char)(more ? nx->dh & 0xff : 0);
+        }
+    }
+    for (int s = lane; s <= count; s += kWave) S.tag[s] = 0u;
+    for (int s = lane; s < (kCap + 31) / 32; s += kWave) S.starts[s] = 0u;
+    __syncthreads();
+    auto first_leaf = [&](int item) { return LEAVES ? base + item : S.first[item]; };
+
+    bool on = false;
+    int a = 0, b = 0, h = 0, next = 0;
+    float2 bx = make_float2(0.f, 0.f), by = bx, bz = bx;
+    for (;;) {
+        // lanes without an item take the next ones (a slot's own item is taken before anything waits there)
+        if (next < count) {
+            const unsigned long long want = __ballot(!on);
+            const int k = next + (int)__popcll(want & lt);
+            if (!on && k < count) {
+                on = true;
+                a = b = k;
+                h = LEAVES ? 0 : S.h[k];
+                bx = S.b[0][k + 1];
+                by = S.b[1][k + 1];
+                bz = S.b[2][k + 1];
+            }
+            next += (int)__popcll(want);
+        }
+        if (!__ballot(on)) break;
+        int s = 0;
+        bool left = false;
+        unsigned other = 0u;
+        if (on) {
+            const int da = S.d[a], db = S.d[b + 1];
+            if ((da | db) == 0) {   // the whole tree
+                *root_height = (unsigned)h;
+                on = false;
+            } else {
+                left = db > da;
+                s = left ? b + 1 : a;
+                other = atomicExch(&S.tag[s], 0x80000000u | (left ? 0x40000000u : 0u) | ((unsigned)h << 16) |
+                                                  (unsigned)(left ? a : b));
+            }
+        }
+        // all lanes' arrivals are in (one wave, in order): the first ones' bounds are stored before the second
+        // ones read them, also where both come in the same step
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup", "local");
+        if (on && !other) {
+            S.b[0][s] = bx;
+            S.b[1][s] = by;
+            S.b[2][s] = bz;
+            on = false;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup", "local");
+        if (on) {
+            const float2 ox = S.b[0][s], oy = S.b[1][s], oz = S.b[2][s];
+            S.tag[s] = 0u;
+            const int far = (int)(other & 0xffffu), oh = (int)((other >> 16) & 0x3fffu);
+            Bound L, R;
+            L.min_x = left ? bx.x : ox.x; L.max_x = left ? bx.y : ox.y;
+            L.min_y = left ? by.x : oy.x; L.max_y = left ? by.y : oy.y;
+            L.min_z = left ? bz.x : oz.x; L.max_z = left ? bz.y : oz.y;
+            R.min_x = left ? ox.x : bx.x; R.max_x = left ? ox.y : bx.y;
+            R.min_y = left ? oy.x : by.x; R.max_y = left ? oy.y : by.y;
+            R.min_z = left ? oz.x : bz.x; R.max_z = left ? oz.y : bz.y;
+            const Bound M = merge_bounds(L, R);
+            bx = make_float2(M.min_x, M.max_x);
+            by = make_float2(M.min_y, M.max_y);
+            bz = make_float2(M.min_z, M.max_z);
+            if (left) b = far; else a = far;
+            h = (h > oh ? h : oh) + 1;
+            const int lo = first_leaf(a), g = first_leaf(s) - 1, hi = first_leaf(b + 1) - 1;
+            const int rl = lo == g ? ~g : g, rr = g + 1 == hi ? ~hi : g + 1;
+            const int p = S.d[b + 1] > S.d[a] ? hi : lo;
+            if ((unsigned)p < (unsigned)(n - 1)) tnodes[p] = make_tnode(L, R, rl, rr, rl < 0 ? 1 : 0, rr < 0 ? 1 : 0);
+        }
+    }
+    if (!out) return;
+    // the items that still wait, in leaf order
+    auto start_of = [&](int s, unsigned t) { return t & 0x40000000u ? (int)(t & 0xffffu) : s; };
+    __syncthreads();
+    for (int s = lane; s <= count; s += kWave) {
+        const unsigned t = S.tag[s];
+        const int a0 = start_of(s, t);
+        if (t && a0 < count) atomicOr(&S.starts[a0 >> 5], 1u << (a0 & 31));
     }
     __syncthreads();
-    for (int q = threadIdx.x; q < kMChunk; q += (int)blockDim.x) {
-        const int k = base + q;
-        if (k >= cend) break;
-        int child = ~k, ch = 0;
-        int p = slp[q];
-        bool spans = false;
-        int steps = 0;
-        while (p >= 0) {
-            if (++steps > kMaxClimb) {
-                atomicOr(err, 4u);
-                p = -1;
-                child = -1;
-                break;
-            }
-            // a node whose leaf range lies inside the chunk has its index there too (Karras numbering:
-            // the index is an end of the range), so an index outside the chunk means a spanning node
-            if (p < base || p >= base + kMChunk) {
-                spans = true;
-                break;
-            }
-            const int4 P = smn[p - base];
-            if (P.z < base || P.w >= base + kMChunk) {
-                spans = true;
-                break;
-            }
-            // The sibling's bound and height are in LDS, so the counter orders LDS only: an LDS-scope
-            // release / acquire, which (unlike a workgroup-scope one over all memory) does not wait
-            // for this thread's earlier tnodes stores to reach memory.
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-            const unsigned old = __hip_atomic_fetch_add(&cnt[p - base], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-            if (old == 0) break;
-            Bound L, R;
-            int hl, hr;
-            {
-                const int a = P.x < 0 ? ~P.x - base : P.x - base;
-                float (*src)[kMChunk] = P.x < 0 ? lb : nb;
-                L.min_x = src[0][a]; L.max_x = src[1][a]; L.min_y = src[2][a];
-                L.max_y = src[3][a]; L.min_z = src[4][a]; L.max_z = src[5][a];
-                hl = P.x < 0 ? 0 : nh[a];
-            }
-            {
-                const int a = P.y < 0 ? ~P.y - base : P.y - base;
-                float (*src)[kMChunk] = P.y < 0 ? lb : nb;
-                R.min_x = src[0][a]; R.max_x = src[1][a]; R.min_y = src[2][a];
-                R.max_y = src[3][a]; R.min_z = src[4][a]; R.max_z = src[5][a];
-                hr = P.y < 0 ? 0 : nh[a];
-            }
-            const Bound M = merge_bounds(L, R);
-            const int c = p - base;
-            nb[0][c] = M.min_x; nb[1][c] = M.max_x; nb[2][c] = M.min_y;
-            nb[3][c] = M.max_y; nb[4][c] = M.min_z; nb[5][c] = M.max_z;
-            ch = (hl > hr ? hl : hr) + 1;
-            nh[c] = ch;
-            tnodes[p] = make_tnode(L, R, P.x, P.y, P.x < 0 ? 1 : 0, P.y < 0 ? 1 : 0);
-            child = p;
-            p = spar[c];
-        }
-        if (spans) {
-            // publish the child's bound and height, queue the arrival at its spanning parent
-            const int pz = (p >= base && p < base + kMChunk) ? smn[p - base].z : mnode[p].z;
-            if (child >= 0) {
-                const int c = child - base;
-                for (int f = 0; f < 6; f++) gbi[(size_t)child * 6 + f] = nb[f][c];
-                gh[child] = ch;
-            }
-            const unsigned sc = (unsigned)pz / kMSuper;
-            const unsigned slot = atomicAdd(xcnt + sc, 1u);
-            if (slot < kXCap) xlist[(size_t)sc * kXCap + slot] = make_int2(p, child);
-            else atomicOr(err, 2u);
-        } else if (p < 0 && child >= 0) {
-            *root_height = (unsigned)ch;   // the root closed inside this chunk
-        }
+    int total = 0;
+    for (int w = 0; w < (kCap + 31) / 32; w++) total += __popc(S.starts[w]);
+    if (lane == 0) {
+        out_cnt[bid] = total;
+        if (total > kMItems - 3) atomicOr(err, 2u);
+    }
+    MItem *o = out + (size_t)bid * kMItems;
+    for (int s = lane; s <= count; s += kWave) {
+        const unsigned t = S.tag[s];
+        const int a0 = start_of(s, t);
+        if (!t || a0 >= count) continue;
+        int rank = __popc(S.starts[a0 >> 5] & ((1u << (a0 & 31)) - 1u));
+        for (int w = 0; w < (a0 >> 5); w++) rank += __popc(S.starts[w]);
+        if (rank >= kMItems - 3) continue;
+        MItem m;
+        const float2 x = S.b[0][s], y = S.b[1][s];
+        m.q0 = make_float4(x.x, x.y, y.x, y.y);
+        m.q1 = S.b[2][s];
+        m.first = first_leaf(a0);
+        m.dh = (int)S.d[a0] | (int)(((t >> 16) & 0x3fffu) << 8);
+        o[rank] = m;
     }
 }
 
-// Passes 2 and 3: child bounds written by an earlier pass are visible (earlier launch); those written
-// by another thread of the same workgroup are ordered by the workgroup-scope acquire/release counter.
-// One node's refit from its two children (the second arrival's work in the passes below): bound and
-// height into gbi / gh, the traversal node into tnodes; returns the height.
-__device__ __forceinline__ int mrefit_node(int p, const int4 &P, const BVHNodeGPU *btl, TNode *tnodes, float *gbi,
-                                           int *gh) {
-    Bound L, R;
-    int hl = 0, hr = 0;
-    if (P.x < 0) L = load_bound(&btl[~P.x].bound);
-    else {
-        const float *f = gbi + (size_t)P.x * 6;
-        L.min_x = f[0]; L.max_x = f[1]; L.min_y = f[2]; L.max_y = f[3]; L.min_z = f[4]; L.max_z = f[5];
-        hl = gh[P.x];
+// Lists of each level over n leaves; their count.
+inline int mtree_levels(int n, int *lists) {
+    int k = 0;
+    lists[0] = (n + kMChunk - 1) / kMChunk;
+    while (lists[k] > 1) {
+        lists[k + 1] = (lists[k] + kMFan - 1) / kMFan;
+        k++;
     }
-    if (P.y < 0) R = load_bound(&btl[~P.y].bound);
-    else {
-        const float *f = gbi + (size_t)P.y * 6;
-        R.min_x = f[0]; R.max_x = f[1]; R.min_y = f[2]; R.max_y = f[3]; R.min_z = f[4]; R.max_z = f[5];
-        hr = gh[P.y];
-    }
-    const Bound M = merge_bounds(L, R);
-    float *o = gbi + (size_t)p * 6;
-    o[0] = M.min_x; o[1] = M.max_x; o[2] = M.min_y; o[3] = M.max_y; o[4] = M.min_z; o[5] = M.max_z;
-    const int hp = (hl > hr ? hl : hr) + 1;
-    gh[p] = hp;
-    tnodes[p] = make_tnode(L, R, P.x, P.y, P.x < 0 ? 1 : 0, P.y < 0 ? 1 : 0);
-    return hp;
-}
-
-// Pass 2: one workgroup per super-chunk climbs from its list's arrivals through the nodes whose leaf
-// range lies inside the super-chunk (their visit counters see no other workgroup); a climb that
-// reaches a node spanning super-chunks queues the arrival for pass 3.
-__device__ __forceinline__ void mrefit_mid_body(const int4 *mnode, const int *mpar_int, const BVHNodeGPU *btl,
-                                                TNode *tnodes, float *gbi, int *gh, const int2 *xlist,
-                                                const unsigned *xcnt, unsigned *gcnt, int2 *xtop, unsigned *xtop_count,
-                                                unsigned xtop_cap, unsigned *root_height, unsigned *err, unsigned sc) {
-    const unsigned c = xcnt[sc];
-    const unsigned count = c < kXCap ? c : kXCap;
-    auto defer = [&](int node, int child) {
-        const unsigned slot = atomicAdd(xtop_count, 1u);
-        if (slot < xtop_cap) xtop[slot] = make_int2(node, child);
-        else atomicOr(err, 2u);
-    };
-    for (unsigned e = threadIdx.x; e < count; e += blockDim.x) {
-        const int2 E = xlist[(size_t)sc * kXCap + e];
-        int p = E.x;
-        int4 P = mnode[p];
-        if ((unsigned)P.w / kMSuper != sc) {   // spans super-chunks: pass 3
-            defer(p, E.y);
-            continue;
-        }
-        for (int steps = 0;; steps++) {
-            if (steps > kMaxClimb) {
-                atomicOr(err, 4u);
-                break;
-            }
-            const unsigned old = __hip_atomic_fetch_add(gcnt + p, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
-            if (old == 0) break;
-            const int hp = mrefit_node(p, P, btl, tnodes, gbi, gh);
-            const int pp = mpar_int[p];
-            if (pp < 0) {
-                *root_height = (unsigned)hp;
-                break;
-            }
-            const int4 PP = mnode[pp];
-            if ((unsigned)PP.z / kMSuper != (unsigned)PP.w / kMSuper) {
-                defer(pp, p);
-                break;
-            }
-            p = pp;
-            P = PP;
-        }
-    }
-}
-
-// Pass 3: the nodes spanning super-chunks, one workgroup, arrivals from pass 2's queue.
-__device__ __forceinline__ void mrefit_top_body(const int4 *mnode, const int *mpar_int, const BVHNodeGPU *btl,
-                                                TNode *tnodes, float *gbi, int *gh, const int2 *xlist,
-                                                const unsigned *xcount, unsigned xcap, unsigned *gcnt,
-                                                unsigned *root_height, unsigned *err) {
-    const unsigned c = *xcount;
-    const unsigned count = c < xcap ? c : xcap;
-    for (unsigned e = threadIdx.x; e < count; e += blockDim.x) {
-        int p = xlist[e].x;
-        for (int steps = 0;; steps++) {
-            if (steps > kMaxClimb) {
-                atomicOr(err, 4u);
-                break;
-            }
-            const unsigned old = __hip_atomic_fetch_add(gcnt + p, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
-            if (old == 0) break;
-            const int hp = mrefit_node(p, mnode[p], btl, tnodes, gbi, gh);
-            const int pp = mpar_int[p];
-            if (pp < 0) {
-                *root_height = (unsigned)hp;
-                break;
-            }
-            p = pp;
-        }
-    }
+    return k + 1;
 }
 
 }  // namespace ptgpu
