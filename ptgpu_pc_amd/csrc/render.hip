@@ -149,15 +149,43 @@ __global__ __launch_bounds__(256) void k_pack_table(float *tab) {
 
 // The path-tracing megakernel.  Lane state: one pixel (gid), its remaining samples, the RNG state
 // and running mean; path state: ray, radiance, throughput, specularBounce, depth.
-template <int STACK, bool STATS>
+// BRUTE: no tree, and no more than kBrutePrims primitives: they, the first shapes and lights and the camera
+// are read from LDS.
+template <int STACK, bool STATS, bool BRUTE>
 __global__ __launch_bounds__(256) void k_render(RenderParams P) {
     if (recorded_tree_unfit(P)) return;
-    __shared__ int s_stack[STACK * 256];
+    __shared__ int s_stack[BRUTE ? 1 : STACK * 256];
     __shared__ float s_pack[kPackEntries];
     load_pack_table(P.pack_tab, s_pack);
-    __syncthreads();
     int *stk = s_stack + threadIdx.x;
     const DevAccel &A = P.acc;
+    constexpr int kLdsShapes = BRUTE ? 64 : 1, kLdsLights = BRUTE ? 32 : 1;
+    __shared__ BruteScene<BRUTE ? kBrutePrims : 1> s_scene;
+    __shared__ float s_shapes[kLdsShapes * 17], s_lights[kLdsLights * 14];
+    __shared__ Camera s_cam;
+    const Camera *cam = P.camera;
+    if (BRUTE) {
+        brute_stage(A.prims, A.nprims, s_scene);
+        const int ns = A.nshapes < kLdsShapes ? A.nshapes : kLdsShapes;
+        for (int i = threadIdx.x; i < ns * 17; i += blockDim.x)
+            s_shapes[i] = reinterpret_cast<const float *>(P.shapes + i / 17)[i % 17];
+        const int nl = P.nlights < kLdsLights ? P.nlights : kLdsLights;
+        for (int i = threadIdx.x; i < nl * 14; i += blockDim.x) {
+            const float *sw = reinterpret_cast<const float *>(P.shapes + P.lights[i / 14]);
+            s_lights[i] = sw[i % 14 == 13 ? 25 : i % 14];
+        }
+        constexpr int kCamWords = (int)(sizeof(Camera) / sizeof(float));
+        if ((int)threadIdx.x < kCamWords)
+            reinterpret_cast<float *>(&s_cam)[threadIdx.x] = reinterpret_cast<const float *>(P.camera)[threadIdx.x];
+        cam = &s_cam;
+    }
+    __syncthreads();
+    unsigned long long spheres = 0;
+    if (BRUTE) {
+        const unsigned long long m = s_scene.spheres;
+        spheres = (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)m) |
+                  ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(m >> 32)) << 32);
+    }
     const unsigned long long lt = lanemask_lt();
 
     bool active = false, drained = false;
@@ -193,7 +221,7 @@ __global__ __launch_bounds__(256) void k_render(RenderParams P) {
                         s1 = P.seeds[2 * gid + 1];
                         k = 0;
                         if (P.currentSample > 0) col = ldvec(P.colors + ci);
-                        camera_ray(P.camera, s0, s1, P.width, P.height, x, y, ro, rd);
+                        camera_ray(cam, s0, s1, P.width, P.height, x, y, ro, rd);
                         rad = mk(0.f, 0.f, 0.f); thr = mk(1.f, 1.f, 1.f); spec = 1; depth = 0;
                     }
                 }
@@ -209,12 +237,15 @@ __global__ __launch_bounds__(256) void k_render(RenderParams P) {
         } else {
             n_closest++;
             float t;
-            const int id = closest<STACK>(A, ro, rd, &t, stk, pnv, ppt);
+            const int id = BRUTE ? brute_closest_lds(s_scene, spheres, A.nprims, ro, rd, &t)
+                                 : closest<STACK>(A, ro, rd, &t, stk, pnv, ppt);
             if (id < 0) {
                 ended = true;
             } else {
                 const f3 hp = add3(ro, smul(t, rd));
-                const Surface S = surface_at(P.shapes + id, hp, rd);
+                Surface S;
+                if (BRUTE && A.nshapes <= kLdsShapes) S = surface_of(s_shapes + id * 17, hp, rd);
+                else S = surface_at(P.shapes + id, hp, rd);
                 if (!iszero3(S.e)) {
                     if (spec) rad = add3(rad, mul3(thr, smul(fabsf(S.dp), S.e)));
                     ended = true;
@@ -225,9 +256,18 @@ __global__ __launch_bounds__(256) void k_render(RenderParams P) {
                     for (int li = 0; li < P.nlights; li++) {
                         f3 sd, contrib;
                         float len;
-                        if (!sample_light(P.shapes + P.lights[li], s0, s1, hp, S.nl, &sd, &len, &contrib)) continue;
+                        bool shadow;
+                        if (BRUTE && li < kLdsLights)
+                            shadow = sample_light_words(s_lights + li * 14, s_lights[li * 14 + 13], s0, s1, hp, S.nl, &sd,
+                                                        &len, &contrib);
+                        else
+                            shadow = sample_light(P.shapes + P.lights[li], s0, s1, hp, S.nl, &sd, &len, &contrib);
+                        if (!shadow) continue;
                         n_any++;
-                        if (!anyhit<STACK>(A, hp, sd, len - kEpsilon, stk, pnv, ppt)) Ld = add3(Ld, contrib);
+                        const float maxt = len - kEpsilon;
+                        const bool dark = BRUTE ? brute_any_lds(s_scene, spheres, A.nprims, hp, sd, maxt)
+                                                : anyhit<STACK>(A, hp, sd, maxt, stk, pnv, ppt);
+                        if (!dark) Ld = add3(Ld, contrib);
                     }
                     Ld = mul3(thr, Ld);
                     rad = add3(rad, Ld);
@@ -246,7 +286,7 @@ __global__ __launch_bounds__(256) void k_render(RenderParams P) {
             k++;
             if (k < P.spp) {
                 const int x = gid % P.width, y = gid / P.width;
-                camera_ray(P.camera, s0, s1, P.width, P.height, x, y, ro, rd);
+                camera_ray(cam, s0, s1, P.width, P.height, x, y, ro, rd);
                 rad = mk(0.f, 0.f, 0.f); thr = mk(1.f, 1.f, 1.f); spec = 1; depth = 0;
             } else {
                 float *cp = reinterpret_cast<float *>(P.colors + ci);
@@ -1537,11 +1577,13 @@ int launch_render(ptgpu_ctx *ctx, const DevAccel &acc, const RenderLaunch &L) {
 #undef PT_LANES_W
 #undef PT_LANES
     } else if (L.trav_stats) {
-        if (st == 24) hipLaunchKernelGGL((k_render<24, true>), dim3(blocks), dim3(256), 0, ctx->stream, P);
-        else hipLaunchKernelGGL((k_render<64, true>), dim3(blocks), dim3(256), 0, ctx->stream, P);
+        if (st == 24) hipLaunchKernelGGL((k_render<24, true, false>), dim3(blocks), dim3(256), 0, ctx->stream, P);
+        else hipLaunchKernelGGL((k_render<64, true, false>), dim3(blocks), dim3(256), 0, ctx->stream, P);
+    } else if (acc.mode == PTGPU_ACCEL_NONE && acc.nprims <= kBrutePrims) {
+        hipLaunchKernelGGL((k_render<24, false, true>), dim3(blocks), dim3(256), 0, ctx->stream, P);
     } else {
-        if (st == 24) hipLaunchKernelGGL((k_render<24, false>), dim3(blocks), dim3(256), 0, ctx->stream, P);
-        else hipLaunchKernelGGL((k_render<64, false>), dim3(blocks), dim3(256), 0, ctx->stream, P);
+        if (st == 24) hipLaunchKernelGGL((k_render<24, false, false>), dim3(blocks), dim3(256), 0, ctx->stream, P);
+        else hipLaunchKernelGGL((k_render<64, false, false>), dim3(blocks), dim3(256), 0, ctx->stream, P);
     }
     PT_HIP(hipGetLastError());
     return PTGPU_OK;

@@ -160,12 +160,6 @@ __device__ __forceinline__ float prim_isect_vals(const float4 &p0, const float4 
     if ((__float_as_int(p2.w) & 0xff) == SPHERE) return sph_isect(p0, p1.x, o, d);
     return tri_isect(p0, p1, p2, o, d);
 }
-__device__ __forceinline__ float prim_isect_run(const Prim *__restrict__ prims, int k, f3 o, f3 d, int *id,
-                                                bool *last) {
-    const float4 p0 = prims[k].p0, p1 = prims[k].p1, p2 = prims[k].p2;
-    return prim_isect_vals(p0, p1, p2, o, d, id, last);
-}
-
 // the two binary16 halves of a TNode4H word, widened exactly to fp32
 __device__ __forceinline__ float half_lo(unsigned w) {
     return (float)__builtin_bit_cast(_Float16, (unsigned short)(w & 0xffffu));
@@ -354,13 +348,33 @@ __device__ bool trace_any(const DevAccel &A, f3 o, f3 d, float maxt, int skip_id
     return false;
 }
 
-// Brute-force mode (ACCELSTR 0): prims in shape-index order.
+// Buffers that no kernel which reads them this way writes, at addresses that are the same in all lanes: through the
+// constant address space their loads are scalar ones.  (The compiler cannot know that a render's stores to
+// its colours leave the shapes alone, and loads them per lane, each wait a round trip to the L2.)
+typedef float vec4f __attribute__((ext_vector_type(4)));
+template <class T>
+using cmem = const __attribute__((address_space(4))) T;
+template <class T>
+__device__ __forceinline__ cmem<T> *to_cmem(const void *p) {
+    return reinterpret_cast<cmem<T> *>(reinterpret_cast<unsigned long long>(p));
+}
+__device__ __forceinline__ float prim_isect_uniform(cmem<vec4f> *prims, int k, f3 o, f3 d, int *id) {
+    const vec4f a = prims[3 * k], b = prims[3 * k + 1], c = prims[3 * k + 2];
+    const float4 p0 = make_float4(a.x, a.y, a.z, a.w), p1 = make_float4(b.x, b.y, b.z, b.w);
+    const float4 p2 = make_float4(c.x, c.y, c.z, c.w);
+    *id = __float_as_int(p0.w);
+    if ((__float_as_int(p2.w) & 0xff) == SPHERE) return sph_isect(p0, p1.x, o, d);
+    return tri_isect(p0, p1, p2, o, d);
+}
+
+// Brute-force mode (ACCELSTR 0): prims in shape-index order, all lanes at the same one.
 __device__ int brute_closest(const Prim *prims, int n, f3 o, f3 d, float *tout, unsigned *prims_tested) {
+    cmem<vec4f> *const cp = to_cmem<vec4f>(prims);
     float tb = kInf;
     int bid = -1;
     for (int i = n - 1; i >= 0; i--) {
         int id;
-        const float t = prim_isect(prims, i, o, d, &id);
+        const float t = prim_isect_uniform(cp, i, o, d, &id);
         if (t != 0.f && t < tb) { tb = t; bid = id; }
     }
     if (prims_tested) *prims_tested += (unsigned)n;
@@ -368,13 +382,134 @@ __device__ int brute_closest(const Prim *prims, int n, f3 o, f3 d, float *tout, 
     return bid;
 }
 __device__ bool brute_any(const Prim *prims, int n, f3 o, f3 d, float maxt, unsigned *prims_tested) {
+    cmem<vec4f> *const cp = to_cmem<vec4f>(prims);
     for (int i = n - 2; i >= 0; i--) {
         int id;
         if (prims_tested) (*prims_tested)++;
-        const float t = prim_isect(prims, i, o, d, &id);
+        const float t = prim_isect_uniform(cp, i, o, d, &id);
         if (t != 0.f && t < maxt) return true;
     }
     return false;
+}
+
+// The same for up to kBrutePrims primitives held in LDS, four tests at a time.  A frame of 256x256 pixels is one
+// wave per SIMD, so what bounds it is each test's chain of a load, a root and branches; four spheres tested
+// without a branch share one wait and fill each other's latencies.  256x256x4 spp of nine spheres, the whole
+// call: 242 -> 192 us (one scalar load a test: 223 us).  256 triangles: 1.33 -> 1.26 ms; past 256 the scalar
+// loop is as fast (257: 1.26 ms).
+constexpr int kBrutePrims = 256;
+template <int CAP>
+struct BruteScene {
+    float4 p[3 * CAP];                // Prims; a sphere's p[3k].w is its radius squared
+    unsigned long long spheres;       // bit g: primitives 4g .. 4g+3 are spheres (or past the end)
+};
+// by the whole workgroup; the caller synchronises
+template <int CAP>
+__device__ __forceinline__ void brute_stage(const Prim *prims, int n, BruteScene<CAP> &S) {
+    const int padded = (n + 3) & ~3;
+    for (int k = threadIdx.x; k < padded; k += blockDim.x) {
+        const Prim *q = prims + (k < n ? k : 0);
+        float4 p0 = q->p0, p1 = q->p1, p2 = q->p2;
+        if (k >= n || (__float_as_int(p2.w) & 0xff) == SPHERE) {
+            if (k >= n) p1.x = __builtin_nanf("");   // past the end: no hit
+            p0.w = p1.x * p1.x;
+            p2.w = __int_as_float(SPHERE);
+        }
+        S.p[3 * k] = p0;
+        S.p[3 * k + 1] = p1;
+        S.p[3 * k + 2] = p2;
+    }
+    if (threadIdx.x < kWave) {
+        bool all = true;
+        for (int j = 0; j < 4; j++) {
+            const int k = 4 * (int)threadIdx.x + j;
+            all = all && (k >= n || (__float_as_int(prims[k].p2.w) & 0xff) == SPHERE);
+        }
+        const unsigned long long m = __ballot(all);
+        if (threadIdx.x == 0) S.spheres = m;
+    }
+}
+// t of primitives 4g .. 4g+3 (infinity: no hit), as sph_isect and tri_isect give them
+template <int CAP>
+__device__ __forceinline__ void brute_four(const BruteScene<CAP> &S, unsigned long long spheres, int g, f3 o, f3 d, float *t) {
+    constexpr float inf = __builtin_inff();
+    if ((spheres >> g) & 1ull) {
+        float4 c[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) c[j] = S.p[3 * (4 * g + j)];
+        asm volatile("" ::: "memory");   // compiler-only: the four loads stay together
+        float b[4], det[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const f3 op = sub3(mk(c[j].x, c[j].y, c[j].z), o);
+            b[j] = dot3(op, d);
+            det[j] = b[j] * b[j] - dot3(op, op) + c[j].w;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            // sqrt_exact's steps; the root of a negative determinant is a NaN, which fails both comparisons
+            const float y = __builtin_amdgcn_rsqf(det[j]);
+            const float q = det[j] * y;
+            const float r = __builtin_fmaf(__builtin_fmaf(-q, q, det[j]), 0.5f * y, q);
+            const float t0 = b[j] - r, t1 = b[j] + r;
+            const float tt = t0 > kEpsilon ? t0 : t1;
+            t[j] = tt > kEpsilon ? tt : inf;
+        }
+        // a determinant at the ends of the exponent range (from its bits: below 2^-96 from +0 on, or above 2^126)
+        auto bits = [&](int j) { return __float_as_int(det[j]); };
+        auto umin = [](unsigned x, unsigned y) { return x < y ? x : y; };
+        auto imax = [](int x, int y) { return x > y ? x : y; };
+        const unsigned lo = umin(umin(bits(0), bits(1)), umin(bits(2), bits(3)));
+        const int hi = imax(imax(bits(0), bits(1)), imax(bits(2), bits(3)));
+        if (__builtin_expect(__ballot(lo < 0x0f800000u || hi > 0x7e800000) != 0ull, 0)) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const float x = sph_isect(c[j], S.p[3 * (4 * g + j) + 1].x, o, d);
+                t[j] = x != 0.f && x == x ? x : inf;
+            }
+        }
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const float4 p0 = S.p[3 * (4 * g + j)], p1 = S.p[3 * (4 * g + j) + 1], p2 = S.p[3 * (4 * g + j) + 2];
+        float x;
+        if (__builtin_amdgcn_readfirstlane(__float_as_int(p2.w) & 0xff) == SPHERE) x = sph_isect(p0, p1.x, o, d);
+        else x = tri_isect(p0, p1, p2, o, d);
+        t[j] = x != 0.f ? x : inf;
+    }
+}
+template <int CAP>
+__device__ __forceinline__ int brute_closest_lds(const BruteScene<CAP> &S, unsigned long long spheres, int n, f3 o, f3 d,
+                                                 float *tout) {
+    float tb = kInf;
+    int bid = -1;
+    for (int g = (n - 1) >> 2; g >= 0; g--) {
+        float t[4];
+        brute_four(S, spheres, g, o, d, t);
+#pragma unroll
+        for (int j = 3; j >= 0; j--) {
+            bid = t[j] < tb ? 4 * g + j : bid;
+            tb = t[j] < tb ? t[j] : tb;
+        }
+    }
+    *tout = tb;
+    return bid;
+}
+template <int CAP>
+__device__ __forceinline__ bool brute_any_lds(const BruteScene<CAP> &S, unsigned long long spheres, int n, f3 o, f3 d, float maxt) {
+    bool hit = false;
+    for (int g = (n - 2) >> 2; g >= 0 && __ballot(!hit) != 0ull; g--) {
+        float t[4];
+        brute_four(S, spheres, g, o, d, t);
+        if (4 * g + 4 > n - 1) {   // the last shape casts no shadow
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (4 * g + j >= n - 1) t[j] = __builtin_inff();
+        }
+        hit = hit || fminf(fminf(t[0], t[1]), fminf(t[2], t[3])) < maxt;
+    }
+    return hit;
 }
 
 template <int STACK>
@@ -435,14 +570,8 @@ struct Surface {
     float dp;
     int refl;
 };
-PT_HD Surface surface_at(const Shape *sh, f3 hp, f3 rd) {
-    // words 0-16 loaded together before the type is looked at: one memory round trip, where loads
-    // placed in the type's branches would wait for the type word first
-    float w[17];
-    const float *src = reinterpret_cast<const float *>(sh);
-#pragma unroll
-    for (int i = 0; i < 17; i++) w[i] = src[i];
-    asm volatile("" ::: "memory");   // compiler-only: keeps the loads here, ahead of the branches
+// w: words 0-16 of the Shape
+PT_HD Surface surface_of(const float *w, f3 hp, f3 rd) {
     const int type = __builtin_bit_cast(int, w[0]);
     Surface S;
     f3 nrm;
@@ -461,6 +590,16 @@ PT_HD Surface surface_at(const Shape *sh, f3 hp, f3 rd) {
     S.c = mk(w[13], w[14], w[15]);
     S.refl = __builtin_bit_cast(int, w[16]);
     return S;
+}
+PT_HD Surface surface_at(const Shape *sh, f3 hp, f3 rd) {
+    // words 0-16 loaded together before the type is looked at: one memory round trip, where loads
+    // placed in the type's branches would wait for the type word first
+    float w[17];
+    const float *src = reinterpret_cast<const float *>(sh);
+#pragma unroll
+    for (int i = 0; i < 17; i++) w[i] = src[i];
+    asm volatile("" ::: "memory");   // compiler-only: keeps the loads here, ahead of the branches
+    return surface_of(w, hp, rd);
 }
 
 // ---- one light of SampleLights (rendering_kernel.cl:421-490): draws two randoms (u1 first),
