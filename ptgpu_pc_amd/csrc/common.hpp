@@ -227,9 +227,11 @@ int record_stage(ptgpu_ctx *ctx, hipStream_t stream, const void *src, size_t cop
 
 namespace ptgpu {
 // light list: indices of the first `light_cnt` shapes with non-zero emission, in index order
-// (the scan order of SampleLights, rendering_kernel.cl:415-423).  Writes *found on the host.
+// (the scan order of SampleLights, rendering_kernel.cl:415-423).  Their number is read back into *found; with
+// on_device it stays on the device instead (the emitters of all shapes, in the word **on_device points to, none
+// where light_cnt is 0), *found is light_cnt, and nothing is waited for.
 int build_light_list(ptgpu_ctx *ctx, const Shape *d_shapes, int n, int light_cnt, DevBuf &out_lights,
-                     DevBuf &scan_tmp, int *found);
+                     DevBuf &scan_tmp, int *found, const unsigned **on_device = nullptr);
 int build_pack_table(ptgpu_ctx *ctx);
 // brute-force layout: prims in shape-index order
 int build_index_prims(ptgpu_ctx *ctx, const Shape *d_shapes, int n, DevBuf &out_prims);
@@ -246,7 +248,7 @@ size_t wide_bytes(const DevAccel &acc);
 int build_wide_into(ptgpu_ctx *ctx, DevAccel *acc, TNode4 *w4);   // room for wide_bytes(*acc)
 size_t light_scan_bytes(int n);
 int build_light_list_into(ptgpu_ctx *ctx, const Shape *d_shapes, int n, int light_cnt, int *out, unsigned *scan,
-                          int *found);
+                          int *found, const unsigned **on_device = nullptr);
 size_t ref_parents_bytes(int n);
 int convert_bvh_ref_into(ptgpu_ctx *ctx, const Shape *d_shapes, int n, const BVHNodeGPU *d_btn,
                          const BVHNodeGPU *d_btl, TNode *nodes, Prim *prims, int *parents, DevAccel *acc);
@@ -265,7 +267,8 @@ struct RenderLaunch {
     const Shape *shapes;
     unsigned int shapeCnt;
     const int *lights;
-    int nlights;
+    int nlights;                             // lights in the list; with lights_found: the most it may hold
+    const unsigned *lights_found = nullptr;  // device word: emitters found (their count was not read back)
     int width, height, currentSample, spp, max_depth;
     unsigned int *pixels;
     unsigned long long *ray_counter;
@@ -276,9 +279,10 @@ struct RenderLaunch {
     bool no_alloc = false;   // the allocation-free entry: kernels that need no scratch memory only
 };
 int launch_render(ptgpu_ctx *ctx, const DevAccel &acc, const RenderLaunch &L);
-// ptgpu_render's checks and preparation (traversal structure, light list) without the launch
+// ptgpu_render's checks and preparation (traversal structure, light list) without the launch; lights_on_device:
+// the number of lights may stay on the device (RenderLaunch::lights_found)
 int prepare_render(ptgpu_ctx *ctx, ptgpu_clbvh *bvh, ptgpu_kdtree *kd, const ptgpu_render_args *a, DevAccel *acc,
-                   RenderLaunch *L);
+                   RenderLaunch *L, bool lights_on_device = false);
 // ptgpu_render's preparation, then a launch over the listed tiles (device int2 origins, tile_w x tile_h
 // each); acc and L receive the resolved structure and launch description (host tiles use them too)
 int render_tiles(ptgpu_ctx *ctx, ptgpu_clbvh *bvh, ptgpu_kdtree *kd, const ptgpu_render_args *a, const int2 *d_tiles,

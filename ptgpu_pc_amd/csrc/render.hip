@@ -48,6 +48,7 @@ struct RenderParams {
     const Shape *shapes;
     const int *lights;
     int nlights;
+    const unsigned *lights_found; // single frames: device word with the emitters found; NULL: nlights is their number
     int width, height, currentSample, spp, max_depth;
     unsigned *pixels;
     unsigned long long *ray_counter;
@@ -133,6 +134,13 @@ __device__ __forceinline__ int claimed_pixel(const RenderParams &P, unsigned m) 
     return (x < P.width && y < P.height) ? y * P.width + x : -1;
 }
 
+// the launch's lights
+__device__ __forceinline__ int launch_lights(const RenderParams &P) {
+    if (!P.lights_found) return P.nlights;
+    const int found = __builtin_amdgcn_readfirstlane((int)*P.lights_found);
+    return found < P.nlights ? found : P.nlights;
+}
+
 __device__ __forceinline__ void load_pack_table(const float *tab, float *s_pack) {
     for (int i = threadIdx.x; i < kPackEntries; i += blockDim.x) s_pack[i] = tab[i];
 }
@@ -159,6 +167,7 @@ __global__ __launch_bounds__(256) void k_render(RenderParams P) {
     load_pack_table(P.pack_tab, s_pack);
     int *stk = s_stack + threadIdx.x;
     const DevAccel &A = P.acc;
+    const int nlights = launch_lights(P);
     constexpr int kLdsShapes = BRUTE ? 64 : 1, kLdsLights = BRUTE ? 32 : 1;
     __shared__ BruteScene<BRUTE ? kBrutePrims : 1> s_scene;
     __shared__ float s_shapes[kLdsShapes * 17], s_lights[kLdsLights * 14];
@@ -169,7 +178,7 @@ __global__ __launch_bounds__(256) void k_render(RenderParams P) {
         const int ns = A.nshapes < kLdsShapes ? A.nshapes : kLdsShapes;
         for (int i = threadIdx.x; i < ns * 17; i += blockDim.x)
             s_shapes[i] = reinterpret_cast<const float *>(P.shapes + i / 17)[i % 17];
-        const int nl = P.nlights < kLdsLights ? P.nlights : kLdsLights;
+        const int nl = nlights < kLdsLights ? nlights : kLdsLights;
         for (int i = threadIdx.x; i < nl * 14; i += blockDim.x) {
             const float *sw = reinterpret_cast<const float *>(P.shapes + P.lights[i / 14]);
             s_lights[i] = sw[i % 14 == 13 ? 25 : i % 14];
@@ -253,7 +262,7 @@ __global__ __launch_bounds__(256) void k_render(RenderParams P) {
                     spec = 0;
                     thr = mul3(thr, S.c);
                     f3 Ld = mk(0.f, 0.f, 0.f);
-                    for (int li = 0; li < P.nlights; li++) {
+                    for (int li = 0; li < nlights; li++) {
                         f3 sd, contrib;
                         float len;
                         bool shadow;
@@ -381,8 +390,9 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
     __shared__ float s_pack[kPackEntries];
     load_pack_table(P.pack_tab, s_pack);
     int n_lds_lights = 0;
+    const int p_nlights = MULTI ? 0 : launch_lights(P);
     if (!MULTI) {
-        n_lds_lights = P.nlights < kLdsLights ? P.nlights : kLdsLights;
+        n_lds_lights = p_nlights < kLdsLights ? p_nlights : kLdsLights;
         for (int i = threadIdx.x; i < n_lds_lights * 16; i += blockDim.x) {
             const int l = i >> 4, w = i & 15;
             const float *sw = reinterpret_cast<const float *>(P.shapes + P.lights[l]);
@@ -410,7 +420,7 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
     // claim on (a field read through the job table is one more dependent load)
     const gmem<const Shape> *j_shapes = to_gmem(P.shapes);
     const gmem<const int> *j_lights = to_gmem(P.lights);
-    int j_nlights = P.nlights, j_max_depth = P.max_depth;
+    int j_nlights = p_nlights, j_max_depth = P.max_depth;
     // and those every new sample reads
     const gmem<const Camera> *j_camera = to_gmem(P.camera);
     int j_width = P.width, j_height = P.height, j_spp = P.spp, j_currentSample = P.currentSample;
@@ -640,7 +650,7 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
                 rd = rd2;
                 n_any++;
                 start(true, maxt2);
-            } else if (li < JFR(nlights)) {
+            } else if (li < j_nlights) {
                 st = kLight;
             } else {
                 end_bounce();
@@ -772,7 +782,7 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
                 // bounce.
                 float len = 0.f;
                 bool shoot = false;
-                const int nlights = JFR(nlights);
+                const int nlights = j_nlights;
                 while (li < nlights && !more) {
                     f3 sd, con;
                     const bool sh = !MULTI && li < n_lds_lights
@@ -1039,60 +1049,64 @@ __global__ void k_index_prims(const Shape *shapes, int n, Prim *prims) {
     if (i < n) prims[i] = prim_of(shapes + i, i, kLastInLeaf);
 }
 
-__device__ __forceinline__ bool emits(const Shape *s) {
-    const float *w = reinterpret_cast<const float *>(s);
-    return !(w[10] == 0.f && w[11] == 0.f && w[12] == 0.f);
-}
-
+// A block's 4096 shapes, sixteen a thread, their emission loaded at once: bit q is shape base + 256 q + thread.
 constexpr int kLightChunk = 4096;
+__device__ __forceinline__ unsigned emitters(const Shape *shapes, int n, int base) {
+    float e[16][3];
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+        const int i = base + 256 * q + (int)threadIdx.x;
+        const float *w = reinterpret_cast<const float *>(shapes + (i < n ? i : 0));
+        e[q][0] = w[10]; e[q][1] = w[11]; e[q][2] = w[12];
+    }
+    asm volatile("" ::: "memory");   // compiler-only: the loads stay together
+    unsigned m = 0;
+#pragma unroll
+    for (int q = 0; q < 16; q++)
+        if (base + 256 * q + (int)threadIdx.x < n && !(e[q][0] == 0.f && e[q][1] == 0.f && e[q][2] == 0.f)) m |= 1u << q;
+    return m;
+}
 __global__ __launch_bounds__(256) void k_light_count(const Shape *shapes, int n, unsigned *counts) {
     __shared__ unsigned s_c;
     if (threadIdx.x == 0) s_c = 0;
     __syncthreads();
-    unsigned c = 0;
-    const int base = blockIdx.x * kLightChunk;
-    for (int q = threadIdx.x; q < kLightChunk; q += 256) {
-        const int i = base + q;
-        if (i < n && emits(shapes + i)) c++;
-    }
+    const unsigned c = (unsigned)__popc(emitters(shapes, n, blockIdx.x * kLightChunk));
     if (c) atomicAdd(&s_c, c);
     __syncthreads();
     if (threadIdx.x == 0) counts[blockIdx.x] = s_c;
 }
-__global__ void k_light_scan(unsigned *counts, int nb, unsigned *total) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    unsigned run = 0;
-    for (int b = 0; b < nb; b++) {
-        unsigned c = counts[b];
-        counts[b] = run;
-        run += c;
-    }
-    *total = run;
-}
-__global__ __launch_bounds__(256) void k_light_write(const Shape *shapes, int n, const unsigned *offs, int cap,
-                                                     int *out) {
-    __shared__ unsigned s_w[4];
+// The list itself and its length; a block starts after the emitters of the blocks before it (a single one needs no
+// counts).  What bounds it for one frame's scene is its launch and two round trips: with the flags loaded one
+// by one, a scan kernel between and the length read back, the nine shapes of a 256x256x4 frame took 42 of its 192 us for the list.
+__global__ __launch_bounds__(256) void k_light_write(const Shape *shapes, int n, const unsigned *counts, int cap,
+                                                     int *out, unsigned *total) {
+    __shared__ unsigned s_w[4][16], s_run;
     const int base = blockIdx.x * kLightChunk;
-    unsigned run = offs[blockIdx.x];
-    for (int q0 = 0; q0 < kLightChunk; q0 += 256) {
-        const int i = base + q0 + threadIdx.x;
-        const unsigned f = (i < n && emits(shapes + i)) ? 1u : 0u;
-        // block exclusive scan of f
-        const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-        unsigned x = f;
-        for (int o = 1; o < 64; o <<= 1) {
-            unsigned y = __shfl_up(x, o, 64);
-            if (lane >= o) x += y;
-        }
-        if (lane == 63) s_w[w] = x;
-        __syncthreads();
-        unsigned pre = 0, tot = 0;
-        for (int k2 = 0; k2 < 4; k2++) { if (k2 < w) pre += s_w[k2]; tot += s_w[k2]; }
-        __syncthreads();
-        const unsigned pos = run + pre + x - f;
-        if (f && (int)pos < cap) out[pos] = i;
-        run += tot;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (threadIdx.x == 0) s_run = 0;
+    __syncthreads();
+    unsigned before = 0;
+    for (int b = threadIdx.x; b < (int)blockIdx.x; b += 256) before += counts[b];
+    if (before) atomicAdd(&s_run, before);
+    const unsigned m = emitters(shapes, n, base);
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+        const unsigned long long f = __ballot((m >> q) & 1u);
+        if (lane == 0) s_w[w][q] = (unsigned)__popcll(f);
     }
+    __syncthreads();
+    unsigned run = s_run;
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+        const unsigned long long f = __ballot((m >> q) & 1u);
+        unsigned pos = run + (unsigned)__popcll(f & ((1ull << lane) - 1ull));
+        for (int k = 0; k < 4; k++) {
+            if (k < w) pos += s_w[k][q];
+            run += s_w[k][q];
+        }
+        if (((m >> q) & 1u) && pos < (unsigned)cap) out[pos] = base + 256 * q + (int)threadIdx.x;
+    }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *total = run;
 }
 
 // TNode -> TNode4: the four grandchildren of binary node i (a leaf child is kept as it is).  Refs
@@ -1290,8 +1304,9 @@ int build_wide_into(ptgpu_ctx *ctx, DevAccel *acc, TNode4 *w4) {
 size_t light_scan_bytes(int n) { return ((size_t)((n + kLightChunk - 1) / kLightChunk) + 4) * 4; }
 
 int build_light_list(ptgpu_ctx *ctx, const Shape *d_shapes, int n, int light_cnt, DevBuf &out, DevBuf &scan,
-                     int *found) {
+                     int *found, const unsigned **on_device) {
     *found = 0;
+    if (on_device) *on_device = nullptr;
     if (light_cnt <= 0 || n <= 0) {
         PT_TRY(out.ensure(4));
         return PTGPU_OK;
@@ -1299,23 +1314,29 @@ int build_light_list(ptgpu_ctx *ctx, const Shape *d_shapes, int n, int light_cnt
     PT_NO_CAPTURE(ctx, "building a light list");
     PT_TRY(scan.ensure(light_scan_bytes(n)));
     PT_TRY(out.ensure((size_t)light_cnt * 4));
-    return build_light_list_into(ctx, d_shapes, n, light_cnt, out.as<int>(), scan.as<unsigned>(), found);
+    return build_light_list_into(ctx, d_shapes, n, light_cnt, out.as<int>(), scan.as<unsigned>(), found, on_device);
 }
 
 int build_light_list_into(ptgpu_ctx *ctx, const Shape *d_shapes, int n, int light_cnt, int *out, unsigned *scan,
-                          int *found) {
+                          int *found, const unsigned **on_device) {
     *found = 0;
+    if (on_device) *on_device = nullptr;
     if (light_cnt <= 0 || n <= 0) return PTGPU_OK;
     PT_NO_CAPTURE(ctx, "building a light list");
     const int nb = (n + kLightChunk - 1) / kLightChunk;
     unsigned *counts = scan;
     unsigned *total = counts + nb;
-    hipLaunchKernelGGL(k_light_count, dim3(nb), dim3(256), 0, ctx->stream, d_shapes, n, counts);
+    if (nb > 1) {
+        hipLaunchKernelGGL(k_light_count, dim3(nb), dim3(256), 0, ctx->stream, d_shapes, n, counts);
+        PT_HIP(hipGetLastError());
+    }
+    hipLaunchKernelGGL(k_light_write, dim3(nb), dim3(256), 0, ctx->stream, d_shapes, n, counts, light_cnt, out, total);
     PT_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_light_scan, dim3(1), dim3(64), 0, ctx->stream, counts, nb, total);
-    PT_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_light_write, dim3(nb), dim3(256), 0, ctx->stream, d_shapes, n, counts, light_cnt, out);
-    PT_HIP(hipGetLastError());
+    if (on_device) {
+        *on_device = total;
+        *found = light_cnt;
+        return PTGPU_OK;
+    }
     unsigned h_total = 0;
     PT_HIP(hipMemcpyAsync(&h_total, total, 4, hipMemcpyDeviceToHost, ctx->stream));
     PT_HIP(hipStreamSynchronize(ctx->stream));
@@ -1504,6 +1525,7 @@ int launch_render(ptgpu_ctx *ctx, const DevAccel &acc, const RenderLaunch &L) {
     P.shapes = L.shapes;
     P.lights = L.lights;
     P.nlights = L.nlights;
+    P.lights_found = L.lights_found;
     P.width = L.width;
     P.height = L.height;
     P.currentSample = L.currentSample;
@@ -1706,8 +1728,10 @@ static int radiance_gpu_impl(ptgpu_ctx *ctx, int accel, const ptgpu_radiance_arg
         PT_TRY(resolve_accel(ctx, nullptr, nullptr, a->shapes, a->shapeCnt, &acc));
     }
     int nl = 0;
-    PT_TRY(build_light_list(ctx, a->shapes, n, (int)a->lightCnt, ctx->tmp_lights, ctx->tmp_scan, &nl));
     RenderLaunch L;
+    // (the wavefront engine sizes its queues by the number of lights)
+    PT_TRY(build_light_list(ctx, a->shapes, n, (int)a->lightCnt, ctx->tmp_lights, ctx->tmp_scan, &nl,
+                            ctx->engine == 2 ? nullptr : &L.lights_found));
     L.colors = a->colors;
     L.seeds = a->seeds;
     L.camera = a->camera;
@@ -1893,7 +1917,7 @@ int ptgpu_radiance_gpu_noalloc(ptgpu_ctx *ctx, int accel, const ptgpu_radiance_a
 // Checks a ptgpu_render argument set, resolves its traversal structure and light list (the handle's
 // prepared layout, or index-order primitives without a tree) and fills the launch description.
 int ptgpu::prepare_render(ptgpu_ctx *ctx, ptgpu_clbvh *bvh, ptgpu_kdtree *kd, const ptgpu_render_args *a,
-                          DevAccel *acc, RenderLaunch *L) {
+                          DevAccel *acc, RenderLaunch *L, bool lights_on_device) {
     PT_CHECK(ctx && a, PTGPU_ERR_INVALID, "null argument");
     PT_CHECK(a->colors && a->seeds && a->camera && a->shapes, PTGPU_ERR_INVALID, "null buffer");
     PT_CHECK(a->shapeCnt >= 1, PTGPU_ERR_INVALID, "shapeCnt is 0");
@@ -1919,7 +1943,7 @@ int ptgpu::prepare_render(ptgpu_ctx *ctx, ptgpu_clbvh *bvh, ptgpu_kdtree *kd, co
         PT_TRY(kdtree_lights(kd, a->shapes, (int)a->shapeCnt, (int)a->lightCnt, &lights, &nl));
     } else {
         PT_TRY(build_light_list(ctx, a->shapes, (int)a->shapeCnt, (int)a->lightCnt, ctx->tmp_lights, ctx->tmp_scan,
-                                &nl));
+                                &nl, lights_on_device && ctx->engine != 2 ? &L->lights_found : nullptr));
         lights = ctx->tmp_lights.as<int>();
     }
     L->colors = a->colors;
@@ -1959,7 +1983,7 @@ extern "C" {
 int ptgpu_render(ptgpu_ctx *ctx, ptgpu_clbvh *bvh, ptgpu_kdtree *kd, const ptgpu_render_args *a) {
     DevAccel acc;
     RenderLaunch L;
-    PT_TRY(prepare_render(ctx, bvh, kd, a, &acc, &L));
+    PT_TRY(prepare_render(ctx, bvh, kd, a, &acc, &L, true));
     return launch_render(ctx, acc, L);
 }
 
