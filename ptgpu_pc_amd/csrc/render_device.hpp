@@ -203,38 +203,39 @@ PT_HD float slab(float lx, float ly, float lz, float hx, float hy, float hz, f3 
 // A ray's side of the test, set once per query (RaySlab): per axis, the rotation that brings the
 // near bound of a bound word into its low half (0 when the reciprocal direction is >= 0, where lo is
 // nearer; 16 otherwise), the reciprocal, and the offset -o/d once lowered (near) and once raised (far)
-// by 2^-21 of itself.  Choosing near and far by the direction's sign gives the values a min and a max
+// by a step.  Choosing near and far by the direction's sign gives the values a min and a max
 // of the two distances would (rounding is monotone), with no min/max pair per axis.
 //
-// Against slab()'s (bound - o) * (1/d) the rounded product o * (1/d) brings an error of at most 2^-24
-// of itself, and the fma's own rounding the relative error that slab() has too; the widened offsets
-// cover the first eight times over, and the slack on the exit distance is slab()'s.  So the test accepts
-// every box slab() accepts and a few more.  The reciprocal is held to +-2^100: a larger one (a ray
-// in an axis plane) would make bound * (1/d) + (-o/d) infinity minus infinity.  At that size a plane at
-// any distance a binary32 coordinate shows is beyond every query's limit (1e20), so the clamp changes no
-// answer.  Where a distance is NaN all the same (an origin beyond 1e8 on such a ray) the test ignores
+// Against slab()'s (bound - o) * (1/d) the product o * (1/d) is rounded: the offsets are moved one step of binary32
+// to the safe side of it.  The fma's own rounding is the relative error that slab() has too, and the slack on
+// the exit distance is slab()'s.  So the test accepts every box slab() accepts and hardly more.
+//
+// The reciprocal is held to +-2^100: a larger one (a ray in an axis plane) would make bound * (1/d) + (-o/d)
+// infinity minus infinity.  Being a power of two it makes both terms exact, so a box is hit on that axis if the
+// origin lies within its bounds, as with slab(), where the bound that the origin lies on does not count (zero
+// times infinity); the offsets' step, at least 2^-40 of the coordinate's unit, keeps that one from counting here,
+// also at zero.  Where a distance is NaN all the same (an origin beyond 1e8 on such a ray) the test ignores
 // that axis's bound, which only accepts more boxes.
 struct RaySlab {
     unsigned rx, ry, rz;
     f3 inv, on, of;
 };
-__device__ __forceinline__ RaySlab ray_slab_inv(f3 o, f3 inv) {
-    RaySlab r;
-    r.inv = inv;
-    r.rx = inv.x >= 0.f ? 0u : 16u;
-    r.ry = inv.y >= 0.f ? 0u : 16u;
-    r.rz = inv.z >= 0.f ? 0u : 16u;
-    constexpr float kWiden = 4.76837158e-7f;   // 2^-21
-    const f3 p = mk(-o.x * inv.x, -o.y * inv.y, -o.z * inv.z);
-    r.on = mk(p.x - fabsf(p.x) * kWiden, p.y - fabsf(p.y) * kWiden, p.z - fabsf(p.z) * kWiden);
-    r.of = mk(p.x + fabsf(p.x) * kWiden, p.y + fabsf(p.y) * kWiden, p.z + fabsf(p.z) * kWiden);
-    return r;
-}
 __device__ __forceinline__ RaySlab ray_slab(f3 o, f3 d) {
-    // the hardware's reciprocal (one ulp): it scales both of an axis's distances alike, far within the slack
-    constexpr float kMost = 0x1p100f;
-    auto inv = [](float x) { return fminf(fmaxf(__builtin_amdgcn_rcpf(x), -kMost), kMost); };
-    return ray_slab_inv(o, mk(inv(d.x), inv(d.y), inv(d.z)));
+    RaySlab r;
+    auto axis = [](float ox, float dx, unsigned &rot, float &inv, float &on, float &of) {
+        constexpr float kMost = 0x1p100f;
+        // the hardware's reciprocal (one ulp): it scales both of an axis's distances alike, far within the slack
+        inv = fminf(fmaxf(__builtin_amdgcn_rcpf(dx), -kMost), kMost);
+        rot = inv >= 0.f ? 0u : 16u;
+        const float p = -ox * inv;
+        const float s = fmaxf(fabsf(p) * 0x1.8p-24f, fabsf(inv) * 0x1p-40f);
+        on = p - s;
+        of = p + s;
+    };
+    axis(o.x, d.x, r.rx, r.inv.x, r.on.x, r.of.x);
+    axis(o.y, d.y, r.ry, r.inv.y, r.on.y, r.of.y);
+    axis(o.z, d.z, r.rz, r.inv.z, r.on.z, r.of.z);
+    return r;
 }
 
 // The entry distance's bits (as an unsigned number they order as the distances do), at least 4, or 0 on a miss.

@@ -136,6 +136,38 @@ def test_unusual_rays(ctx):
     _both_walks(ctx, bvh, None, d_sh, len(s), rays, maxt)
 
 
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_rays_in_box_planes(ctx, axis):
+    """Rays with zero direction components from planes that boxes on both sides share, at zero and elsewhere: both
+    sides' boxes are walked.  Three layers of a grid of triangles on multiples of 1/8, where every test is exact: a
+    ray through an edge or a corner hits all its triangles at one t, and the answer is the highest of their ids.
+    (Not compared with the binary nodes' walk, whose test drops a box that has the origin on its bound.)"""
+    say("case rays in box planes", axis)
+    i, j, k = (v.ravel() for v in np.meshgrid(np.arange(-8, 8), np.arange(-8, 8), np.arange(3), indexing="ij"))
+    lo = np.stack([i, j, -k], axis=1) / 8.0
+    corner = lambda dx, dy: np.roll(lo + np.array([dx, dy, 0.0]) / 8.0, axis, axis=1).astype(F32)
+    s = scenes.soup(2 * len(lo), seed=1)[0][-2 * len(lo):].copy()
+    s["p1"], s["p2"], s["p3"] = (np.concatenate(v) for v in ((corner(0, 0), corner(1, 1)), (corner(1, 0), corner(0, 1)),
+                                                             (corner(0, 1), corner(1, 0))))
+    s["b"] = _moved(s, 0.0)["b"]
+    s, _ = O.clbvh_construct(s)
+    x, y = (v.ravel() for v in np.meshgrid(np.arange(-17, 18), np.arange(-17, 18), indexing="ij"))
+    rays = random_rays(2 * len(x), 1)
+    o = np.stack([x / 16.0, y / 16.0, np.ones(len(x))], axis=1)
+    rays["o"] = np.roll(np.concatenate([o, o]), axis, axis=1).astype(F32)
+    d = np.concatenate([np.tile([0.0, 0.0, -1.0], (len(x), 1)), np.tile([-0.0, -0.0, -1.0], (len(x), 1))])
+    rays["d"] = np.roll(d, axis, axis=1).astype(F32)
+    d_sh = ctx.to_device(s)
+    bvh = pt.CLBVH(ctx, d_sh)
+    bvh.buildRadixTree()
+    bvh.buildBVHTree()
+    t, ids = gpu_trace(ctx, bvh, None, d_sh, len(s), rays)
+    t_o, id_o = O.trace_closest(s, O.accel_none(), rays)
+    assert (id_o >= 0).sum() > 1000
+    np.testing.assert_array_equal(ids, id_o)
+    np.testing.assert_array_equal(t[id_o >= 0], t_o[id_o >= 0])
+
+
 # binary16 bounds are absolute: from offsets of some tens of the scene's size on they blur its shapes
 @pytest.mark.parametrize("offset", [0.0, 8.0, 40.0, 1000.0, 60000.0, 70000.0])
 def test_far_scenes(ctx, offset):
