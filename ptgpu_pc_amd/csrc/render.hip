@@ -371,7 +371,7 @@ enum : int {
 };
 constexpr unsigned kShadowMin = 8;   // finished shadow rays that a full wave leaves the traversal loop for
 
-template <int STACK, bool STATS, bool WIDE, bool MULTI, bool HALF>
+template <int STACK, bool STATS, bool WIDE, bool MULTI, bool HALF, bool WAIT = false>
 __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && STACK <= 48 ? 3 : 1) void k_render_lanes(RenderParams P) {
     if (!MULTI && recorded_tree_unfit(P)) return;
     if (MULTI && P.status && recorded_jobs_unfit(P)) return;
@@ -535,6 +535,9 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
             if ((unsigned)__popcll(trav) <= dense_min || (unsigned)__popcll(live & ~trav) >= regroup ||
                 (unsigned)__popcll(__ballot(st == kADone)) >= shadow_min)
                 break;
+            if (HALF && st == kTrav) {
+                if (half_step<STACK, STATS, WAIT>(Q, T, stk, &st_nodes, &st_prims)) st = qany ? kADone : kCDone;
+            }
             if (!WIDE && st == kTrav) {
                 bool done = false;
                 if ((unsigned)node >= (unsigned)t_nnodes || ++nv > kMaxVisits) {
@@ -572,9 +575,6 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
                     }
                 }
                 if (done) st = qany ? kADone : kCDone;
-            }
-            if (HALF && st == kTrav) {
-                if (half_step<STACK, STATS>(Q, T, stk, &st_nodes, &st_prims)) st = qany ? kADone : kCDone;
             }
             if (WIDE && !HALF && st == kTrav) {
                 bool done = false;
@@ -953,7 +953,7 @@ __device__ __forceinline__ bool half_blurs(const DevAccel &A) {
 // take rays from cost more than it evened out (0.74 ms with one stretch a wave, 2 ms with the counter).  Bound by
 // the step's instructions and its loads.  One million closest-hit and as many any-hit queries of a 65,538-shape
 // soup, half of them from inside it in any direction: 1.42 -> 0.65 ms; 30,000: 0.53 -> 0.12; 1,000: 0.43 -> 0.063.
-template <int STACK>
+template <int STACK, bool WAIT>
 __global__ __launch_bounds__(256, STACK <= 36 ? 4 : 2) void k_trace_half(DevAccel A, const Ray *rays, const float *maxt,
                                                                          int n, float *tout, int *idout, int *hitout,
                                                                          int any, int lanes, int regroup_max, int quad,
@@ -1034,7 +1034,7 @@ __global__ __launch_bounds__(256, STACK <= 36 ? 4 : 2) void k_trace_half(DevAcce
         for (;;) {
             walk = __ballot(st == kWalk);
             if (__popcll(walk) <= quad || (unsigned)__popcll(live & ~walk) >= regroup) break;
-            if (st == kWalk && half_step<STACK, false>(W, T, stk, nullptr, nullptr)) st = kDone;
+            if (st == kWalk && half_step<STACK, false, WAIT>(W, T, stk, nullptr, nullptr)) st = kDone;
         }
         const unsigned ready = (unsigned)__popcll(live & ~walk);
         if (walk && ready < regroup &&
@@ -1576,6 +1576,14 @@ int launch_render(ptgpu_ctx *ctx, const DevAccel &acc, const RenderLaunch &L) {
         if (tiny) {
             if (L.trav_stats) PT_LANES(kStackTiny, true, true, true);
             else PT_LANES(kStackTiny, false, true, true);
+        } else if (half && acc.mode == PTGPU_ACCEL_KD && !L.trav_stats && (shortst || sw == 32)) {
+            // leaves of several primitives (counting launches keep one walk order)
+            if (shortst)
+                hipLaunchKernelGGL((k_render_lanes<kStackShort, false, true, false, true, true>), dim3(blocks), dim3(256),
+                                   0, ctx->stream, P);
+            else
+                hipLaunchKernelGGL((k_render_lanes<32, false, true, false, true, true>), dim3(blocks), dim3(256), 0,
+                                   ctx->stream, P);
         } else if (shortst) {
             if (L.trav_stats) PT_LANES(kStackShort, true, true, true);
             else PT_LANES(kStackShort, false, true, true);
@@ -1631,14 +1639,17 @@ int launch_trace(ptgpu_ctx *ctx, const DevAccel &acc, unsigned int shapeCnt, con
         const int per_cu = sw == 32 ? 4 : shortst ? (lanes == kWave ? 3 : 4) : sw == 48 ? 3 : 2;
         long long blocks = ((long long)n + 4 * lanes - 1) / (4 * lanes);
         if (blocks > (long long)cus * per_cu) blocks = (long long)cus * per_cu;
-#define PT_TRACE(ST)                                                                                                  \
-    hipLaunchKernelGGL(k_trace_half<ST>, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, acc, d_rays, d_maxt, n, d_t, d_id, \
-                       d_hit, any ? 1 : 0, lanes, 8, ctx->quad, half_slack(ST, acc))
+#define PT_TRACE_W(ST, WAIT)                                                                                          \
+    hipLaunchKernelGGL((k_trace_half<ST, WAIT>), dim3((unsigned)blocks), dim3(256), 0, ctx->stream, acc, d_rays, d_maxt, n, \
+                       d_t, d_id, d_hit, any ? 1 : 0, lanes, 8, ctx->quad, half_slack(ST, acc))
+#define PT_TRACE(ST) \
+    do { if (acc.mode == PTGPU_ACCEL_KD) PT_TRACE_W(ST, true); else PT_TRACE_W(ST, false); } while (0)
         if (sw == 32) PT_TRACE(32);
         else if (shortst) PT_TRACE(kStackShort);
         else if (sw == 48) PT_TRACE(48);
         else PT_TRACE(64);
 #undef PT_TRACE
+#undef PT_TRACE_W
         PT_HIP(hipGetLastError());
         return PTGPU_OK;
     }

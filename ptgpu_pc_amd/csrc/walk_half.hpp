@@ -17,6 +17,7 @@ namespace ptgpu {
 constexpr int kStackShort = 36;
 constexpr int kStackTiny = 8;   // a test class: nearly every walk outgrows it (tuning short_stack 2)
 constexpr int kOverflowSp = 1 << 20;
+constexpr int kLeafMin = 24;
 template <int STACK>
 constexpr bool kIsShort = STACK == kStackShort || STACK == kStackTiny;
 
@@ -87,6 +88,19 @@ __device__ __forceinline__ bool half_refill(HalfWalk &W, const int *stk) {
     W.sp = n - (both ? 2 : 1);
     return n == 0;
 }
+// The same in a step without leaf tests: a lane whose leaf waits takes the top entry only if that is a node.
+__device__ __forceinline__ bool half_refill_waiting(HalfWalk &W, const int *stk) {
+    const int n = W.sp;
+    const int e1 = stk[(n > 1 ? n - 1 : 0) * 256], e2 = stk[(n > 1 ? n - 2 : 0) * 256];
+    const bool waits = W.leaf < 0;
+    const bool both = !waits && n > 1 && (e1 ^ e2) < 0;
+    const int x = both ? e2 : e1;
+    const int node = e1 > x ? e1 : x;
+    W.node = n > 0 ? node : -1;
+    W.leaf = waits ? W.leaf : e1 < x ? e1 : x;
+    W.sp = n - (both ? 2 : waits && (e1 < 0 || n == 0) ? 0 : 1);
+    return n == 0 && !waits;
+}
 
 // A walk that outgrew the short stack is finished against every primitive, from the best hit found
 // so far.  The closest hit is the least (t, then the higher id) whatever the order of the tests,
@@ -116,13 +130,29 @@ __device__ void half_finish_overflowed(HalfWalk &W, const HalfTree &T, unsigned 
 // one with no node reads node 0 (both exist in a tree with binary16 nodes), and ignores them.  With no
 // branch around the loads the wait for the primitive leaves the node's four loads in flight, so the
 // triangle test overlaps the node's latency.
-template <int STACK, bool STATS>
+//
+// WAIT: leaves wait until kLeafMin lanes have one, or an eighth of the lanes can do nothing else, and a lane whose
+// leaf waits goes on with its nodes.  The test takes as long for one lane as for all, and longer where leaves hold
+// several primitives (KD trees): 640x480x4 of a 20,492-shape SAH tree 3.04 -> 2.75 ms,
+// a million queries of a 20,000-shape one 0.64 -> 0.51 ms.  A leaf of one primitive is not
+// worth the wait, which leaves the box tests a stale limit (327,692-shape mesh: 18.2 -> 18.8 ms).
+template <int STACK, bool STATS, bool WAIT>
 __device__ __forceinline__ bool half_step(HalfWalk &W, const HalfTree &T, int *stk, unsigned *st_nodes,
                                           unsigned *st_prims) {
     constexpr bool kShort = kIsShort<STACK>;
+    bool test = true;
+    if (WAIT) {
+        const unsigned long long leaves = __ballot(W.leaf < 0), nodes = __ballot(W.node >= 0);
+        test = __popcll(leaves) >= kLeafMin || 8 * __popcll(leaves & ~nodes) >= __popcll(leaves | nodes);
+    }
     const int first = ~W.leaf;
     const Prim *pp = from_gmem(T.prims) + (first > 0 ? first : 0);
-    float4 a0 = pp->p0, a1 = pp->p1, a2 = pp->p2;
+    float4 a0, a1, a2;
+    if (test) {
+        a0 = pp->p0;
+        a1 = pp->p1;
+        a2 = pp->p2;
+    }
     // compiler-only barrier (no operands, no instruction): the primitive's loads stay
     // here, ahead of the node's, instead of sinking into the branch that tests them
     asm volatile("" ::: "memory");
@@ -130,7 +160,7 @@ __device__ __forceinline__ bool half_step(HalfWalk &W, const HalfTree &T, int *s
     const uint4 q0 = np->c[0], q1 = np->c[1], q2 = np->c[2], q3 = np->c[3];
     bool done = false;
     // the pending run (one primitive per LBVH leaf), before the boxes so tb is tight
-    if (W.leaf < 0) {
+    if (test && W.leaf < 0) {
         // true: the run ends here (an occluder found, or its last primitive)
         auto test_prim = [&](const float4 &b0, const float4 &b1, const float4 &b2) -> bool {
             int id;
@@ -179,7 +209,7 @@ __device__ __forceinline__ bool half_step(HalfWalk &W, const HalfTree &T, int *s
             W.sp += nh;
         }
     }
-    if (!done) done = half_refill(W, stk);
+    if (!done) done = test ? half_refill(W, stk) : half_refill_waiting(W, stk);
     if (kShort && W.sp == kOverflowSp) half_finish_overflowed<STATS>(W, T, st_prims);
     return done;
 }
