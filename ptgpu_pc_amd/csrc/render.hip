@@ -134,6 +134,17 @@ __device__ __forceinline__ int claimed_pixel(const RenderParams &P, unsigned m) 
     return (x < P.width && y < P.height) ? y * P.width + x : -1;
 }
 
+// The kernel's arguments, to be read where they are used: the shading pass of the per-lane-state kernel reads some
+// forty words of them, which the compiler would load once and keep, and then has no scalar register left for
+// the traversal loop (32 of them were spilled to lanes of a vector register, and 12 vector registers to scratch;
+// now 11 and 7).  1024x768x16 of the 327,692-shape mesh 18.2 -> 17.75 ms, 800x600 of a 20,492-shape one 2.25 -> 2.09,
+// 97x61 of a 332-shape one 0.265 -> 0.250.
+__device__ __forceinline__ cmem<RenderParams> *launch_args() {
+    auto *p = (cmem<RenderParams> *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return p;
+}
+
 // the launch's lights
 __device__ __forceinline__ int launch_lights(const RenderParams &P) {
     if (!P.lights_found) return P.nlights;
@@ -669,31 +680,32 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
                 continue;
             }
         }
+        cmem<RenderParams> *const args = launch_args();
         // ---- shading pass: pixels for lanes that need one (one atomic per wave) ----
         const unsigned long long need = __ballot(st == kNeed);
         if (need) {
             const unsigned cnt = (unsigned)__popcll(need);
             const int leader = __ffsll((long long)need) - 1;
             unsigned base = 0;
-            if ((int)__lane_id() == leader) base = atomicAdd(P.work_counter, cnt);
+            if ((int)__lane_id() == leader) base = atomicAdd(args->work_counter, cnt);
             base = __shfl(base, leader, kWave);
-            if (base + cnt >= (unsigned)P.total) drained = true;
+            if (base + cnt >= (unsigned)args->total) drained = true;
             if (st == kNeed) {
                 const unsigned my = base + (unsigned)__popcll(need & lt);
-                if (my < (unsigned)P.total) {
+                if (my < (unsigned)args->total) {
                     if (MULTI) {   // the job holding work item `my` (prefix sums of the jobs' pixel counts)
                         // two loops rather than one over a selected pointer, so the LDS search
                         // compiles to LDS reads (a pointer that may be either would be a flat one)
-                        int lo = 0, hi = P.njobs - 1;
+                        int lo = 0, hi = args->njobs - 1;
                         unsigned first;
-                        if (P.njobs <= kLdsJobs) {
+                        if (args->njobs <= kLdsJobs) {
                             while (lo < hi) {
                                 const int mid = (lo + hi + 1) >> 1;
                                 if (s_job_begin[mid] <= my) lo = mid; else hi = mid - 1;
                             }
                             first = s_job_begin[lo];
                         } else {
-                            const gmem<const unsigned> *jbg = to_gmem(P.job_begin);
+                            const gmem<const unsigned> *jbg = to_gmem(args->job_begin);
                             while (lo < hi) {
                                 const int mid = (lo + hi + 1) >> 1;
                                 if (jbg[mid] <= my) lo = mid; else hi = mid - 1;
@@ -726,14 +738,14 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
                         gid = claimed_pixel(P, my);
                     }
                     if (gid >= 0) {
-                        const int W = JFR(width), H = JFR(height);
+                        const int W = (MULTI ? j_width : args->width), H = (MULTI ? j_height : args->height);
                         const int x = gid % W, y = gid / W;
-                        s0 = JF(seeds)[2 * gid];
-                        s1 = JF(seeds)[2 * gid + 1];
+                        s0 = to_gmem(MULTI ? P.jobs[jb].seeds : args->seeds)[2 * gid];
+                        s1 = to_gmem(MULTI ? P.jobs[jb].seeds : args->seeds)[2 * gid + 1];
                         k = 0;
-                        if (JFR(currentSample) > 0) {
+                        if ((MULTI ? j_currentSample : args->currentSample) > 0) {
                             const gmem<const float> *cv =
-                                reinterpret_cast<const gmem<const float> *>(JF(colors) + (H - y - 1) * W + x);
+                                reinterpret_cast<const gmem<const float> *>(to_gmem(MULTI ? P.jobs[jb].colors : args->colors) + (H - y - 1) * W + x);
                             col = mk(cv[0], cv[1], cv[2]);
                         }
                         camera_ray(MULTI ? from_gmem(j_camera) : &s_cam, s0, s1, W, H, x, y, ro, rd);
@@ -754,7 +766,7 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
                     st = kEnded;
                 } else {
                     const f3 hp = add3(ro, smul(tb, rd));
-                    const Surface S = surface_at(JSHAPES + bid, hp, rd);
+                    const Surface S = surface_at((MULTI ? from_gmem(j_shapes) : args->shapes) + bid, hp, rd);
                     if (!iszero3(S.e)) {
                         if (spec) rad = add3(rad, mul3(thr, smul(fabsf(S.dp), S.e)));
                         st = kEnded;
@@ -788,7 +800,7 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
                     const bool sh = !MULTI && li < n_lds_lights
                                         ? sample_light_words(s_lights + 16 * li, s_lights[16 * li + 13], s0, s1, ro,
                                                              nl, &sd, &len, &con)
-                                        : sample_light(JSHAPES + (MULTI ? from_gmem(j_lights) : P.lights)[li], s0, s1, ro, nl, &sd, &len,
+                                        : sample_light((MULTI ? from_gmem(j_shapes) : args->shapes) + (MULTI ? from_gmem(j_lights) : args->lights)[li], s0, s1, ro, nl, &sd, &len,
                                                        &con);
                     li++;
                     if (!sh) continue;
@@ -812,22 +824,22 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
                 }
                 end_bounce();
             }
-            if (st == kSeg && depth > JFR(max_depth)) st = kEnded;
+            if (st == kSeg && depth > (MULTI ? j_max_depth : args->max_depth)) st = kEnded;
             if (st == kEnded) {
-                col = running_mean(col, rad, JFR(currentSample) + k);
+                col = running_mean(col, rad, (MULTI ? j_currentSample : args->currentSample) + k);
                 k++;
-                const int W = JFR(width), H = JFR(height);
+                const int W = (MULTI ? j_width : args->width), H = (MULTI ? j_height : args->height);
                 const int x = gid % W, y = gid / W;
-                if (k < JFR(spp)) {
+                if (k < (MULTI ? j_spp : args->spp)) {
                     camera_ray(MULTI ? from_gmem(j_camera) : &s_cam, s0, s1, W, H, x, y, ro, rd);
                     rad = mk(0.f, 0.f, 0.f); thr = mk(1.f, 1.f, 1.f); spec = true; depth = 0;
                     st = kSeg;
                 } else {
-                    gmem<float> *cp = reinterpret_cast<gmem<float> *>(JF(colors) + (H - y - 1) * W + x);
+                    gmem<float> *cp = reinterpret_cast<gmem<float> *>(to_gmem(MULTI ? P.jobs[jb].colors : args->colors) + (H - y - 1) * W + x);
                     cp[0] = col.x; cp[1] = col.y; cp[2] = col.z;
-                    gmem<unsigned> *px = JF(pixels);
+                    gmem<unsigned> *px = to_gmem(MULTI ? P.jobs[jb].pixels : args->pixels);
                     if (px) px[y * W + x] = pack_rgba_tab(col, s_pack);
-                    gmem<unsigned> *sd = JF(seeds);
+                    gmem<unsigned> *sd = to_gmem(MULTI ? P.jobs[jb].seeds : args->seeds);
                     sd[2 * gid] = s0;
                     sd[2 * gid + 1] = s1;
                     st = drained ? kIdle : kNeed;
@@ -840,26 +852,27 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
         }
         if (fresh) set_up();
     }
-    if (P.ray_counter) {
+    cmem<RenderParams> *const args = launch_args();
+    if (args->ray_counter) {
         unsigned long long a = n_closest, b = n_any;
         for (int o = 32; o > 0; o >>= 1) {
             a += __shfl_down(a, o, kWave);
             b += __shfl_down(b, o, kWave);
         }
         if (__lane_id() == 0) {
-            atomicAdd(P.ray_counter, a);
-            atomicAdd(P.ray_counter + 1, b);
+            atomicAdd(args->ray_counter, a);
+            atomicAdd(args->ray_counter + 1, b);
         }
     }
-    if (STATS && P.trav_stats) {
+    if (STATS && args->trav_stats) {
         unsigned long long a = st_nodes, b = st_prims;
         for (int o = 32; o > 0; o >>= 1) {
             a += __shfl_down(a, o, kWave);
             b += __shfl_down(b, o, kWave);
         }
         if (__lane_id() == 0) {
-            atomicAdd(P.trav_stats, a);
-            atomicAdd(P.trav_stats + 1, b);
+            atomicAdd(args->trav_stats, a);
+            atomicAdd(args->trav_stats + 1, b);
         }
     }
 #undef JF
