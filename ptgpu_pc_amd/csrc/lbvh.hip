@@ -77,15 +77,21 @@ __global__ __launch_bounds__(256) void k_morton(Shape *shapes, int n, const floa
                                                 const ShapeBox *boxes) {
     morton_body(shapes, n, scene6, keys, boxes, blockIdx.x);
 }
+// Small scenes: every block folds the partial bounds itself.  Up to 64 of them are two round trips; the launch that
+// folds them is 6 us of a 1,003-shape build's 115.
+constexpr int kFoldBlocks = 64;
+__global__ __launch_bounds__(256) void k_morton_fold(Shape *shapes, int n, const float *partials, int nblocks, float *scene6,
+                                                     unsigned *keys, const ShapeBox *boxes) {
+    __shared__ float s_scene6[6];
+    bounds_final_body(partials, nblocks, s_scene6);
+    __syncthreads();
+    if (blockIdx.x == 0 && threadIdx.x < 6) scene6[threadIdx.x] = s_scene6[threadIdx.x];
+    morton_body(shapes, n, s_scene6, keys, boxes, blockIdx.x);
+}
 
 template <int BITS>
 __global__ __launch_bounds__(kSortThreads) void k_sort_hist(const unsigned *keys, int n, unsigned *hist) {
     sort_hist_body<BITS>(keys, n, hist, blockIdx.x, gridDim.x);
-}
-
-template <int BITS>
-__global__ __launch_bounds__(kSortThreads) void k_sort_scan(unsigned *hist) {
-    sort_scan_body<BITS>(hist);
 }
 
 template <int BITS, int IN, int OUT>
@@ -93,13 +99,13 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_pass(const unsigned *__re
                                                             const unsigned *__restrict__ vals_in,
                                                             unsigned *__restrict__ keys_out,
                                                             unsigned *__restrict__ vals_out, int n, int shift,
-                                                            const unsigned *__restrict__ digit_base,
+                                                            const unsigned *__restrict__ digit_count,
                                                             unsigned *status, unsigned *tile_counter,
                                                             unsigned *err) {
     __shared__ unsigned s_tile;
     if (threadIdx.x == 0) s_tile = atomicAdd(tile_counter, 1u);
     __syncthreads();
-    sort_pass_body<BITS, IN, OUT>(keys_in, vals_in, keys_out, vals_out, n, shift, digit_base, status,
+    sort_pass_body<BITS, IN, OUT>(keys_in, vals_in, keys_out, vals_out, n, shift, digit_count, status,
                                   __builtin_amdgcn_readfirstlane(s_tile), err);
 }
 
@@ -182,11 +188,17 @@ static int clbvh_construct(ptgpu_clbvh *h) {
     hipLaunchKernelGGL(k_bounds, dim3(blocks), dim3(kBoundsThreads), 0, st, (const Shape *)h->d_shapes, n,
                        misc_partials(h), h->boxes.as<ShapeBox>());
     PT_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(kBoundsThreads), 0, st, (const float *)misc_partials(h), blocks,
-                       misc_scene6(h));
-    PT_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_morton, dim3((n + 255) / 256), dim3(256), 0, st, h->d_shapes, n, misc_scene6(h),
-                       h->keysA.as<unsigned>(), (const ShapeBox *)h->boxes.as<ShapeBox>());
+    if (blocks <= kFoldBlocks) {
+        hipLaunchKernelGGL(k_morton_fold, dim3((n + 255) / 256), dim3(256), 0, st, h->d_shapes, n,
+                           (const float *)misc_partials(h), blocks, misc_scene6(h), h->keysA.as<unsigned>(),
+                           (const ShapeBox *)h->boxes.as<ShapeBox>());
+    } else {
+        hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(kBoundsThreads), 0, st, (const float *)misc_partials(h), blocks,
+                           misc_scene6(h));
+        PT_HIP(hipGetLastError());
+        hipLaunchKernelGGL(k_morton, dim3((n + 255) / 256), dim3(256), 0, st, h->d_shapes, n, misc_scene6(h),
+                           h->keysA.as<unsigned>(), (const ShapeBox *)h->boxes.as<ShapeBox>());
+    }
     PT_HIP(hipGetLastError());
     PT_HIP(hipEventRecord(h->ev[1], st));
     h->timed[0] = true;
@@ -284,8 +296,6 @@ static int clbvh_sort(ptgpu_clbvh *h) {
     if (hblocks < 1) hblocks = 1;
     hipLaunchKernelGGL(k_sort_hist<BITS>, dim3(hblocks), dim3(kSortThreads), 0, st, h->keysA.as<unsigned>(), n, hist);
     PT_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_sort_scan<BITS>, dim3(1), dim3(kSortThreads), 0, st, hist);
-    PT_HIP(hipGetLastError());
     // The first pass reads the Morton keys (values: the shape indices) and writes packed (key, value)
     // words; the middle passes go between the two packed buffers; the last writes the sorted keys back
     // over the Morton keys and the sorted values beside them (an even number of passes).
@@ -315,7 +325,7 @@ static int clbvh_sort(ptgpu_clbvh *h) {
 namespace ptgpu {
 // The Morton-keyed tree's height is known on the device after the refit; the traversal stack is
 // sized from it, so the first use after a build reads it back (one 4-byte copy).
-int clbvh_prepare_traversal(ptgpu_clbvh *h, bool recording, bool exact) {
+int clbvh_prepare_traversal(ptgpu_clbvh *h, bool recording, bool exact, bool wide) {
     const int known = h->known_height[h->optimized ? 1 : 0];
     const bool no_readback = recording || h->ctx->capturing || (h->speculate && known > 0);
     if (h->height_pending && exact)
@@ -343,9 +353,11 @@ int clbvh_prepare_traversal(ptgpu_clbvh *h, bool recording, bool exact) {
         h->known_height[h->optimized ? 1 : 0] = (int)w[2];
         h->height_pending = false;
     }
-    if (h->wide_pending) {
+    if (h->wide_pending && wide) {
         PT_TRY(build_wide(h->ctx, &h->acc, h->tnodes4));
         h->wide_pending = false;
+    } else if (h->wide_pending && h->n > 1) {   // (a later recording may not allocate)
+        PT_TRY(h->tnodes4.ensure((size_t)(h->n - 1) * (sizeof(TNode4) + sizeof(TNode4H))));
     }
     return PTGPU_OK;
 }

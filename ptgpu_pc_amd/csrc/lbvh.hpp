@@ -8,8 +8,9 @@
 namespace ptgpu {
 // Makes the handle's traversal layout current (tree height, four-wide nodes).  `recording`: the
 // caller's stream is being recorded into a graph, so nothing may be read back.  `exact`: the caller
-// needs the tree's height itself, not a bound checked on the device (exports, batch queries).
-int clbvh_prepare_traversal(ptgpu_clbvh *h, bool recording = false, bool exact = false);
+// needs the tree's height itself, not a bound checked on the device (exports, batch queries).  `wide` false:
+// the four-wide nodes stay pending (the caller is about to change the tree).
+int clbvh_prepare_traversal(ptgpu_clbvh *h, bool recording = false, bool exact = false, bool wide = true);
 // Height bound of a traversal recorded before the height could be read back: the height last read
 // for a build of the same kind (plain or optimised) plus this margin, or the default without one.
 constexpr int kRecordedHeightMargin = 4;

@@ -1,6 +1,6 @@
 // lbvh_batch.hip -- many LBVH builds in one sequence of launches (ptgpu_clbvh_build_batch).
 //
-// Every stage of the build (bounds, Morton, Karras topology, radix-sort histogram / scan / passes,
+// Every stage of the build (bounds, Morton, Karras topology, radix-sort histogram / passes,
 // level refit, Morton-keyed traversal tree) runs as ONE launch over all scenes.  A per-stage table
 // of block offsets (prefix sums of each scene's block count) is the work queue: block b of a launch
 // finds its scene by binary search and plays block (b - offset) of that scene, running the same
@@ -100,11 +100,6 @@ __global__ __launch_bounds__(kSortThreads) void kb_sort_hist(const BuildSeg *g, 
     const int s = seg_find(starts, ns, blockIdx.x);
     const BuildSeg &S = g[s];
     sort_hist_body<BITS>(S.keysA, S.n, S.hist, blockIdx.x - starts[s], starts[s + 1] - starts[s]);
-}
-
-template <int BITS>
-__global__ __launch_bounds__(kSortThreads) void kb_sort_scan(const BuildSeg *g) {
-    sort_scan_body<BITS>(g[blockIdx.x].hist);
 }
 
 // Pass p of every scene's sort.  Pass 0 reads the Morton keys in keysA with implicit values
@@ -296,8 +291,6 @@ int build_batch(ptgpu_ctx *ctx, ptgpu_clbvh *const *hs, int ns) {
     PT_BATCH_LAUNCH(kb_morton, kStMorton, 256);
     PT_BATCH_LAUNCH(kb_karras, kStKarras, 256);
     PT_BATCH_LAUNCH(kb_sort_hist<BITS>, kStHist, kSortThreads);
-    hipLaunchKernelGGL(kb_sort_scan<BITS>, dim3(ns), dim3(kSortThreads), 0, st, d_segs);
-    PT_HIP(hipGetLastError());
     static_assert(C::kPasses % 2 == 0, "the passes end in the packed buffer the first one wrote");
     for (int p = 0; p < C::kPasses; p++) {
         if (p == 0) {

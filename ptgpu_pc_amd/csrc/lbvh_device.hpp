@@ -238,8 +238,7 @@ __device__ __forceinline__ void morton_body(Shape *shapes, int n, const float *s
 // -------------------------------------------------------------------------------------------
 // Stage 2: onesweep LSD radix sort (Adinets & Merrill 2022) for wave64.
 //   k_sort_hist:   one read of the keys builds the digit histograms of every pass.
-//   k_sort_scan:   exclusive scan of each pass histogram (global digit bases).
-//   k_sort_pass:   per 4096-key tile: wave-level match ranking in input order (stable), tile
+//   k_sort_pass:   per 4096-key tile: the pass's digit bases from its histogram, wave-level match ranking in input order (stable), tile
 //                  histogram, decoupled look-back over earlier tiles per digit, LDS shuffle into
 //                  digit order, coalesced scatter.  Tile ids come from an atomic counter so every
 //                  tile a block waits on has already started.
@@ -297,21 +296,6 @@ __device__ __forceinline__ unsigned block_exscan256(unsigned v, unsigned *s_w, u
     return pre + x - v;
 }
 
-template <int BITS>
-__device__ __forceinline__ void sort_scan_body(unsigned *hist) {
-    using C = SortCfg<BITS>;
-    __shared__ unsigned s_w[kSortWaves];
-    for (int p = 0; p < C::kPasses; p++) {
-        for (int base = 0; base < C::kRadix; base += kSortThreads) {
-            int d = base + threadIdx.x;
-            unsigned v = d < C::kRadix ? hist[p * C::kRadix + d] : 0u;
-            unsigned tot;
-            unsigned ex = block_exscan256(v, s_w, &tot);
-            if (d < C::kRadix) hist[p * C::kRadix + d] = ex;   // kRadix <= 256: one round
-        }
-    }
-}
-
 // The element forms of a pass's input and output.  kSplit: a key array and a value array (an input
 // without a value array takes each element's index as its value).  kPacked: one 8-byte word per
 // element, the key in its low half and the value in its high half, read from / written to the
@@ -323,7 +307,7 @@ enum SortForm { kSplit = 0, kPacked = 1 };
 template <int BITS, int IN = kSplit, int OUT = kSplit>
 __device__ __forceinline__ void sort_pass_body(const unsigned *__restrict__ keys_in, const unsigned *__restrict__ vals_in,
                                                unsigned *__restrict__ keys_out, unsigned *__restrict__ vals_out, int n,
-                                               int shift, const unsigned *__restrict__ digit_base, unsigned *status,
+                                               int shift, const unsigned *__restrict__ digit_count, unsigned *status,
                                                unsigned tile, unsigned *err) {
     using C = SortCfg<BITS>;
     __shared__ unsigned long long s_kv[kSortTile];   // the tile in digit order, key | value << 32
@@ -391,6 +375,7 @@ __device__ __forceinline__ void sort_pass_body(const unsigned *__restrict__ keys
             cnt = run;
         }
         unsigned tot;
+        const unsigned dbase = block_exscan256(d < C::kRadix ? digit_count[d] : 0u, s_w, &tot);   // kRadix <= 256
         unsigned lofs = block_exscan256(cnt, s_w, &tot);
         if (d < C::kRadix) {
             s_lofs[d] = lofs;
@@ -431,7 +416,7 @@ __device__ __forceinline__ void sort_pass_body(const unsigned *__restrict__ keys
                 }
                 st_relaxed(my, kFlagPrefix | ((prefix + cnt) & kValMask));
             }
-            s_gofs[d] = digit_base[d] + prefix;
+            s_gofs[d] = dbase + prefix;
         }
     }
     __syncthreads();

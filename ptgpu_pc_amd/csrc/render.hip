@@ -137,8 +137,8 @@ __device__ __forceinline__ int claimed_pixel(const RenderParams &P, unsigned m) 
 // The kernel's arguments, to be read where they are used: the shading pass of the per-lane-state kernel reads some
 // forty words of them, which the compiler would load once and keep, and then has no scalar register left for
 // the traversal loop (32 of them were spilled to lanes of a vector register, and 12 vector registers to scratch;
-// now 11 and 7).  1024x768x16 of the 327,692-shape mesh 18.2 -> 17.75 ms, 800x600 of a 20,492-shape one 2.25 -> 2.09,
-// 97x61 of a 332-shape one 0.265 -> 0.250.
+// now 11 and 7).  1024x768x16 of the 327,692-shape mesh 18.2 -> 17.75 ms, 640x480 of the 65,538-shape soup by
+// RadianceGPU 2.25 -> 2.09, 97x61 of a 332-shape mesh 0.265 -> 0.250.
 __device__ __forceinline__ cmem<RenderParams> *launch_args() {
     auto *p = (cmem<RenderParams> *)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(p));

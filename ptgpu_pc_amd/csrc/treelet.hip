@@ -166,6 +166,9 @@ __global__ __launch_bounds__(64 * WAVES) void k_treelet(const int *__restrict__ 
     __shared__ int s_int[NG][kMaxTreelet];
     __shared__ int s_nl[NG];
     __shared__ float s_cur[NG];
+    // the rebuilt treelet's child slots (node, subset | side << 7, child), written by all lanes of the group
+    __shared__ int s_enode[NG][2 * kMaxTreelet - 2], s_eref[NG][2 * kMaxTreelet - 2], s_ne[NG];
+    __shared__ unsigned char s_eset[NG][2 * kMaxTreelet - 2];
     const int lane = threadIdx.x, grp = lane / kGroup, sub = lane % kGroup;
     // a treelet leaf j: ref, box and subtree cost, taken from the record of its parent
     auto put_leaf = [&](int j, int ref, const float *box, float cost) {
@@ -285,9 +288,10 @@ __global__ __launch_bounds__(64 * WAVES) void k_treelet(const int *__restrict__ 
                 }
                 __syncthreads();
             }
-            if (root >= 0 && sub == 0) {
+            if (sub == 0) {
                 float root_cost = s_cur[grp];
-                if (nl >= 3 && s_cost[grp][full] < s_cur[grp] * (1.f - 1e-6f)) {
+                int ne = 0;
+                if (root >= 0 && nl >= 3 && s_cost[grp][full] < s_cur[grp] * (1.f - 1e-6f)) {
                     root_cost = s_cost[grp][full];
                     // rebuild top-down, reusing the treelet's internal nodes (the root keeps its slot)
                     int st_set[kMaxTreelet], st_node[kMaxTreelet], sp = 0, next = 1;
@@ -297,7 +301,6 @@ __global__ __launch_bounds__(64 * WAVES) void k_treelet(const int *__restrict__ 
                         --sp;
                         const int S = st_set[sp], node = st_node[sp];
                         const int parts[2] = {s_best[grp][S], S ^ s_best[grp][S]};
-                        OptNode &o = on[node];
                         for (int side = 0; side < 2; side++) {
                             const int X = parts[side];
                             int cref;
@@ -308,20 +311,31 @@ __global__ __launch_bounds__(64 * WAVES) void k_treelet(const int *__restrict__ 
                                 st_set[sp] = X;
                                 st_node[sp++] = cref;
                             }
-                            if (cref >= 0) on[cref].parent = node;
-                            float lo[3], hi[3];
-                            union_of(X, lo, hi);
-                            for (int a = 0; a < 3; a++) {
-                                o.cb[side][a] = lo[a];
-                                o.cb[side][3 + a] = hi[a];
-                            }
-                            o.c[side] = cref;
-                            o.cc[side] = s_cost[grp][X];
+                            s_enode[grp][ne] = node;
+                            s_eref[grp][ne] = cref;
+                            s_eset[grp][ne++] = (unsigned char)(X | (side << 7));
                         }
                     }
                 }
+                s_ne[grp] = ne;
                 // hand the subtree's cost to the parent's record (siblings write different slots)
-                if (par >= 0) on[par].cc[pslot] = root_cost;
+                if (root >= 0 && par >= 0) on[par].cc[pslot] = root_cost;
+            }
+            __syncthreads();
+            // the slots' boxes and costs, a lane each: the leader alone took a quarter of a treelet's time for them
+            for (int e = sub; e < s_ne[grp]; e += kGroup) {
+                const int X = s_eset[grp][e] & 127, side = s_eset[grp][e] >> 7, node = s_enode[grp][e];
+                const int cref = s_eref[grp][e];
+                if (cref >= 0) on[cref].parent = node;
+                OptNode &o = on[node];
+                float lo[3], hi[3];
+                union_of(X, lo, hi);
+                for (int a = 0; a < 3; a++) {
+                    o.cb[side][a] = lo[a];
+                    o.cb[side][3 + a] = hi[a];
+                }
+                o.c[side] = cref;
+                o.cc[side] = s_cost[grp][X];
             }
             __syncthreads();
         }
@@ -372,7 +386,7 @@ int opt_layout(ptgpu_clbvh *h, OptLayout *L) {
 int clbvh_optimize(ptgpu_clbvh *h, int tsize) {
     const int n = h->n, m = n - 1;
     if (m < 2) return PTGPU_OK;   // at most two leaves: one shape only
-    PT_TRY(clbvh_prepare_traversal(h));   // current height: the number of levels to visit
+    PT_TRY(clbvh_prepare_traversal(h, false, false, false));   // current height: the number of levels to visit
     const int levels = h->acc.depth;      // internal depths are 0 .. height - 1
     PT_CHECK(levels >= 1 && levels < kMaxLevels, PTGPU_ERR_UNSUPPORTED, "tree height %d", levels);
     hipStream_t st = h->ctx->stream;
