@@ -1573,12 +1573,13 @@ int launch_render(ptgpu_ctx *ctx, const DevAccel &acc, const RenderLaunch &L) {
     // auto and engine 3: per-lane states whenever there is a tree to walk (measured fastest at every
     // size tried); brute force and single-leaf scenes keep the lockstep megakernel
     if (lanes_engine) {
-        const int sw = acc.nodes4 && ctx->wide ? stack_for_wide(acc, ctx->stack_min) : -1;
+        int sw = acc.nodes4 && ctx->wide ? stack_for_wide(acc, ctx->stack_min) : -1;
+        if (half && L.no_alloc && sw == 32) sw = 48;   // (the 32-entry class spills too, see below)
         if (sw > 0) P.depth_cap = wide_depth_cap(sw);
         // the binary16 walk of a tree in the 48-entry class runs on the short stack, four workgroups
         // per CU (short_stack 2, a test setting, runs every binary16 walk on the 8-entry class).  Held
-        // to 128 registers, the short class keeps one in scratch memory, which the allocation-free
-        // entry does not ask the runtime for.
+        // to 128 registers, it and the 32-entry class keep seven or eight in scratch memory, which the
+        // allocation-free entry does not ask the runtime for.
         const bool tiny = half && sw > 0 && ctx->short_stack == 2 && !L.no_alloc;
         const bool shortst = half && sw == 48 && ctx->short_stack == 1 && !L.no_alloc;
         if (half && sw > 0) P.slack = half_slack(tiny ? kStackTiny : shortst ? kStackShort : sw, acc);
