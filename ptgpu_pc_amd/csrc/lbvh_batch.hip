@@ -202,7 +202,7 @@ int build_batch(ptgpu_ctx *ctx, ptgpu_clbvh *const *hs, int ns) {
         blocks(kStMorton, s) = (n + 255) / 256;
         blocks(kStKarras, s) = 0;   // the refit writes whole btn/btl records (topology included)
         int hb = (int)((n + kSortThreads * 8 - 1) / (kSortThreads * 8));
-        blocks(kStHist, s) = hb > 2048 ? 2048 : hb < 1 ? 1 : hb;
+        blocks(kStHist, s) = hb > 512 ? 512 : hb < 1 ? 1 : hb;
         blocks(kStTiles, s) = S.tiles;
         for (int p = 0; p < kMaxRefitPasses; p++) {
             const int s0 = p * kRefitLog;

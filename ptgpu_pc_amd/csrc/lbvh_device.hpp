@@ -87,6 +87,17 @@ __device__ __forceinline__ void wave_store_records(const unsigned *stage, unsign
     const int rem = total - 4 * full;
     if (lane < rem) dst[4 * full + lane] = stage[4 * full + lane];
 }
+// words [w0, w1) of the stage
+__device__ __forceinline__ void wave_store_words(const unsigned *stage, unsigned *dst, int w0, int w1, int lane) {
+    for (int c = (w0 >> 2) + lane; 4 * c < w1; c += kWave) {
+        if (4 * c >= w0 && 4 * c + 4 <= w1) {
+            *reinterpret_cast<uint4 *>(dst + 4 * c) = *reinterpret_cast<const uint4 *>(stage + 4 * c);
+        } else {
+            for (int e = 4 * c; e < 4 * c + 4; e++)
+                if (e >= w0 && e < w1) dst[e] = stage[e];
+        }
+    }
+}
 template <int WORDS>
 __device__ __forceinline__ void wave_load_records(const unsigned *src, unsigned *stage, int count, int lane) {
     const int total = count * WORDS;
@@ -263,10 +274,17 @@ __device__ __forceinline__ void sort_hist_body(const unsigned *keys, int n, unsi
     __shared__ unsigned sh[C::kPasses * C::kRadix];
     for (int j = threadIdx.x; j < C::kPasses * C::kRadix; j += kSortThreads) sh[j] = 0;
     __syncthreads();
-    for (int i = bid * kSortThreads + threadIdx.x; i < n; i += nblocks * kSortThreads) {
-        unsigned k = keys[i];
+    const long long stride = (long long)nblocks * kSortThreads;
+    for (long long i = (long long)bid * kSortThreads + threadIdx.x; i < n; i += 4 * stride) {
+        unsigned k[4];   // four keys' loads together
 #pragma unroll
-        for (int p = 0; p < C::kPasses; p++) atomicAdd(&sh[p * C::kRadix + ((k >> (p * BITS)) & C::kMask)], 1u);
+        for (int j = 0; j < 4; j++) k[j] = i + j * stride < n ? keys[i + j * stride] : 0u;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (i + j * stride >= n) break;
+#pragma unroll
+            for (int p = 0; p < C::kPasses; p++) atomicAdd(&sh[p * C::kRadix + ((k[j] >> (p * BITS)) & C::kMask)], 1u);
+        }
     }
     __syncthreads();
     for (int j = threadIdx.x; j < C::kPasses * C::kRadix; j += kSortThreads)
@@ -684,7 +702,12 @@ __device__ __forceinline__ void refit_levels_body(const ShapeBox *boxes, const u
             sb[0][ls] = M.min_x; sb[1][ls] = M.max_x; sb[2][ls] = M.min_y;
             sb[3][ls] = M.max_y; sb[4][ls] = M.min_z; sb[5][ls] = M.max_z;
             const int idx = karras_index(lo, hi, n);
-            write_node_record(btn + idx, (int)lo, (int)hi, (int)mid, index_tree_parent(lo, s, n), M);
+            if (LEAF) {   // kept at the split, which no later level reads, for the records below
+                sb[0][rs] = M.min_x; sb[1][rs] = M.max_x; sb[2][rs] = M.min_y;
+                sb[3][rs] = M.max_y; sb[4][rs] = M.min_z; sb[5][rs] = M.max_z;
+            } else {
+                write_node_record(btn + idx, (int)lo, (int)hi, (int)mid, index_tree_parent(lo, s, n), M);
+            }
             if (tnodes_on) {
                 const int rl = child_ref(lo, mid - 1, n), rr = child_ref(mid, hi, n);
                 tnodes[idx] = make_tnode(L, R, rl, rr, rl < 0 ? 1 : 0, rr < 0 ? 1 : 0);
@@ -693,6 +716,52 @@ __device__ __forceinline__ void refit_levels_body(const ShapeBox *boxes, const u
         __syncthreads();
     }
     if (threadIdx.x < 6 && out_bounds) out_bounds[(long long)bid * 6 + threadIdx.x] = sb[threadIdx.x][0];
+    if (LEAF) {
+        // The block's node records in the order of their indices, a wave's 64 as one contiguous run (as 15 words a
+        // lane, 60 bytes apart: 307 us for the pass over 4,000,003 shapes, so: 262).  An odd index is the last leaf of a left child: its
+        // trailing ones give the node's level; an even one is the first leaf of any other node.  Nodes
+        // that reach out of the block, at most its first and last index, belong to a later pass.
+        const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+        unsigned *st = stage[wv];
+#pragma unroll 1
+        for (int q = 0; q < kPer; q++) {
+            const long long first = item_base + (threadIdx.x - lane) + q * 256;
+            const int i = (int)(first + lane);
+            bool mine = first + lane <= (long long)n - 2;
+            if (mine) {
+                long long lo, hi;
+                if (i & 1) {
+                    const int k = __builtin_ctz(~(unsigned)i);
+                    lo = (long long)i + 1 - (1ll << k);
+                    hi = i;
+                } else {
+                    lo = i;
+                    hi = i ? (long long)i + (1ll << __builtin_ctz((unsigned)i)) - 1 : (long long)n - 1;
+                    if (hi > n - 1) hi = n - 1;
+                }
+                mine = lo >= item_base && hi < item_base + kRefitItems;
+                if (mine) {
+                    const int s = 32 - __clz((int)(hi - lo));   // ceil(log2(len)), len >= 2
+                    const long long mid = lo + (1ll << (s - 1));
+                    const int m0 = (int)(mid - item_base);
+                    Bound M;
+                    M.min_x = sb[0][m0]; M.max_x = sb[1][m0]; M.min_y = sb[2][m0];
+                    M.max_y = sb[3][m0]; M.min_z = sb[4][m0]; M.max_z = sb[5][m0];
+                    BVHNodeGPU rec;
+                    write_node_record(&rec, (int)lo, (int)hi, (int)mid, index_tree_parent(lo, s, n), M);
+                    const unsigned *rw = reinterpret_cast<const unsigned *>(&rec);
+#pragma unroll
+                    for (int f = 0; f < 15; f++) st[lane * 15 + f] = rw[f];
+                }
+            }
+            const unsigned long long have = __ballot(mine);
+            __builtin_amdgcn_wave_barrier();
+            if (have)
+                wave_store_words(st, reinterpret_cast<unsigned *>(btn + first), 15 * (__ffsll((long long)have) - 1),
+                                 15 * (64 - __builtin_clzll(have)), lane);
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
 }
 
 // -------------------------------------------------------------------------------------------
