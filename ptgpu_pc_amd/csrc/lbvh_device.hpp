@@ -718,9 +718,9 @@ __device__ __forceinline__ void refit_levels_body(const ShapeBox *boxes, const u
     if (threadIdx.x < 6 && out_bounds) out_bounds[(long long)bid * 6 + threadIdx.x] = sb[threadIdx.x][0];
     if (LEAF) {
         // The block's node records in the order of their indices, a wave's 64 as one contiguous run (as 15 words a
-        // lane, 60 bytes apart: 307 us for the pass over 4,000,003 shapes, so: 262).  An odd index is the last leaf of a left child: its
-        // trailing ones give the node's level; an even one is the first leaf of any other node.  Nodes
-        // that reach out of the block, at most its first and last index, belong to a later pass.
+        // lane, 60 bytes apart: 307 us for the pass over 4,000,003 shapes, so: 262).  An odd index is the last
+        // leaf of a left child: its trailing ones give the node's level; an even one is the first leaf of any other
+        // node.  Nodes that reach out of the block, at most its first and last index, belong to a later pass.
         const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
         unsigned *st = stage[wv];
 #pragma unroll 1

@@ -367,8 +367,8 @@ __global__ __launch_bounds__(256) void k_render(RenderParams P) {
 //     shadow ray starts the next query between passes;
 //   * divisions and roots are correctly rounded in three and five instructions (rcp_exact, sqrt_exact);
 //   * a wave with few queries left shares them among its lanes (half_sparse).
-// Times before and after, one frame: 512x512x8 spp of the 65,538-shape soup 7.6 -> 5.3 ms; 1024x768x16 of the
-// 327,692-shape mesh 36.2 -> 18.3 ms; 640x480x4 of a 20,492-shape SAH KD tree 5.1 -> 3.2 ms; 97x61x1 of a
+// Times before and after, one frame: 512x512x8 spp of the 65,538-shape soup 7.75 -> 5.2 ms; 1024x768x16 of the
+// 327,692-shape mesh 36.0 -> 17.6 ms; 640x480x4 of a 20,492-shape SAH KD tree 5.0 -> 2.7 ms; 97x61x1 of a
 // 332-shape mesh 0.57 -> 0.25 ms.
 enum : int {
     kNeed = 0,    // wants a pixel
