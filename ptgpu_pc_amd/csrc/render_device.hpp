@@ -202,10 +202,12 @@ PT_HD float slab(float lx, float ly, float lz, float hx, float hy, float hz, f3 
 //
 // The reciprocal is held to +-2^100: a larger one (a ray in an axis plane) would make bound * (1/d) + (-o/d)
 // infinity minus infinity.  Being a power of two it makes both terms exact, so a box is hit on that axis if the
-// origin lies within its bounds, as with slab(), where the bound that the origin lies on does not count (zero
-// times infinity); the offsets' step, at least 2^-40 of the coordinate's unit, keeps that one from counting here,
-// also at zero.  Where a distance is NaN all the same (an origin beyond 1e8 on such a ray) the test ignores
-// that axis's bound, which only accepts more boxes.
+// origin lies within its bounds; the offsets' step, at least 2^-32 of the coordinate's unit, keeps the bound that
+// the origin lies on from counting, also at zero.  The held reciprocal understates how long such a ray stays between
+// the bounds: along an axis it drifts less than t / 2^100, which up to 2^66 (no closest hit lies farther than
+// 1e20) is 2^-34, within that step: so a direction of any length meets the boxes it passes.  (With a step of 2^-40 one
+// of length 2^-63 lost the triangles above a plane at zero.)  Where a distance is NaN all the same (an origin beyond
+// 1e8 on such a ray) the test ignores that axis's bound, which only accepts more boxes.
 struct RaySlab {
     unsigned rx, ry, rz;
     f3 inv, on, of;
@@ -218,7 +220,7 @@ __device__ __forceinline__ RaySlab ray_slab(f3 o, f3 d) {
         inv = fminf(fmaxf(__builtin_amdgcn_rcpf(dx), -kMost), kMost);
         rot = inv >= 0.f ? 0u : 16u;
         const float p = -ox * inv;
-        const float s = fmaxf(fabsf(p) * 0x1.8p-24f, fabsf(inv) * 0x1p-40f);
+        const float s = fmaxf(fabsf(p) * 0x1.8p-24f, fabsf(inv) * 0x1p-32f);
         on = p - s;
         of = p + s;
     };
