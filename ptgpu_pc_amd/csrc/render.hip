@@ -651,6 +651,7 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
                 if (done) st = qany ? kADone : kCDone;
             }
         }
+        if (HALF) half_finish_overflowed<STACK, STATS>(Q, T, t_root, stk, &st_prims);
         // ---- finished shadow rays: the bounce's other shadow ray, or its next segment, both drawn when the
         // bounce was shaded, start here without a shading pass ----
         if (st == kADone) {
@@ -1012,6 +1013,7 @@ __global__ __launch_bounds__(256, STACK <= 36 ? 4 : 2) void k_trace_half(DevAcce
     W.node = W.leaf = W.sp = 0;
     W.any = any != 0;
     for (;;) {
+        half_finish_overflowed<STACK, false>(W, T, A.root, stk, nullptr);
         // results of the finished queries, then the next rays
         if (st == kDone) {
             if (any) {

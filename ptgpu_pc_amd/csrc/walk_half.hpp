@@ -13,7 +13,7 @@ namespace ptgpu {
 
 // The short traversal-stack class of the binary16 walk: 36 entries per lane, so a workgroup's stack
 // takes 36 KB of LDS and four workgroups fit on a CU (three with the 48-entry class).  A walk that
-// would push past it ends with sp = kOverflowSp and is finished against every primitive.
+// would push past it ends with sp = kOverflowSp and is walked again (half_finish_overflowed).
 constexpr int kStackShort = 36;
 constexpr int kStackTiny = 8;   // a test class: nearly every walk outgrows it (tuning short_stack 2)
 constexpr int kOverflowSp = 1 << 20;
@@ -23,8 +23,10 @@ constexpr bool kIsShort = STACK == kStackShort || STACK == kStackTiny;
 
 // Entries of a `stack`-entry stack above the need of a depth-first walk of the tree (three pushes per two
 // levels); half_sparse may use them.  0 where the tree's height is not known before the launch.  The
-// short classes hold less than that need, and their walks stay far below it (no push past 36 entries
-// was counted over a whole 512x512 frame of the 65,538-shape soup): a margin of 16 entries is kept.
+// short classes hold less than that need, and walks that take one entry at a time stay far below it; those of
+// half_sparse reach it where many boxes overlap, and are then walked again.  A margin of 16 entries is
+// kept: with more, fewer walks start again, but all take more steps (97x61x1 spp of the 65,538-shape soup: 0.31 ms, with
+// a margin of 24 0.44, with 32 0.56; of 65,536 triangles with vertices within 0.2 of their centres 1.5, 1.6 and 1.7).
 __host__ __device__ inline int half_slack(int stack, const DevAccel &A) {
     if (A.height_check) return 0;
     if (stack == kStackShort || stack == kStackTiny) return stack - 16;
@@ -102,24 +104,32 @@ __device__ __forceinline__ bool half_refill_waiting(HalfWalk &W, const int *stk)
     return n == 0 && !waits;
 }
 
-// A walk that outgrew the short stack is finished against every primitive, from the best hit found
-// so far.  The closest hit is the least (t, then the higher id) whatever the order of the tests,
-// and an occluder ends an any-hit query, so the result is the walk's.
-template <bool STATS>
-__device__ void half_finish_overflowed(HalfWalk &W, const HalfTree &T, unsigned *st_prims) {
-    for (int q = 0; q < T.nprims && !(W.any && W.bid >= 0); q++) {
-        const Prim *tq = from_gmem(T.prims) + q;
-        int id;
-        bool last;
-        const float t = prim_isect_vals(tq->p0, tq->p1, tq->p2, W.o, W.d, &id, &last);
-        if (STATS) (*st_prims)++;
-        if (W.any) {
-            if (t != 0.f && t < W.tb && id != T.skip) W.bid = 1;
-        } else if (t != 0.f && (t < W.tb || (t == W.tb && id > W.bid))) {
-            W.tb = t;
-            W.bid = id;
-        }
+// The children of a node that the ray enters go on the stack without a branch: child k's place above the old top is
+// the number of children it is nearer than, so the nearest hit ends on top, and a miss (key 0 and its slot) ends
+// above every hit, past the new top.  Returns the new top; kOverflowSp where the short stack cannot hold them.
+template <int STACK>
+__device__ __forceinline__ int half_push(const uint4 &q0, const uint4 &q1, const uint4 &q2, const uint4 &q3,
+                                         const RaySlab &rs, float tb, int *stk, int sp) {
+    const unsigned t0 = slab_hn(q0.x, q0.y, q0.z, rs, tb), t1 = slab_hn(q1.x, q1.y, q1.z, rs, tb);
+    const unsigned t2 = slab_hn(q2.x, q2.y, q2.z, rs, tb), t3 = slab_hn(q3.x, q3.y, q3.z, rs, tb);
+    const unsigned k0 = t0 & ~3u, k1 = (t1 & ~3u) | 1u, k2 = (t2 & ~3u) | 2u, k3 = t3 | 3u;
+    const int c01 = k0 < k1, c02 = k0 < k2, c03 = k0 < k3, c12 = k1 < k2, c13 = k1 < k3, c23 = k2 < k3;
+    const int p0 = c01 + c02 + c03, p1 = 1 - c01 + c12 + c13, p2 = 2 - c02 - c12 + c23, p3 = 3 - c03 - c13 - c23;
+    const int nh = (t0 != 0u) + (t1 != 0u) + (t2 != 0u) + (t3 != 0u);
+    int *const top = stk + sp * 256;   // the other classes hold every walk of their trees
+    if (kIsShort<STACK> && sp > STACK - 4) {   // no room for the misses' places
+        if (sp + nh > STACK) return kOverflowSp;
+        if (p0 < nh) top[p0 * 256] = (int)q0.w;
+        if (p1 < nh) top[p1 * 256] = (int)q1.w;
+        if (p2 < nh) top[p2 * 256] = (int)q2.w;
+        if (p3 < nh) top[p3 * 256] = (int)q3.w;
+    } else {
+        top[p0 * 256] = (int)q0.w;
+        top[p1 * 256] = (int)q1.w;
+        top[p2 * 256] = (int)q2.w;
+        top[p3 * 256] = (int)q3.w;
     }
+    return sp + nh;
 }
 
 // One step of one lane: the current node (if any) and the pending leaf run (if any), loaded together: a
@@ -186,32 +196,53 @@ __device__ __forceinline__ bool half_step(HalfWalk &W, const HalfTree &T, int *s
         }
     }
     if (!done && W.node >= 0) {
-        // The four children go on the stack without a branch: child k's place above the old top is the
-        // number of children it is nearer than, so the nearest hit ends on top, and a miss (key 0 and its
-        // slot) ends above every hit, past the new top.
-        const unsigned t0 = slab_hn(q0.x, q0.y, q0.z, W.rs, W.tb), t1 = slab_hn(q1.x, q1.y, q1.z, W.rs, W.tb);
-        const unsigned t2 = slab_hn(q2.x, q2.y, q2.z, W.rs, W.tb), t3 = slab_hn(q3.x, q3.y, q3.z, W.rs, W.tb);
         if (STATS)
             *st_nodes += (q0.x != kEmptyHalf) + (q1.x != kEmptyHalf) + (q2.x != kEmptyHalf) + (q3.x != kEmptyHalf);
-        const unsigned k0 = t0 & ~3u, k1 = (t1 & ~3u) | 1u, k2 = (t2 & ~3u) | 2u, k3 = t3 | 3u;
-        const int c01 = k0 < k1, c02 = k0 < k2, c03 = k0 < k3, c12 = k1 < k2, c13 = k1 < k3, c23 = k2 < k3;
-        const int p0 = c01 + c02 + c03, p1 = 1 - c01 + c12 + c13, p2 = 2 - c02 - c12 + c23, p3 = 3 - c03 - c13 - c23;
-        const int nh = (t0 != 0u) + (t1 != 0u) + (t2 != 0u) + (t3 != 0u);
-        if (kShort && W.sp > STACK - 4) {   // finished against every primitive
-            W.sp = kOverflowSp;
-            done = true;
-        } else {
-            int *const top = stk + W.sp * 256;   // the other classes hold every walk of their trees
-            top[p0 * 256] = (int)q0.w;
-            top[p1 * 256] = (int)q1.w;
-            top[p2 * 256] = (int)q2.w;
-            top[p3 * 256] = (int)q3.w;
-            W.sp += nh;
-        }
+        W.sp = half_push<STACK>(q0, q1, q2, q3, W.rs, W.tb, stk, W.sp);
+        done = kShort && W.sp == kOverflowSp;
     }
     if (!done) done = test ? half_refill(W, stk) : half_refill_waiting(W, stk);
-    if (kShort && W.sp == kOverflowSp) half_finish_overflowed<STATS>(W, T, st_prims);
     return done;
+}
+
+// Walks that outgrew the short stack start again at the root, one entry at a time and from the best hit found so far.
+// Where even that does not fit, the lane tests every primitive.  The closest hit is the least (t, then the higher id)
+// whatever the order of the tests, and an occluder ends an any-hit query, so the result is the walk's.  Only
+// half_sparse's walks outgrow the stack in practice, a few in a hundred thousand where many boxes overlap: 97x61x1 spp of
+// 65,536 triangles with vertices within 0.2 of their centres, every primitive at once / the walk again: 28.3 / 1.5 ms.
+// Called between traversal phases, by the whole wave.
+template <int STACK, bool STATS>
+__device__ __forceinline__ void half_finish_overflowed(HalfWalk &W, const HalfTree &T, int root, int *stk, unsigned *st_prims) {
+    if (!kIsShort<STACK> || __ballot(W.sp == kOverflowSp) == 0ull || W.sp != kOverflowSp) return;
+    // true: the run ends here (an occluder found, or its last primitive)
+    auto test_prim = [&](int q) -> bool {
+        const Prim *tq = from_gmem(T.prims) + q;
+        int id;
+        bool last;
+        const float t = prim_isect_vals(tq->p0, tq->p1, tq->p2, W.o, W.d, &id, &last);
+        if (STATS) (*st_prims)++;
+        if (W.any) {
+            if (t != 0.f && t < W.tb && id != T.skip) { W.bid = 1; return true; }
+        } else if (t != 0.f && (t < W.tb || (t == W.tb && id > W.bid))) {
+            W.tb = t;
+            W.bid = id;
+        }
+        return last;
+    };
+    int sp = 1;
+    stk[0] = root;
+    while (sp > 0 && sp != kOverflowSp && !(W.any && W.bid >= 0)) {
+        const int ref = stk[--sp * 256];
+        if (ref < 0) {
+            for (int q = ~ref; !test_prim(q); q++) {}
+        } else {
+            const TNode4H *np = from_gmem(T.nodes) + ref;
+            sp = half_push<STACK>(np->c[0], np->c[1], np->c[2], np->c[3], W.rs, W.tb, stk, sp);
+        }
+    }
+    if (sp == kOverflowSp)
+        for (int q = 0; q < T.nprims && !(W.any && W.bid >= 0); q++) test_prim(q);
+    W.sp = 0;
 }
 
 // The sparse phase: a wave whose traversing lanes (`trav`) are 16 or fewer lends its idle lanes to the
@@ -228,8 +259,8 @@ __device__ __forceinline__ bool half_step(HalfWalk &W, const HalfTree &T, int *s
 //
 // Stack: popping m entries may push 4m.  `slack` is what the stack class leaves above a depth-first
 // walk's need: with sp + 3m within it, a walk that goes on one entry at a time still fits (m = 1 is
-// the depth-first walk itself).  The short classes have no such bound; their slack is a guess and a
-// walk that does not fit ends as overflowed.
+// the depth-first walk itself).  The short classes have no such bound, and a walk that does not fit ends
+// as overflowed.
 //
 // Called by the whole wave.  `ready`: lanes already waiting for shading; the phase ends when they and
 // the finished queries reach `regroup`, or all queries are finished.  Returns true on a lane whose own
@@ -387,8 +418,7 @@ __device__ __forceinline__ bool half_sparse(HalfWalk &W, const HalfTree &T, int 
         W.tb = b_tb;
         done = b_end;
         W.rs = ray_slab(W.o, W.d);   // again, so that the phase does not hold it beside its group's
-        if (kShort && W.sp == kOverflowSp) half_finish_overflowed<STATS>(W, T, st_prims);
-        else if (!done) done = half_refill(W, my_stk);
+        if (!done) done = half_refill(W, my_stk);
     }
     return done;
 }
