@@ -1013,9 +1013,9 @@ __global__ __launch_bounds__(256, STACK <= 36 ? 4 : 2) void k_trace_half(DevAcce
     W.node = W.leaf = W.sp = 0;
     W.any = any != 0;
     for (;;) {
-        half_finish_overflowed<STACK, false>(W, T, A.root, stk, nullptr);
         // results of the finished queries, then the next rays
         if (st == kDone) {
+            half_finish_overflowed<STACK, false>(W, T, A.root, stk, nullptr);
             if (any) {
                 hitout[cur] = W.bid >= 0 ? 1 : 0;
             } else {

@@ -116,19 +116,12 @@ __device__ __forceinline__ int half_push(const uint4 &q0, const uint4 &q1, const
     const int c01 = k0 < k1, c02 = k0 < k2, c03 = k0 < k3, c12 = k1 < k2, c13 = k1 < k3, c23 = k2 < k3;
     const int p0 = c01 + c02 + c03, p1 = 1 - c01 + c12 + c13, p2 = 2 - c02 - c12 + c23, p3 = 3 - c03 - c13 - c23;
     const int nh = (t0 != 0u) + (t1 != 0u) + (t2 != 0u) + (t3 != 0u);
-    int *const top = stk + sp * 256;   // the other classes hold every walk of their trees
-    if (kIsShort<STACK> && sp > STACK - 4) {   // no room for the misses' places
-        if (sp + nh > STACK) return kOverflowSp;
-        if (p0 < nh) top[p0 * 256] = (int)q0.w;
-        if (p1 < nh) top[p1 * 256] = (int)q1.w;
-        if (p2 < nh) top[p2 * 256] = (int)q2.w;
-        if (p3 < nh) top[p3 * 256] = (int)q3.w;
-    } else {
-        top[p0 * 256] = (int)q0.w;
-        top[p1 * 256] = (int)q1.w;
-        top[p2 * 256] = (int)q2.w;
-        top[p3 * 256] = (int)q3.w;
-    }
+    if (kIsShort<STACK> && sp > STACK - 4) return kOverflowSp;   // (the other classes hold every walk of their trees)
+    int *const top = stk + sp * 256;
+    top[p0 * 256] = (int)q0.w;
+    top[p1 * 256] = (int)q1.w;
+    top[p2 * 256] = (int)q2.w;
+    top[p3 * 256] = (int)q3.w;
     return sp + nh;
 }
 
@@ -210,10 +203,10 @@ __device__ __forceinline__ bool half_step(HalfWalk &W, const HalfTree &T, int *s
 // whatever the order of the tests, and an occluder ends an any-hit query, so the result is the walk's.  Only
 // half_sparse's walks outgrow the stack in practice, a few in a hundred thousand where many boxes overlap: 97x61x1 spp of
 // 65,536 triangles with vertices within 0.2 of their centres, every primitive at once / the walk again: 28.3 / 1.5 ms.
-// Called between traversal phases, by the whole wave.
+// Called between traversal phases.
 template <int STACK, bool STATS>
 __device__ __forceinline__ void half_finish_overflowed(HalfWalk &W, const HalfTree &T, int root, int *stk, unsigned *st_prims) {
-    if (!kIsShort<STACK> || __ballot(W.sp == kOverflowSp) == 0ull || W.sp != kOverflowSp) return;
+    if (!kIsShort<STACK> || W.sp != kOverflowSp) return;
     // true: the run ends here (an occluder found, or its last primitive)
     auto test_prim = [&](int q) -> bool {
         const Prim *tq = from_gmem(T.prims) + q;
