@@ -40,6 +40,12 @@ struct RenderJob {
     unsigned *pixels;
 };
 
+// A single-frame launch's shape (launch_shape): workgroups that work, lanes of a wave that take pixels; the others help
+// in the sparse phase.
+struct LaunchShape {
+    int blocks, lanes;
+};
+
 struct RenderParams {
     DevAccel acc;
     Vec *colors;
@@ -63,8 +69,7 @@ struct RenderParams {
     const int2 *tiles;            // tiled launches (RadianceBoxGPU): tile origins; NULL renders the whole frame
     int tile_w, tile_h;
     int slack;                    // binary16 walk: stack entries above a depth-first walk's need (half_sparse)
-    int blocks_open;              // workgroups that stay when the camera is outside the scene's box
-    int lanes;                    // lanes of a wave that take pixels; the others help in the sparse phase
+    LaunchShape inside, outside;  // for a camera inside and outside the scene's box
     int depth_cap;                // deepest tree the launch's stack holds (checked when acc.height_check is set)
     const float *pack_tab;        // to_int_tab's table
     unsigned *status;             // the context's check words: [0] flags, [1] deepest height seen
@@ -386,7 +391,10 @@ template <int STACK, bool STATS, bool WIDE, bool MULTI, bool HALF, bool WAIT = f
 __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && STACK <= 48 ? 3 : 1) void k_render_lanes(RenderParams P) {
     if (!MULTI && recorded_tree_unfit(P)) return;
     if (MULTI && P.status && recorded_jobs_unfit(P)) return;
-    if (HALF && !MULTI && (int)blockIdx.x >= P.blocks_open && camera_outside(P)) return;
+    LaunchShape shape = P.inside;
+    if (HALF && !MULTI && (P.outside.blocks != P.inside.blocks || P.outside.lanes != P.inside.lanes) && camera_outside(P))
+        shape = P.outside;
+    if (!MULTI && (int)blockIdx.x >= shape.blocks) return;
     __shared__ int s_stack[STACK * 256];
     int *stk = s_stack + threadIdx.x;
     static_assert(!kIsShort<STACK> || (WIDE && HALF), "the short stack class serves the binary16 walk");
@@ -447,8 +455,13 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
     T.skip = P.acc.nshapes - 1;
     int t_nnodes = P.acc.nnodes, t_root = P.acc.root, t_slack = P.slack;
 
-    int st = (int)__lane_id() < P.lanes ? kNeed : kIdle;
+    int st = (int)__lane_id() < shape.lanes ? kNeed : kIdle;
     bool drained = false;
+    // Each wave's first pixels follow from its number; the counter deals out the rest, if there are any.  A frame that
+    // is spread over 4,096 waves took 20 us of its 50 to 250 for their 8,192 turns at the counter.
+    const unsigned first_deal = (blockIdx.x * 4 + threadIdx.x / kWave) * (unsigned)shape.lanes;
+    const unsigned dealt = MULTI ? 0u : (unsigned)shape.blocks * 4u * (unsigned)shape.lanes;
+    unsigned deal = __builtin_amdgcn_readfirstlane((int)(MULTI ? ~0u : first_deal));
     int gid = 0, k = 0, depth = 0, li = 0;
     bool spec = true;
     unsigned s0 = 0, s1 = 0;
@@ -686,11 +699,16 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
         const unsigned long long need = __ballot(st == kNeed);
         if (need) {
             const unsigned cnt = (unsigned)__popcll(need);
-            const int leader = __ffsll((long long)need) - 1;
-            unsigned base = 0;
-            if ((int)__lane_id() == leader) base = atomicAdd(args->work_counter, cnt);
-            base = __shfl(base, leader, kWave);
-            if (base + cnt >= (unsigned)args->total) drained = true;
+            unsigned base = deal;
+            if (deal != ~0u) {
+                deal = ~0u;
+                drained = dealt >= (unsigned)args->total;
+            } else {
+                const int leader = __ffsll((long long)need) - 1;
+                if ((int)__lane_id() == leader) base = dealt + atomicAdd(args->work_counter, cnt);
+                base = __shfl(base, leader, kWave);
+                if (base + cnt >= (unsigned)args->total) drained = true;
+            }
             if (st == kNeed) {
                 const unsigned my = base + (unsigned)__popcll(need & lt);
                 if (my < (unsigned)args->total) {
@@ -1494,38 +1512,47 @@ static int stack_for(const DevAccel &acc, int least) {
     return -1;
 }
 
-// Workgroups of a single-frame launch and the wave's share of pixels, for `total` work items.
+// Workgroups of a single-frame launch and the wave's share of pixels, for `total` work items.  Returns the grid.
 //
 // Set by the caller ("blocks_per_cu"): that many persistent workgroups per CU, never more than needed.
-// By default, for the binary16 walk:
-//   * Up to 8 pixels per wave slot (16 slots per CU: 32,768 pixels on 256 CUs) only the first 1, 2, 4 or 8
-//     lanes of a wave take pixels and the others help their queries (half_sparse): such a frame ends with
-//     its longest path whatever else runs, and shared queries take fewer steps.  97x61x1 spp of the
-//     332-shape mesh: 380 us with 64 pixels a wave, 230 us with two; 200x150 of the 5,132-shape mesh:
-//     428 us, with eight 397 us; at 320x240 sharing loses (510 us, with eight 855 us), so the line lies there.
+// By default, for the binary16 walk (the kernel looks where the camera is: it is device memory):
+//   * In a small frame only the first 1, 2, 4 or 8 lanes of a wave take pixels and the others help their queries
+//     (half_sparse): such a frame ends with its longest path whatever else runs, and shared queries take fewer
+//     steps, each of which does more work.  (Times below in us: one frame alone, three in flight on a stream each.)
+//     From outside much of a frame is background, so it is spread over all the waves that four workgroups per CU
+//     hold, up to 8 pixels each (16 waves per CU: 32,768 pixels on 256 CUs): 180x180 of the 65,538-shape soup, 64
+//     pixels a wave / eight: 831, 311 / 466, 213; at 256x256 eight halve the rate of a 20,482-shape mesh in flight.
+//     Inside, every path is long and frames in flight need the room: up to three workgroups per CU for one and two
+//     pixels a wave, two for four and eight, where deep trees (many steps to save) may have three.  97x61 of the
+//     332-shape mesh, 64 / two: 399, 140 / 236, 118; 128x128 of the 5,132-shape mesh, 64 / eight on two per CU / four
+//     on four per CU: 443, 161 / 411, 185 / 428, 296; 180x180 of it, 64 / eight on four per CU: 452, 167 / 479, 353;
+//     150x150 of the 20,492-shape mesh, 64 / eight: 487, 184 / 367, 201; 100x100, eight / four: 329, 126 / 306, 136.
 //   * Larger frames get four workgroups per CU (what the registers and the stack leave room for), but a
-//     frame of fewer than two pixels a lane whose camera is outside the scene's box keeps two (the kernel
-//     decides: the camera is device memory).  Seen from inside, every pixel's path is long and more waves
+//     frame of fewer than two pixels a lane whose camera is outside the scene's box keeps two.
+//     Seen from inside, every pixel's path is long and more waves
 //     keep the SIMDs busy: 1024x768x16 of the 327,692-shape mesh, two / four a CU: 28.8 / 18.5 ms.  From
 //     outside, much of the frame is background and the few long paths decide: on two a CU they run with
 //     fewer neighbours and lanes whose pixel was background take another (512x512x8 of the 65,538-shape
 //     soup, two / four: 5.1 / 5.7 ms; at 1024x1024x4, 6.9 / 5.0 ms).
 static int launch_shape(const ptgpu_ctx *ctx, int total, bool half, RenderParams &P) {
     const int cus = ctx->cu_count;
-    int per_cu = ctx->blocks_per_cu;
-    if (ctx->blocks_auto && half) {
-        per_cu = 4;
-        if (ctx->quad > 0 && !P.trav_stats) {   // (counting launches keep one walk order for every shape)
-            int lanes = 1;
-            while (lanes < kWave && total > lanes * 16 * cus) lanes *= 2;
-            P.lanes = lanes <= 8 ? lanes : kWave;
-        }
-        if (total < 2 * 4 * 256 * cus) P.blocks_open = 2 * cus;
+    const bool deep = stack_for_wide(P.acc, 0) != 32;
+    auto shape = [&](int lanes, int per_cu) {
+        const int all = cus * per_cu, need = (total + 4 * lanes - 1) / (4 * lanes);
+        return LaunchShape{need < 1 ? 1 : need < all ? need : all, lanes};
+    };
+    if (!ctx->blocks_auto || !half) {
+        P.inside = P.outside = shape(kWave, ctx->blocks_per_cu);
+        return P.inside.blocks;
     }
-    int blocks = cus * per_cu;
-    const int need = (total + 4 * P.lanes - 1) / (4 * P.lanes);
-    if (blocks > need) blocks = need;
-    return blocks < 1 ? 1 : blocks;
+    int in = kWave, out = kWave;
+    if (ctx->quad > 0 && !P.trav_stats) {   // (counting launches keep one walk order for every shape)
+        in = total <= 12 * cus ? 1 : total <= 24 * cus ? 2 : total <= (deep ? 48 : 32) * cus ? 4 : total <= (deep ? 96 : 64) * cus ? 8 : kWave;
+        out = total <= 16 * cus ? 1 : total <= 32 * cus ? 2 : total <= 64 * cus ? 4 : total <= 128 * cus ? 8 : kWave;
+    }
+    P.inside = shape(in, 4);
+    P.outside = shape(out, out == kWave && total < 2 * 4 * 256 * cus ? 2 : 4);
+    return std::max(P.inside.blocks, P.outside.blocks);
 }
 
 int launch_render(ptgpu_ctx *ctx, const DevAccel &acc, const RenderLaunch &L) {
@@ -1577,8 +1604,6 @@ int launch_render(ptgpu_ctx *ctx, const DevAccel &acc, const RenderLaunch &L) {
     P.tile_w = L.tile_w;
     P.tile_h = L.tile_h;
     P.slack = 0;
-    P.lanes = kWave;
-    P.blocks_open = 0x7fffffff;
     P.depth_cap = binary_depth_cap(st);
     P.status = nullptr;
     if (acc.height_check) {
@@ -2258,8 +2283,7 @@ int launch_batch(ptgpu_ctx *ctx, BatchChannel &ch, const ptgpu_render_job *jobs,
         P.job_begin = reinterpret_cast<const unsigned *>(static_cast<char *>(d_table) + K.bo);
         P.njobs = (int)K.jobs.size();
         P.slack = 0;
-        P.lanes = kWave;
-    P.blocks_open = 0x7fffffff;
+        P.inside.lanes = kWave;
         P.depth_cap = wide_depth_cap(K.st);
         P.status = K.checks ? ctx->rec_status.as<unsigned>() : nullptr;
         const long long all = (long long)ctx->cu_count * ctx->batch_blocks_per_cu;
