@@ -216,7 +216,7 @@ __global__ __launch_bounds__(256) void k_refit_levels(const ShapeBox *boxes, con
 }
 
 template <bool LEAVES>
-__global__ __launch_bounds__(kWave) void k_mtree(int n, const unsigned *keys, const BVHNodeGPU *btl, const MItem *in,
+__global__ __launch_bounds__(LEAVES ? kWave : kMThreads) void k_mtree(int n, const unsigned *keys, const BVHNodeGPU *btl, const MItem *in,
                                                  const int *in_cnt, int lists_in, MItem *out, int *out_cnt,
                                                  TNode *tnodes, unsigned *root_height, unsigned *err) {
     mtree_body<LEAVES>(n, keys, btl, in, in_cnt, lists_in, out, out_cnt, tnodes, root_height, err, blockIdx.x);
@@ -356,7 +356,7 @@ static int clbvh_traversal_morton(ptgpu_clbvh *h) {
         MItem *out = k + 1 < ms.levels ? ms.items[k & 1] : nullptr;
         const MItem *in = k > 0 ? ms.items[(k - 1) & 1] : nullptr;
         const int *in_cnt = k > 0 ? ms.counts[(k - 1) & 1] : nullptr;
-        const dim3 grid((unsigned)ms.lists[k]), block(kWave);
+        const dim3 grid((unsigned)ms.lists[k]), block(k == 0 ? kWave : kMThreads);
         if (k == 0)
             hipLaunchKernelGGL(k_mtree<true>, grid, block, 0, st, n, h->keysA.as<unsigned>(), h->btl.as<BVHNodeGPU>(), in,
                                in_cnt, 0, out, ms.counts[0], h->tnodes.as<TNode>(), ctr + 11, ctr + 9);

@@ -137,7 +137,7 @@ __global__ __launch_bounds__(256) void kb_refit(const BuildSeg *g, const int *st
 
 // Level k of every scene's Morton-keyed tree.
 template <bool LEAVES>
-__global__ __launch_bounds__(kWave) void kb_mtree(const BuildSeg *g, const int *starts, int ns, int k) {
+__global__ __launch_bounds__(LEAVES ? kWave : kMThreads) void kb_mtree(const BuildSeg *g, const int *starts, int ns, int k) {
     const int s = seg_find(starts, ns, blockIdx.x);
     const BuildSeg &S = g[s];
     MItem *out = k + 1 < S.ms.levels ? S.ms.items[k & 1] : nullptr;
@@ -307,7 +307,7 @@ int build_batch(ptgpu_ctx *ctx, ptgpu_clbvh *const *hs, int ns) {
     }
     PT_BATCH_LAUNCH(kb_mtree<true>, kStMtree, kWave, 0);
     for (int k = 1; k < kMMaxLevels; k++) {
-        PT_BATCH_LAUNCH(kb_mtree<false>, kStMtree + k, kWave, k);
+        PT_BATCH_LAUNCH(kb_mtree<false>, kStMtree + k, kMThreads, k);
     }
 #undef PT_BATCH_LAUNCH
     if (recording) {

@@ -786,7 +786,10 @@ __device__ __forceinline__ int delta_key(const unsigned *keys, int i, int j, int
 // is a left child, its first leaf otherwise.  No topology pass, parent links or counters in memory, and a
 // node's children, range and side are known from the items alone.
 //
-// One wave works a list: 128 leaves, or the leftovers of kMFan lists.  Its lanes hold one item each, and a
+// One wave works a list: 128 leaves, or the leftovers of kMFan lists (which the other waves of its workgroup help to
+// load: a workgroup of a single wave with more than 17 KB of LDS was not placed beside a render's workgroups at all,
+// wherever they left room, and a build on another stream ended with the render; so a 65,538-shape build beside one of two
+// workgroups per CU takes 0.27 ms, not 2 to 6).  Its lanes hold one item each, and a
 // lane whose item waits takes the next one, so the wave's steps stay full until its items run out; one
 // thread per leaf climbing its parents left most lanes of each wave idle after two steps, and read the
 // topology from memory.  What bounds it: the step's instructions and its LDS round trips.  4,000,003 shapes:
@@ -799,8 +802,10 @@ __device__ __forceinline__ int delta_key(const unsigned *keys, int i, int j, int
 // surplus is dropped and the build's error word set.
 constexpr int kMChunk = 128;      // leaves per list of the first level
 constexpr int kMFan = 16;         // lists per list of the next level
+static_assert((kMFan & (kMFan - 1)) == 0, "an item's list is found by halving");
+constexpr int kMThreads = 256;    // of an upper level's workgroups
 constexpr int kMItems = 128;      // room for a list's leftovers (at most 125)
-constexpr int kMMaxLevels = 8;    // lists of 2^30 leaves: 2^21, then a sixteenth at each level
+constexpr int kMMaxLevels = 8;    // lists of 2^30 leaves: 2^23, then a sixteenth at each level
 struct alignas(16) MItem {
     float4 q0;   // bound: min_x, max_x, min_y, max_y
     float2 q1;   // min_z, max_z
@@ -828,7 +833,8 @@ __device__ __forceinline__ void mtree_body(int n, const unsigned *keys, const BV
                                            unsigned *root_height, unsigned *err, int bid) {
     __shared__ MTreeList<LEAVES> S;
     constexpr int kCap = MTreeList<LEAVES>::kCap;
-    const int lane = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    constexpr int kThreads = LEAVES ? kWave : kMThreads;
     const unsigned long long lt = lanemask_lt();
     const int base = bid * kMChunk;
     int count;
@@ -864,7 +870,7 @@ __device__ __forceinline__ void mtree_body(int n, const unsigned *keys, const BV
         __syncthreads();
         count = S.offs[kMFan];
 #pragma unroll 4
-        for (int i = lane; i < count; i += kWave) {
+        for (int i = tid; i < count; i += kThreads) {
             int q = 0;
             for (int x = kMFan >> 1; x > 0; x >>= 1)
                 if (S.offs[q + x] <= i) q += x;
@@ -874,16 +880,17 @@ __device__ __forceinline__ void mtree_body(int n, const unsigned *keys, const BV
             S.d[i] = (unsigned char)(m.dh & 0xff);
             S.h[i] = (unsigned char)(m.dh >> 8);
         }
-        if (lane == 0) {
+        if (tid == 0) {
             const bool more = l0 + kMFan < lists_in;
             const MItem *nx = in + (size_t)(l0 + kMFan) * kMItems;
             S.first[count] = more ? nx->first : n;
             S.d[count] = (unsigned char)(more ? nx->dh & 0xff : 0);
         }
     }
-    for (int s = lane; s <= count; s += kWave) S.tag[s] = 0u;
-    for (int s = lane; s < (kCap + 31) / 32; s += kWave) S.starts[s] = 0u;
+    for (int s = tid; s <= count; s += kThreads) S.tag[s] = 0u;
+    for (int s = tid; s < (kCap + 31) / 32; s += kThreads) S.starts[s] = 0u;
     __syncthreads();
+    if (tid >= kWave) return;   // one wave from here on: no barriers
     auto first_leaf = [&](int item) { return LEAVES ? base + item : S.first[item]; };
 
     bool on = false;
@@ -956,13 +963,13 @@ __device__ __forceinline__ void mtree_body(int n, const unsigned *keys, const BV
     if (!out) return;
     // the items that still wait, in leaf order
     auto start_of = [&](int s, unsigned t) { return t & 0x40000000u ? (int)(t & 0xffffu) : s; };
-    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup", "local");
     for (int s = lane; s <= count; s += kWave) {
         const unsigned t = S.tag[s];
         const int a0 = start_of(s, t);
         if (t && a0 < count) atomicOr(&S.starts[a0 >> 5], 1u << (a0 & 31));
     }
-    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup", "local");
     int total = 0;
     for (int w = 0; w < (kCap + 31) / 32; w++) total += __popc(S.starts[w]);
     if (lane == 0) {
