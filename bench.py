@@ -747,6 +747,13 @@ def record_batch_step(ctx, batch_h, jobs, frames, pix_plain, steps, warmup):
     return t_rec, same_rec
 
 
+def apply_tuning(ctx, tuning: dict, names) -> None:
+    """The named settings of an autotuner result (of this run or an earlier one), as far as it has them."""
+    for k in names:
+        if k in tuning:
+            ctx.set_tuning(k, 0 if k == "blocks_per_cu" and tuning.get("automatic") else int(tuning[k]))
+
+
 def frames_compare(tuning: dict | None, counts=(1, 2, 4), steps: int = 5, warmup: int = 1):
     """The C2 frame rendered one per launch against 2 and 4 frames of it per launch (ptgpu_render_batch).
     Every frame has its own tree, rebuilt each step (LBVH + the tuned treelet pass, one after another
@@ -762,9 +769,7 @@ def frames_compare(tuning: dict | None, counts=(1, 2, 4), steps: int = 5, warmup
     n = len(shapes)
     ctx = pt.Context(0)
     tun = tuning or {}
-    for k in ("blocks_per_cu", "regroup", "wide", "batch_blocks_per_cu", "batch_regroup"):
-        if k in tun:
-            ctx.set_tuning(k, int(tun[k]))
+    apply_tuning(ctx, tun, ("blocks_per_cu", "regroup", "wide", "batch_blocks_per_cu", "batch_regroup"))
     treelet = int(tun.get("treelet") or 0)
     fmax = max(counts)
     d_sh = [ctx.to_device(shapes) for _ in range(fmax)]
@@ -1184,8 +1189,7 @@ def main():
     if args.tuning:
         # settings from an earlier autotuned run (its line's "tuning" object), e.g. for profiled runs
         tuning = json.loads(Path(args.tuning).read_text())
-        for k in ("blocks_per_cu", "regroup", "wide"):
-            ctx.set_tuning(k, int(tuning[k]))
+        apply_tuning(ctx, tuning, ("blocks_per_cu", "regroup", "wide"))
         bvh.set_digit_bits(int(tuning["digit_bits"]))
         if not args.treelet and tuning["treelet"]:
             treelet, passes = int(tuning["treelet"]), 1
@@ -1205,6 +1209,8 @@ def main():
         ctx.set_tuning(k, v)
         if tuning is not None and k in tuning:
             tuning[k] = v
+            if k == "blocks_per_cu":
+                tuning["automatic"] = v == 0
 
     def step(ray_counter=None, trav_stats=None):
         ctx.record(0)
@@ -1253,11 +1259,8 @@ def main():
         for _ in range(nr - 1):
             r1 = pt.Context(0)
             r1.set_engine(args.engine)
-            for k in ("blocks_per_cu", "regroup", "wide"):
-                v = tuning[k] if tuning else {"blocks_per_cu": args.blocks_per_cu, "regroup": args.regroup,
-                                              "wide": args.wide}[k]
-                if v:
-                    r1.set_tuning(k, int(v))
+            given = {"blocks_per_cu": args.blocks_per_cu, "regroup": args.regroup, "wide": args.wide}
+            apply_tuning(r1, tuning or {k: v for k, v in given.items() if v is not None}, tuple(given))
             for k, v in extra:
                 r1.set_tuning(k, v)
             rctx.append(r1)

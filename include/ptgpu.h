@@ -118,8 +118,9 @@ int ptgpu_ctx_set_max_depth(ptgpu_ctx *ctx, int max_depth);
  * nodes).  All give the same bits. */
 int ptgpu_ctx_set_engine(ptgpu_ctx *ctx, int engine);
 /* Launch tuning, no effect on results: "regroup" (1..64, ready lanes that start a shading pass in
- * engine 3, default 24), "blocks_per_cu" (1..64, persistent workgroups per CU; until it is set, the
- * launch picks the workgroups and the pixels per wave from the frame's size), "wide"
+ * engine 3, default 24), "blocks_per_cu" (1..64, persistent workgroups per CU; 0, the default: the
+ * launch picks the workgroups and the pixels per wave from the frame's size, the tree's height and the
+ * camera's place), "wide"
  * (engine 3's node format: 0 binary, 1 four-wide fp32, 2 four-wide with binary16 boxes rounded
  * outward, half the bytes per node, where the tree's leaves allow it; default 2), "quad" (0..16,
  * with wide 2: when at most this many lanes of a wave are traversing, four or more lanes share each
@@ -133,6 +134,8 @@ int ptgpu_ctx_set_engine(ptgpu_ctx *ctx, int engine);
  * 0 off; 2 walks every binary16 tree on an 8-entry stack, a test setting);
  * "batch_regroup" and "batch_blocks_per_cu" (the same for ptgpu_render_batch, defaults 40 and 3). */
 int ptgpu_ctx_set_tuning(ptgpu_ctx *ctx, const char *name, int value);
+/* The setting of one of these names, as ptgpu_ctx_set_tuning takes it. */
+int ptgpu_ctx_get_tuning(ptgpu_ctx *ctx, const char *name, int *value);
 int ptgpu_malloc(ptgpu_ctx *ctx, size_t bytes, void **d_out);
 int ptgpu_free(ptgpu_ctx *ctx, void *d_ptr);
 int ptgpu_memcpy_h2d(ptgpu_ctx *ctx, void *d_dst, const void *h_src, size_t bytes); /* synchronous */
@@ -415,11 +418,13 @@ typedef struct {
     float render_ms;          /* fastest trial render with the chosen settings */
     float build_ms;           /* fastest rebuild (+ optimise) with the chosen settings */
 } ptgpu_tuning;
-/* Tunes the digit width, the single-frame launch shape (blocks per CU 1..4, regroup 8/16/32, node
- * format: wide 2, 1 or 0) and the treelet size (none, 5, 7; minimising rebuild + optimise +
+/* Tunes the digit width, the single-frame launch shape (the automatic one or blocks per CU 1..4, regroup
+ * 8/16/32, node format: wide 2, 1 or 0) and the treelet size (none, 5, 7; minimising rebuild + optimise +
  * frames_per_build renders).  frames_per_build 0: every frame rebuilds its tree on another stream
  * while the previous frame renders (two frames in flight), so the render time alone is minimised,
- * over treelet sizes whose rebuild + optimise takes at most 1/8 of the render.  Applies the result
+ * over treelet sizes whose rebuild + optimise takes at most 1/8 of the render.  Where the automatic shape is
+ * the fastest, ctx is left on it (ptgpu_ctx_get_tuning gives 0 for "blocks_per_cu", to be set by a caller
+ * who applies the result elsewhere) and out->blocks_per_cu is the most it may take.  Applies the result
  * to ctx and h and leaves h holding a tree built (and optimised) with it.  args: one ptgpu_render
  * call's arguments on h (h: >= 2 shapes). */
 int ptgpu_autotune(ptgpu_ctx *ctx, ptgpu_clbvh *h, const ptgpu_render_args *args, int frames_per_build,

@@ -183,6 +183,7 @@ struct BuildStaging {
     size_t pinned_bytes = 0;
     void release();
 };
+constexpr int kBlocksPerCu = 2;   // of renders that do not walk binary16 nodes, until "blocks_per_cu" is set
 }  // namespace ptgpu
 
 struct ptgpu_ctx {
@@ -196,8 +197,8 @@ struct ptgpu_ctx {
     int regroup = 24;   // per-lane-state megakernel: ready lanes that trigger a shading pass
     int quad = 16;      // per-lane-state megakernel, binary16 nodes: traversing lanes at or below which four lanes share a query
     int batch_regroup = 40;
-    int blocks_per_cu = 2;        // single-frame renders
-    bool blocks_auto = true;      // until "blocks_per_cu" is set, the launch picks (launch_shape, render.hip)
+    int blocks_per_cu = ptgpu::kBlocksPerCu;   // single-frame renders
+    bool blocks_auto = true;      // "blocks_per_cu" 0, the default: the launch picks (launch_shape, render.hip)
     int batch_blocks_per_cu = 3;  // batched renders: throughput-bound, more waves per SIMD
     int wide = 2;        // per-lane-state megakernel: 0 binary nodes, 1 four-wide, 2 four-wide binary16 (when they exist)
     int stack_min = 0;
@@ -260,6 +261,9 @@ int convert_bvh_ref(ptgpu_ctx *ctx, const Shape *d_shapes, int n, const BVHNodeG
 int convert_kd_ref(ptgpu_ctx *ctx, const Shape *d_shapes, int n, const KDNodeGPU *d_kng, int kngCnt,
                    const int *d_kn, int knCnt, DevBuf &nodes, DevBuf &prims, DevAccel *acc);
 // render / trace over a prepared structure
+// Whether the automatic launch shape spreads a frame of so many pixels over the tree (a few pixels a wave; the workgroups
+// end with their pixels).
+bool launch_spreads(const ptgpu_ctx *ctx, const DevAccel &acc, int pixels);
 struct RenderLaunch {
     Vec *colors;
     unsigned int *seeds;

@@ -194,9 +194,9 @@ int ptgpu_ctx_set_tuning(ptgpu_ctx *ctx, const char *name, int value) {
         PT_CHECK(value >= 1 && value <= 64, PTGPU_ERR_INVALID, "regroup %d not in [1, 64]", value);
         ctx->regroup = value;
     } else if (!strcmp(name, "blocks_per_cu")) {
-        PT_CHECK(value >= 1 && value <= 64, PTGPU_ERR_INVALID, "blocks_per_cu %d not in [1, 64]", value);
-        ctx->blocks_per_cu = value;
-        ctx->blocks_auto = false;
+        PT_CHECK(value >= 0 && value <= 64, PTGPU_ERR_INVALID, "blocks_per_cu %d not in [0, 64]", value);
+        ctx->blocks_auto = value == 0;
+        ctx->blocks_per_cu = value ? value : ptgpu::kBlocksPerCu;
     } else if (!strcmp(name, "batch_blocks_per_cu")) {
         PT_CHECK(value >= 1 && value <= 64, PTGPU_ERR_INVALID, "batch_blocks_per_cu %d not in [1, 64]", value);
         ctx->batch_blocks_per_cu = value;
@@ -219,6 +219,22 @@ int ptgpu_ctx_set_tuning(ptgpu_ctx *ctx, const char *name, int value) {
         PT_CHECK(false, PTGPU_ERR_INVALID, "unknown tuning parameter '%s'", name);
     }
     return PTGPU_OK;
+}
+
+int ptgpu_ctx_get_tuning(ptgpu_ctx *ctx, const char *name, int *value) {
+    PT_CHECK(ctx && name && value, PTGPU_ERR_INVALID, "null argument");
+    const struct {
+        const char *name;
+        int value;
+    } all[] = {{"regroup", ctx->regroup}, {"blocks_per_cu", ctx->blocks_auto ? 0 : ctx->blocks_per_cu},
+               {"batch_blocks_per_cu", ctx->batch_blocks_per_cu}, {"batch_regroup", ctx->batch_regroup},
+               {"quad", ctx->quad}, {"wide", ctx->wide}, {"short_stack", ctx->short_stack}, {"stack", ctx->stack_min}};
+    for (const auto &t : all)
+        if (!strcmp(name, t.name)) {
+            *value = t.value;
+            return PTGPU_OK;
+        }
+    PT_CHECK(false, PTGPU_ERR_INVALID, "unknown tuning parameter '%s'", name);
 }
 
 int ptgpu_ctx_set_max_depth(ptgpu_ctx *ctx, int max_depth) {

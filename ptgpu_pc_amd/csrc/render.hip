@@ -45,6 +45,9 @@ struct RenderJob {
 struct LaunchShape {
     int blocks, lanes;
 };
+struct LaunchShapes {
+    LaunchShape inside, outside;   // for a camera inside and outside the scene's box
+};
 
 struct RenderParams {
     DevAccel acc;
@@ -69,7 +72,7 @@ struct RenderParams {
     const int2 *tiles;            // tiled launches (RadianceBoxGPU): tile origins; NULL renders the whole frame
     int tile_w, tile_h;
     int slack;                    // binary16 walk: stack entries above a depth-first walk's need (half_sparse)
-    LaunchShape inside, outside;  // for a camera inside and outside the scene's box
+    LaunchShapes launch;
     int depth_cap;                // deepest tree the launch's stack holds (checked when acc.height_check is set)
     const float *pack_tab;        // to_int_tab's table
     unsigned *status;             // the context's check words: [0] flags, [1] deepest height seen
@@ -391,9 +394,11 @@ template <int STACK, bool STATS, bool WIDE, bool MULTI, bool HALF, bool WAIT = f
 __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && STACK <= 48 ? 3 : 1) void k_render_lanes(RenderParams P) {
     if (!MULTI && recorded_tree_unfit(P)) return;
     if (MULTI && P.status && recorded_jobs_unfit(P)) return;
-    LaunchShape shape = P.inside;
-    if (HALF && !MULTI && (P.outside.blocks != P.inside.blocks || P.outside.lanes != P.inside.lanes) && camera_outside(P))
-        shape = P.outside;
+    LaunchShape shape = P.launch.inside;
+    if (HALF && !MULTI &&
+        (P.launch.outside.blocks != P.launch.inside.blocks || P.launch.outside.lanes != P.launch.inside.lanes) &&
+        camera_outside(P))
+        shape = P.launch.outside;
     if (!MULTI && (int)blockIdx.x >= shape.blocks) return;
     __shared__ int s_stack[STACK * 256];
     int *stk = s_stack + threadIdx.x;
@@ -1512,7 +1517,7 @@ static int stack_for(const DevAccel &acc, int least) {
     return -1;
 }
 
-// Workgroups of a single-frame launch and the wave's share of pixels, for `total` work items.  Returns the grid.
+// Workgroups of a single-frame launch and the wave's share of pixels, for `total` work items.
 //
 // Set by the caller ("blocks_per_cu"): that many persistent workgroups per CU, never more than needed.
 // By default, for the binary16 walk (the kernel looks where the camera is: it is device memory):
@@ -1534,25 +1539,34 @@ static int stack_for(const DevAccel &acc, int least) {
 //     outside, much of the frame is background and the few long paths decide: on two a CU they run with
 //     fewer neighbours and lanes whose pixel was background take another (512x512x8 of the 65,538-shape
 //     soup, two / four: 5.1 / 5.7 ms; at 1024x1024x4, 6.9 / 5.0 ms).
-static int launch_shape(const ptgpu_ctx *ctx, int total, bool half, RenderParams &P) {
+static LaunchShapes launch_shapes(const ptgpu_ctx *ctx, const DevAccel &acc, int total, bool automatic, bool share) {
     const int cus = ctx->cu_count;
-    const bool deep = stack_for_wide(P.acc, 0) != 32;
+    const bool deep = stack_for_wide(acc, 0) != 32;
     auto shape = [&](int lanes, int per_cu) {
         const int all = cus * per_cu, need = (total + 4 * lanes - 1) / (4 * lanes);
         return LaunchShape{need < 1 ? 1 : need < all ? need : all, lanes};
     };
-    if (!ctx->blocks_auto || !half) {
-        P.inside = P.outside = shape(kWave, ctx->blocks_per_cu);
-        return P.inside.blocks;
+    if (!automatic) {
+        const LaunchShape s = shape(kWave, ctx->blocks_per_cu);
+        return LaunchShapes{s, s};
     }
     int in = kWave, out = kWave;
-    if (ctx->quad > 0 && !P.trav_stats) {   // (counting launches keep one walk order for every shape)
+    if (share) {
         in = total <= 12 * cus ? 1 : total <= 24 * cus ? 2 : total <= (deep ? 48 : 32) * cus ? 4 : total <= (deep ? 96 : 64) * cus ? 8 : kWave;
         out = total <= 16 * cus ? 1 : total <= 32 * cus ? 2 : total <= 64 * cus ? 4 : total <= 128 * cus ? 8 : kWave;
     }
-    P.inside = shape(in, 4);
-    P.outside = shape(out, out == kWave && total < 2 * 4 * 256 * cus ? 2 : 4);
-    return std::max(P.inside.blocks, P.outside.blocks);
+    return LaunchShapes{shape(in, 4), shape(out, out == kWave && total < 2 * 4 * 256 * cus ? 2 : 4)};
+}
+
+static bool walks_half(const ptgpu_ctx *ctx, const DevAccel &acc) {
+    return (ctx->engine == 0 || ctx->engine == 3) && acc.mode != PTGPU_ACCEL_NONE && acc.root >= 0 && ctx->wide == 2 &&
+           acc.nodes4h && stack_for_wide(acc, ctx->stack_min) > 0;
+}
+
+bool launch_spreads(const ptgpu_ctx *ctx, const DevAccel &acc, int pixels) {
+    if (!walks_half(ctx, acc) || ctx->quad == 0) return false;
+    const LaunchShapes s = launch_shapes(ctx, acc, pixels, true, true);
+    return s.inside.lanes < kWave && s.outside.lanes < kWave;
 }
 
 int launch_render(ptgpu_ctx *ctx, const DevAccel &acc, const RenderLaunch &L) {
@@ -1611,8 +1625,10 @@ int launch_render(ptgpu_ctx *ctx, const DevAccel &acc, const RenderLaunch &L) {
         P.status = ctx->rec_status.as<unsigned>();
     }
     const bool lanes_engine = (ctx->engine == 0 || ctx->engine == 3) && acc.mode != PTGPU_ACCEL_NONE && acc.root >= 0;
-    const bool half = lanes_engine && ctx->wide == 2 && acc.nodes4h && stack_for_wide(acc, ctx->stack_min) > 0;
-    const int blocks = launch_shape(ctx, total, half, P);
+    const bool half = walks_half(ctx, acc);
+    // (counting launches keep one walk order for every shape)
+    P.launch = launch_shapes(ctx, acc, total, ctx->blocks_auto && half, ctx->quad > 0 && !L.trav_stats);
+    const int blocks = std::max(P.launch.inside.blocks, P.launch.outside.blocks);
     // auto and engine 3: per-lane states whenever there is a tree to walk (measured fastest at every
     // size tried); brute force and single-leaf scenes keep the lockstep megakernel
     if (lanes_engine) {
@@ -2283,7 +2299,7 @@ int launch_batch(ptgpu_ctx *ctx, BatchChannel &ch, const ptgpu_render_job *jobs,
         P.job_begin = reinterpret_cast<const unsigned *>(static_cast<char *>(d_table) + K.bo);
         P.njobs = (int)K.jobs.size();
         P.slack = 0;
-        P.inside.lanes = kWave;
+        P.launch.inside.lanes = kWave;
         P.depth_cap = wide_depth_cap(K.st);
         P.status = K.checks ? ctx->rec_status.as<unsigned>() : nullptr;
         const long long all = (long long)ctx->cu_count * ctx->batch_blocks_per_cu;

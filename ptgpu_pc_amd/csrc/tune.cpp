@@ -4,14 +4,17 @@
 // for every value (the tests check each one).  The tuner times real work on the caller's own scene
 // and frame with HIP events on the context's stream and keeps the fastest setting:
 //   * LBVH sort digit width (4 or 8 bits): full rebuild time;
-//   * single-frame render: workgroups per CU (1..4; 1..2 when frames_per_build is 0, see below),
-//     shading-pass threshold `regroup` (8, 16, 32), node format (four-wide binary16, four-wide fp32 or
-//     binary);
+//   * single-frame render: launch shape (the automatic one, which is the default, or 1..4 workgroups per CU; see
+//     below for frames_per_build 0), shading-pass threshold `regroup` (8, 16, 32; the default, 24, is within 1.5% of
+//     the better of 16 and 32: 1024x768x16 of the 327,692-shape mesh 17.9 / 18.1 ms with 32, 512x512x8 of the
+//     65,538-shape soup 5.09 / 5.05 with 16), node format (four-wide binary16, four-wide fp32 or binary);
 //   * treelet restructuring (none, 5 or 7 leaves): build + optimise time plus `frames_per_build`
 //     renders on the resulting tree, the cost a caller pays per rebuild.  frames_per_build 0 means
 //     each rebuild runs on another stream beside the previous frame's render: the cost is the render
 //     alone, for a build short enough to hide there (kOverlapBuildShare);
-//   * batched renders: workgroups per CU (2..4) and `batch_regroup` (16, 32, 64) on the caller's job list.
+//   * batched renders: workgroups per CU (2..4) and `batch_regroup` (16, 32, 64; the default, 40, is within 2.5% of the
+//     better of 32 and 64: 16 scenes of 1,000 to 200,000 shapes 6.47 / 6.37 ms with 32, eight of up to 20,000 1.20 /
+//     1.23 with 64) on the caller's job list.
 // Trial renders write to scratch copies of the caller's frame buffers, so the caller's colours,
 // seeds and pixels are untouched.
 #include <cstring>
@@ -145,17 +148,20 @@ int autotune_frame(ptgpu_ctx *ctx, ptgpu_clbvh *h, const ptgpu_render_args *a, i
     PT_TRY(restore());
     PT_TRY(render());   // first use after a build: derived views and light list
     float best_render = 1e30f;
-    int bb = ctx->blocks_per_cu, br = ctx->regroup, bw = ctx->wide;
-    // With frames in flight (frames_per_build 0) the next frame's render starts while this one drains:
-    // a launch that asks for more than half of a CU's workgroups leaves it no room (measured: three or
-    // four per CU render one frame alone as fast, but frames in flight 2-5% slower at C2).
+    int bb = 0, br = ctx->regroup, bw = ctx->wide;
+    // With frames in flight (frames_per_build 0) the next frame's render and the next tree's build start while this one
+    // runs: more than two workgroups per CU leave the build no room (it takes 0.27 ms beside two and ends with the
+    // frame beside four) and hardly speed up the frames (two in flight, two / four per CU: 512x512x8 of the
+    // 65,538-shape soup 2.98 / 3.23 ms a frame, 640x480x2 of the 20,492-shape mesh 1.13 / 1.19).  The automatic shape is
+    // tried there only where it spreads the frame, whose workgroups then end with their pixels.
     const int bpc_max = frames_per_build == 0 ? 2 : 4;
-    ctx->blocks_auto = false;
+    const bool automatic = frames_per_build > 0 || launch_spreads(ctx, h->acc, (int)(a->width * a->height));
     for (int wide : {2, 1, 0})
-        for (int bpc = 1; bpc <= bpc_max; bpc++)
+        for (int bpc = wide == 2 && automatic ? 0 : 1; bpc <= bpc_max; bpc++)   // 0: the automatic shape
             for (int rg : {8, 16, 32}) {
                 ctx->wide = wide;
-                ctx->blocks_per_cu = bpc;
+                ctx->blocks_auto = bpc == 0;
+                ctx->blocks_per_cu = bpc ? bpc : kBlocksPerCu;
                 ctx->regroup = rg;
                 float ms = 0.f;
                 PT_TRY(best_ms(ctx, ev, trials, restore, render, &ms));
@@ -166,7 +172,8 @@ int autotune_frame(ptgpu_ctx *ctx, ptgpu_clbvh *h, const ptgpu_render_args *a, i
                     bw = wide;
                 }
             }
-    ctx->blocks_per_cu = bb;
+    ctx->blocks_auto = bb == 0;
+    ctx->blocks_per_cu = bb ? bb : kBlocksPerCu;
     ctx->regroup = br;
     ctx->wide = bw;
 
@@ -199,7 +206,7 @@ int autotune_frame(ptgpu_ctx *ctx, ptgpu_clbvh *h, const ptgpu_render_args *a, i
     PT_TRY(render());
     PT_HIP(hipStreamSynchronize(ctx->stream));
 
-    out->blocks_per_cu = bb;
+    out->blocks_per_cu = bb ? bb : bpc_max;   // (the automatic shape: as many as it may take)
     out->regroup = br;
     out->wide = bw;
     out->batch_blocks_per_cu = ctx->batch_blocks_per_cu;

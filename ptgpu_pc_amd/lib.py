@@ -81,6 +81,7 @@ _SIGS = {
     "ptgpu_ctx_set_max_depth": [vp, i32],
     "ptgpu_ctx_set_engine": [vp, i32],
     "ptgpu_ctx_set_tuning": [vp, C.c_char_p, i32],
+    "ptgpu_ctx_get_tuning": [vp, C.c_char_p, vp],
     "ptgpu_synchronize": [vp],
     "ptgpu_malloc": [vp, C.c_size_t, C.POINTER(vp)],
     "ptgpu_free": [vp, vp],
@@ -323,6 +324,11 @@ class Context:
 
     def set_tuning(self, name: str, value: int) -> None:
         _check(self.lib.ptgpu_ctx_set_tuning(self.handle, name.encode(), int(value)))
+
+    def get_tuning(self, name: str) -> int:
+        v = i32()
+        _check(self.lib.ptgpu_ctx_get_tuning(self.handle, name.encode(), C.byref(v)))
+        return v.value
 
     def set_max_depth(self, d: int) -> None:
         _check(self.lib.ptgpu_ctx_set_max_depth(self.handle, d))
@@ -680,11 +686,12 @@ def host_radiance_box(accel: int, colors: np.ndarray, seeds: np.ndarray, camera:
 
 def autotune(ctx: Context, bvh: CLBVH, *, frames_per_build: int = 1, trials: int = 2, **render_kwargs) -> dict:
     """ptgpu_autotune: digit width, launch shape and treelet size for this scene and frame (the keyword
-    arguments of `render`); applied to ctx and bvh, which is left holding a tree built with them."""
+    arguments of `render`); applied to ctx and bvh, which is left holding a tree built with them.  "automatic": the
+    automatic launch shape was the fastest (elsewhere: set_tuning("blocks_per_cu", 0))."""
     a = _render_args(**render_kwargs)
     t = Tuning()
     _check(ctx.lib.ptgpu_autotune(ctx.handle, _h(bvh), C.byref(a), int(frames_per_build), int(trials), C.byref(t)))
-    return t.as_dict()
+    return {**t.as_dict(), "automatic": ctx.get_tuning("blocks_per_cu") == 0}
 
 
 def autotune_batch(ctx: Context, jobs: list, trials: int = 2) -> dict:
