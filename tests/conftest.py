@@ -22,3 +22,20 @@ def ctx():
     c = pt.Context(0)
     yield c
     c.close()
+
+
+_TUNING = ("regroup", "blocks_per_cu", "wide", "quad", "stack", "short_stack", "batch_regroup", "batch_blocks_per_cu")
+
+
+@pytest.fixture(autouse=True)
+def session_tuning(request):
+    """The session's context leaves each test with the launch settings it came with (some tests restore numbers of their
+    own, and those after them would run those settings instead of the defaults)."""
+    if "ctx" not in request.fixturenames:
+        yield
+        return
+    c = request.getfixturevalue("ctx")
+    saved = {k: c.get_tuning(k) for k in _TUNING}
+    yield
+    for k, v in saved.items():
+        c.set_tuning(k, v)
