@@ -404,8 +404,9 @@ __device__ __forceinline__ void brute_stage(const Prim *prims, int n, BruteScene
         const Prim *q = prims + (k < n ? k : 0);
         float4 p0 = q->p0, p1 = q->p1, p2 = q->p2;
         if (k >= n || (__float_as_int(p2.w) & 0xff) == SPHERE) {
-            if (k >= n) p1.x = __builtin_nanf("");   // past the end: no hit
-            p0.w = p1.x * p1.x;
+            // past the end: no hit, by a determinant of -infinity (a NaN would send the four to the general form)
+            if (k >= n) p1.x = __builtin_nanf("");
+            p0.w = k < n ? p1.x * p1.x : -__builtin_inff();
             p2.w = __int_as_float(SPHERE);
         }
         S.p[3 * k] = p0;
