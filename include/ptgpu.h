@@ -148,6 +148,11 @@ void ptgpu_host_free(void *h_ptr);
 /* A plain device copy kernel (bytes a multiple of 16) with known traffic, for calibrating hardware
  * memory-traffic counters. */
 int ptgpu_copy_calibration(ptgpu_ctx *ctx, void *d_dst, const void *d_src, size_t bytes);
+/* Compares a helper of the render kernels with its plain form for `count` binary32 bit patterns from `first` on
+ * (wrapping): the reciprocal with 1.0f / x, the root with sqrtf, the pack's byte with the reference's toInt.
+ * *wrong: how many differ (a NaN equals any other). */
+enum { PTGPU_CHECK_RCP = 0, PTGPU_CHECK_SQRT = 1, PTGPU_CHECK_PACK = 2 };
+int ptgpu_check_math(ptgpu_ctx *ctx, int which, unsigned first, unsigned long long count, unsigned long long *wrong);
 /* Stream-ordered timing: record a named event slot (0..15) and read the elapsed ms between two. */
 int ptgpu_event_record(ptgpu_ctx *ctx, int slot);
 int ptgpu_event_elapsed_ms(ptgpu_ctx *ctx, int slot_begin, int slot_end, float *ms);

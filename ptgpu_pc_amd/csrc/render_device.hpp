@@ -31,9 +31,9 @@ PT_HD f3 cross3(f3 a, f3 b) {
 // 1/x and sqrt(x), correctly rounded, in three and five instructions where the compiler's forms take eleven
 // and sixteen (they scale every operand for the ends of the exponent range).  The hardware's reciprocal
 // and reciprocal square root are within one ulp, and one fma correction makes the result the IEEE
-// one for every binary32 x of the stated range: all 4.19e9 values of 2^-125 <= |x| <= 2^125 (1/x) and all
-// of 2^-96 <= x <= 2^126 (sqrt) were compared on gfx950.  A wave with any other x takes the compiler's
-// form (a branch of the whole wave: no lane mask to save and restore).
+// one for every binary32 x of the stated range, 2^-125 <= |x| <= 2^125 (1/x) and 2^-96 <= x <= 2^126 (sqrt).  A
+// wave with any other x takes the compiler's form (a branch of the whole wave: no lane mask to save and
+// restore).  ptgpu_check_math compares both with the compiler's forms for every binary32 x.
 PT_HD float rcp_exact(float x) {
 #if defined(__HIP_DEVICE_COMPILE__)
     const float a = fabsf(x);
@@ -44,12 +44,17 @@ PT_HD float rcp_exact(float x) {
     return 1.0f / x;
 #endif
 }
-PT_HD float sqrt_exact(float x) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    if (__builtin_expect(__ballot(!(x >= 0x1p-96f && x <= 0x1p126f)) != 0ull, 0)) return sqrtf(x);
+constexpr float kRootLeast = 0x1p-96f, kRootMost = 0x1p126f;
+// the root of an x in that range (a NaN below zero)
+__device__ __forceinline__ float sqrt_steps(float x) {
     const float y = __builtin_amdgcn_rsqf(x);
     const float g = x * y;
     return __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * y, g);
+}
+PT_HD float sqrt_exact(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if (__builtin_expect(__ballot(!(x >= kRootLeast && x <= kRootMost)) != 0ull, 0)) return sqrtf(x);
+    return sqrt_steps(x);
 #else
     return sqrtf(x);
 #endif
@@ -441,21 +446,20 @@ __device__ __forceinline__ void brute_four(const BruteScene<CAP> &S, unsigned lo
         }
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            // sqrt_exact's steps; the root of a negative determinant is a NaN, which fails both comparisons
-            const float y = __builtin_amdgcn_rsqf(det[j]);
-            const float q = det[j] * y;
-            const float r = __builtin_fmaf(__builtin_fmaf(-q, q, det[j]), 0.5f * y, q);
+            const float r = sqrt_steps(det[j]);   // of a negative determinant a NaN, which fails both comparisons
             const float t0 = b[j] - r, t1 = b[j] + r;
             const float tt = t0 > kEpsilon ? t0 : t1;
             t[j] = tt > kEpsilon ? tt : inf;
         }
-        // a determinant at the ends of the exponent range (from its bits: below 2^-96 from +0 on, or above 2^126)
+        // a determinant outside the steps' range (from its bits: from +0 to below the least, or above the most)
+        constexpr unsigned least = __builtin_bit_cast(unsigned, kRootLeast);
+        constexpr int most = __builtin_bit_cast(int, kRootMost);
         auto bits = [&](int j) { return __float_as_int(det[j]); };
         auto umin = [](unsigned x, unsigned y) { return x < y ? x : y; };
         auto imax = [](int x, int y) { return x > y ? x : y; };
         const unsigned lo = umin(umin(bits(0), bits(1)), umin(bits(2), bits(3)));
         const int hi = imax(imax(bits(0), bits(1)), imax(bits(2), bits(3)));
-        if (__builtin_expect(__ballot(lo < 0x0f800000u || hi > 0x7e800000) != 0ull, 0)) {
+        if (__builtin_expect(__ballot(lo < least || hi > most) != 0ull, 0)) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const float x = sph_isect(c[j], S.p[3 * (4 * g + j) + 1].x, o, d);
@@ -541,7 +545,7 @@ PT_HD int to_int(float x) {   // vec.h:60 with the OpenCL clamp builtin
 // the table settles it, in about 20 instructions instead of the 150 of powf, which every shading pass that
 // finished a pixel ran three times.  powf is not monotone in its last bits (of all binary32 x two lie one and two
 // places beyond a threshold on the wrong side), so a wave with an x within four places of one calls to_int:
-// the result is to_int's (compared for every binary32 x).
+// the result is to_int's (ptgpu_check_math compares the two for every binary32 x).
 constexpr int kPackEntries = 257;
 __device__ __forceinline__ int to_int_tab(float x, const float *tab) {
     x = fminf(fmaxf(x, 0.f), 1.f);

@@ -81,6 +81,7 @@ _SIGS = {
     "ptgpu_ctx_set_max_depth": [vp, i32],
     "ptgpu_ctx_set_engine": [vp, i32],
     "ptgpu_ctx_set_tuning": [vp, C.c_char_p, i32],
+    "ptgpu_check_math": [vp, i32, u32, C.c_ulonglong, vp],
     "ptgpu_ctx_get_tuning": [vp, C.c_char_p, vp],
     "ptgpu_synchronize": [vp],
     "ptgpu_malloc": [vp, C.c_size_t, C.POINTER(vp)],
@@ -345,6 +346,13 @@ class Context:
 
     def copy_calibration(self, dst: DeviceArray, src: DeviceArray, nbytes: int) -> None:
         _check(self.lib.ptgpu_copy_calibration(self.handle, dst.ptr, src.ptr, nbytes))
+
+    def check_math(self, which: int, first: int = 0, count: int = 1 << 32) -> int:
+        """ptgpu_check_math: bit patterns from `first` on for which the reciprocal (0), the root (1) or the pack's byte
+        (2) of the render kernels differs from its plain form."""
+        wrong = C.c_ulonglong()
+        _check(self.lib.ptgpu_check_math(self.handle, int(which), int(first) & 0xFFFFFFFF, int(count), C.byref(wrong)))
+        return wrong.value
 
     def graph_begin(self) -> None:
         """Start recording this context's library calls into a HIP graph (see ptgpu_graph_begin)."""
