@@ -94,8 +94,10 @@ def cpu_render_rate(shapes, lc, cam, btn, btl, budget_s, w=None, h=None, depth=N
 
 
 RENDER_KERNEL = "k_render_lanes"
-# the timed instance: single frame, no statistics (<stack, STATS, WIDE, MULTI, HALF>)
+# the timed instance: single frame, no statistics (<stack, STATS, WIDE, MULTI, HALF, WAIT>)
 RENDER_INSTANCE = "k_render_lanes<%, false, %, false, %>"
+RENDER_INSTANCE_RE = re.compile(r"k_render_lanes<\d+, false, (true|false), false, (true|false), (true|false)>")
+RENDER_SOURCES = ("render.hip", "walk_half.hpp", "render_device.hpp", "device_util.hpp", "common.hpp")
 WORKLOAD = ("LBVH build + BVH traversal: 65,536-triangle soup (seed 1) + emissive quad, 512x512, 8 spp, depth 5, "
             "30-bit Morton, one leaf per primitive")
 TRAFFIC_FILE = ROOT / "profiles" / "k_render_lanes_c2_traffic.json"
@@ -142,8 +144,7 @@ def profile_summary(d: Path, out_md: Path) -> None:
         for name, val in _db_rows(dbp, "select counter_name, avg(value) from counters_collection where kernel_name "
                                        f"like '%{RENDER_INSTANCE}%' group by counter_name"):
             sq[name] = val
-    timed = re.compile(r"k_render_lanes<\d+, false, (true|false), false, (true|false)>")
-    render_avg = next((r[2] / 1e3 for r in rows if timed.search(r[0])), None)
+    render_avg = next((r[2] / 1e3 for r in rows if RENDER_INSTANCE_RE.search(r[0])), None)
     cmds = json.loads((d / "commands.json").read_text())
     lines = [f"# {RENDER_KERNEL} — C2 (65,538-shape soup, 512x512, 8 spp, depth 5), MI355X", "",
              "Commands (run from the repository root; rocprofv3 output directories as named):", ""]
@@ -189,7 +190,8 @@ def profile_summary(d: Path, out_md: Path) -> None:
         ratios["valu_busy"] = sq["SQ_ACTIVE_INST_VALU"] * 4 / (1024 * sq["GRBM_GUI_ACTIVE"] / 8)
     if "TCC_HIT_sum" in sq:
         ratios["l2_hit"] = sq["TCC_HIT_sum"] / (sq["TCC_HIT_sum"] + sq["TCC_MISS_sum"])
-    TRAFFIC_FILE.write_text(json.dumps({"kernel": RENDER_KERNEL, "workload": WORKLOAD, "traffic_bytes": traffic,
+    TRAFFIC_FILE.write_text(json.dumps({"kernel": RENDER_KERNEL, "workload": WORKLOAD, "version": render_version(),
+                                        "traffic_bytes": traffic,
                                         "fetch_kib": f_k, "write_kib": w_k, "fetch_factor": f_scale,
                                         "write_factor": w_scale, "avg_ms_rocprof": render_avg,
                                         **{k: round(v, 4) for k, v in ratios.items()},
@@ -199,10 +201,8 @@ def profile_summary(d: Path, out_md: Path) -> None:
 
 # stage of each batched-build kernel, for the per-stage algorithmic GB/s of the 64-scene build
 BATCH_STAGE = {"kb_fill": "sort", "kb_bounds": "morton", "kb_bounds_final": "morton", "kb_morton": "morton",
-               "kb_karras": "refit", "kb_sort_hist": "sort", "kb_sort_scan": "sort", "kb_sort_pass": "sort",
-               "kb_refit": "refit", "kb_karras_morton": "refit", "kb_mrefit_chunk": "refit", "kb_mrefit_mid": "refit",
-               "kb_mrefit_top": "refit",
-               "kb_gather": "refit"}
+               "kb_karras": "refit", "kb_sort_hist": "sort", "kb_sort_pass": "sort", "kb_refit": "refit",
+               "kb_mtree": "traversal_tree", "kb_gather": "traversal_tree"}
 
 
 def batch_build_summary(db: Path, cmds: list, out_md: Path) -> None:
@@ -231,10 +231,10 @@ def batch_build_summary(db: Path, cmds: list, out_md: Path) -> None:
         lines.append(f"| `{short}` | {k} | {avg:.4f} | {ms:.4f} |")
     lines += ["", f"Total kernel time per batched build: {total:.3f} ms = {n_total / total / 1e3:.0f} Mtri/s.", "",
               "| stage | ms | algorithmic B/prim | achieved GB/s | fraction of 8 TB/s |", "|---|---|---|---|---|"]
-    for st in STAGE_BYTES:
+    for st, per_prim in (*STAGE_BYTES.items(), ("traversal_tree", TRAV_TREE_BYTES)):
         ms = per_stage.get(st, 0.0)
-        gbs = STAGE_BYTES[st] * n_total / (ms * 1e-3) / 1e9 if ms else 0.0
-        lines.append(f"| {st} | {ms:.3f} | {STAGE_BYTES[st]} | {gbs:.0f} | {gbs / HBM_PEAK_GBS:.3f} |")
+        gbs = per_prim * n_total / (ms * 1e-3) / 1e9 if ms else 0.0
+        lines.append(f"| {st} | {ms:.3f} | {per_prim} | {gbs:.0f} | {gbs / HBM_PEAK_GBS:.3f} |")
     out_md.write_text("\n".join(lines) + "\n")
     print(out_md.read_text())
 
@@ -259,15 +259,26 @@ def c3_summary(db: Path, c3: dict, cmds: list, out_md: Path) -> None:
     print(out_md.read_text())
 
 
+def render_version() -> str:
+    """Names the version of the render kernel that counters were taken of: a hash of its sources, comments and
+    spacing left out."""
+    import hashlib
+    h = hashlib.sha256()
+    for name in RENDER_SOURCES:
+        text = (ROOT / "ptgpu_pc_amd" / "csrc" / name).read_text()
+        h.update("".join(re.sub(r"//[^\n]*", "", text).split()).encode())
+    return h.hexdigest()[:16]
+
+
 def measured_counters():
     """Counter figures of the render kernel from the committed rocprofv3 summary of this workload (or
-    None): HBM bytes per launch (calibrated FETCH_SIZE + WRITE_SIZE), the profile's average duration, L2
+    None where they are another version's): HBM bytes per launch (calibrated FETCH_SIZE + WRITE_SIZE), the profile's average duration, L2
     hit rate, VALU busy fraction and VALU lane utilisation."""
     try:
         t = json.loads(TRAFFIC_FILE.read_text())
     except (OSError, ValueError):
         return None
-    if t.get("kernel") != RENDER_KERNEL or t.get("workload") != WORKLOAD:
+    if t.get("kernel") != RENDER_KERNEL or t.get("workload") != WORKLOAD or t.get("version") != render_version():
         return None
     return t
 
@@ -284,10 +295,9 @@ def measured_traffic():
 # of N, so it has no pass of its own)
 STAGE_BYTES = {"morton": 76, "sort": 68, "refit": 156 + 28}
 BUILD_BYTES_PER_PRIM = sum(STAGE_BYTES.values())   # 328 B per primitive with 8-bit digits
-# the Morton-keyed traversal tree, per primitive: Karras over sorted keys (reads 4 B per key,
-# writes a 16-B node and 8 B of parents) + refit (reads a 24-B leaf bound, the 16-B node and a 4-B
-# parent, writes a 64-B traversal node)
-TRAV_TREE_BYTES = 4 + 16 + 8 + 24 + 16 + 4 + 64
+# the Morton-keyed traversal tree, per primitive: a sorted key and a 24-B leaf bound read, a 64-B traversal node
+# written (the items left over between its levels, some 10 B, are not counted)
+TRAV_TREE_BYTES = 4 + 24 + 64
 
 
 def render_roofline(alg_bytes, avg_ms, box_tests, prim_tests, box_bytes, measured=True, kernel=None, step_ms=None):
