@@ -71,7 +71,6 @@ struct RenderParams {
     int njobs;
     const int2 *tiles;            // tiled launches (RadianceBoxGPU): tile origins; NULL renders the whole frame
     int tile_w, tile_h;
-    int slack;                    // binary16 walk: stack entries above a depth-first walk's need (half_sparse)
     LaunchShapes launch;
     int depth_cap;                // deepest tree the launch's stack holds (checked when acc.height_check is set)
     const float *pack_tab;        // to_int_tab's table
@@ -458,7 +457,8 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
     T.prims = to_gmem(P.acc.prims);
     T.nprims = P.acc.nprims;
     T.skip = P.acc.nshapes - 1;
-    int t_nnodes = P.acc.nnodes, t_root = P.acc.root, t_slack = P.slack;
+    int t_nnodes = P.acc.nnodes, t_root = P.acc.root;
+    int t_slack = HALF && !MULTI ? half_slack(STACK, P.acc) : 0;
 
     int st = (int)__lane_id() < shape.lanes ? kNeed : kIdle;
     bool drained = false;
@@ -993,8 +993,8 @@ __device__ __forceinline__ bool half_blurs(const DevAccel &A) {
 template <int STACK, bool WAIT>
 __global__ __launch_bounds__(256, STACK <= 36 ? 4 : 2) void k_trace_half(DevAccel A, const Ray *rays, const float *maxt,
                                                                          int n, float *tout, int *idout, int *hitout,
-                                                                         int any, int lanes, int regroup_max, int quad,
-                                                                         int slack) {
+                                                                         int any, int lanes, int regroup_max, int quad) {
+    const int slack = half_slack(STACK, A);
     __shared__ int s_stack[STACK * 256];
     int *const stk = s_stack + threadIdx.x;
     if (half_blurs(A)) {
@@ -1617,7 +1617,6 @@ int launch_render(ptgpu_ctx *ctx, const DevAccel &acc, const RenderLaunch &L) {
     P.tiles = L.tiles;
     P.tile_w = L.tile_w;
     P.tile_h = L.tile_h;
-    P.slack = 0;
     P.depth_cap = binary_depth_cap(st);
     P.status = nullptr;
     if (acc.height_check) {
@@ -1641,7 +1640,6 @@ int launch_render(ptgpu_ctx *ctx, const DevAccel &acc, const RenderLaunch &L) {
         // allocation-free entry does not ask the runtime for.
         const bool tiny = half && sw > 0 && ctx->short_stack == 2 && !L.no_alloc;
         const bool shortst = half && sw == 48 && ctx->short_stack == 1 && !L.no_alloc;
-        if (half && sw > 0) P.slack = half_slack(tiny ? kStackTiny : shortst ? kStackShort : sw, acc);
 #define PT_LANES(ST, STATS_, WIDE_, HALF_)                                                                      \
     hipLaunchKernelGGL((k_render_lanes<ST, STATS_, WIDE_, false, HALF_>), dim3(blocks), dim3(256), 0, ctx->stream, P)
 #define PT_LANES_W(ST, STATS_) \
@@ -1714,7 +1712,7 @@ int launch_trace(ptgpu_ctx *ctx, const DevAccel &acc, unsigned int shapeCnt, con
         if (blocks > (long long)cus * per_cu) blocks = (long long)cus * per_cu;
 #define PT_TRACE_W(ST, WAIT)                                                                                          \
     hipLaunchKernelGGL((k_trace_half<ST, WAIT>), dim3((unsigned)blocks), dim3(256), 0, ctx->stream, acc, d_rays, d_maxt, n, \
-                       d_t, d_id, d_hit, any ? 1 : 0, lanes, 8, ctx->quad, half_slack(ST, acc))
+                       d_t, d_id, d_hit, any ? 1 : 0, lanes, 8, ctx->quad)
 #define PT_TRACE(ST) \
     do { if (acc.mode == PTGPU_ACCEL_KD) PT_TRACE_W(ST, true); else PT_TRACE_W(ST, false); } while (0)
         if (sw == 32) PT_TRACE(32);
@@ -2298,8 +2296,7 @@ int launch_batch(ptgpu_ctx *ctx, BatchChannel &ch, const ptgpu_render_job *jobs,
         P.jobs = reinterpret_cast<const RenderJob *>(static_cast<char *>(d_table) + K.jo);
         P.job_begin = reinterpret_cast<const unsigned *>(static_cast<char *>(d_table) + K.bo);
         P.njobs = (int)K.jobs.size();
-        P.slack = 0;
-        P.launch.inside.lanes = kWave;
+            P.launch.inside.lanes = kWave;
         P.depth_cap = wide_depth_cap(K.st);
         P.status = K.checks ? ctx->rec_status.as<unsigned>() : nullptr;
         const long long all = (long long)ctx->cu_count * ctx->batch_blocks_per_cu;
