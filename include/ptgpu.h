@@ -122,7 +122,9 @@ int ptgpu_ctx_set_engine(ptgpu_ctx *ctx, int engine);
  * launch picks the workgroups and the pixels per wave from the frame's size, the tree's height and the
  * camera's place), "wide"
  * (engine 3's node format: 0 binary, 1 four-wide fp32, 2 four-wide with binary16 boxes rounded
- * outward, half the bytes per node, where the tree's leaves allow it; default 2), "quad" (0..16,
+ * outward, half the bytes per node, where the tree's leaves allow it and binary16 steps are not large beside
+ * them, as they are far from the origin; default 2.  Batch queries, ptgpu_trace_closest and ptgpu_trace_any, walk
+ * the same binary16 nodes with 2, and binary nodes otherwise), "quad" (0..16,
  * with wide 2: when at most this many lanes of a wave are traversing, four or more lanes share each
  * query, one child box each and several stack entries at a time; default 16, 0 off); "stack" (0..64, the smallest traversal stack
  * class a launch uses: the launch takes the first class (24 or 64 entries for binary nodes, 32, 48 or 64

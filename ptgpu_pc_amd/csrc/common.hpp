@@ -97,6 +97,8 @@ struct DevAccel {
     int nshapes = 0;       // shapeCnt: any-hit queries ignore shape nshapes-1 (IntersectP, Q10)
     int depth = 0;         // tree height: deepest leaf in edges from the root (bounds the stack)
     int mode = PTGPU_ACCEL_NONE;
+    int blurs = 0;         // 1: binary16 bounds blur the tree (half_bounds.hpp): its walks take binary32 boxes.  A tree whose
+                           // first walk could not wait for the answer keeps that of the build before it.
     int leaf_runs = 0;     // 1: every leaf range is disjoint and its last Prim carries kLastInLeaf
     // A traversal recorded into a graph right after a build, before its height could be read back:
     // `depth` is then a bound, and the build's status words (error word, -, height) are checked

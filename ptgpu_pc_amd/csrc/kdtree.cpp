@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "half_bounds.hpp"
 
 using namespace ptgpu;
 
@@ -308,6 +309,27 @@ Prim host_prim(const Shape &s, int id, bool last) {
     return p;
 }
 
+// Whether binary16 bounds blur the tree (half_bounds.hpp), from all its leaf boxes.
+bool half_blurs_kd(const std::vector<KNode> &nodes) {
+    double exact = 0.0, wide = 0.0;
+    // the binary16 number next to v on the side of `up` (a step is 2^-24 up to 2^-14, else 2^-10 of v's power of two)
+    auto half = [](float v, bool up) -> double {
+        const double a = std::fabs((double)v);
+        const double step = a < 0x1p-14 ? 0x1p-24 : std::ldexp(1.0, std::ilogb(a) - 10);
+        const double h = (up ? std::ceil(v / step) : std::floor(v / step)) * step;
+        return std::fabs(h) > 65504.0 ? std::copysign(HUGE_VAL, h) : h;
+    };
+    auto area = [](double x, double y, double z) { return x * y + y * z + z * x; };
+    for (const KNode &nd : nodes) {
+        if (!nd.leaf || nd.count <= 0) continue;
+        const Bound &b = nd.box;
+        exact += area((double)b.max_x - b.min_x, (double)b.max_y - b.min_y, (double)b.max_z - b.min_z);
+        wide += area(half(b.max_x, true) - half(b.min_x, false), half(b.max_y, true) - half(b.min_y, false),
+                     half(b.max_z, true) - half(b.min_z, false));
+    }
+    return blurred((float)exact, (float)wide);
+}
+
 // depth-first nodes -> TNode (internal nodes only, renumbered) + Prim (kn order), then upload
 int upload_device(ptgpu_kdtree *T) {
     const int nn = (int)T->nodes.size();
@@ -355,6 +377,7 @@ int upload_device(ptgpu_kdtree *T) {
     A.nnodes = ni;
     A.nshapes = T->n;
     A.leaf_runs = 1;
+    A.blurs = half_blurs_kd(T->nodes) ? 1 : 0;
     A.mode = PTGPU_ACCEL_KD;
     const KNode &root = T->nodes[0];
     if (root.leaf) {

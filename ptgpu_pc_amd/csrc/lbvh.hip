@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "device_util.hpp"
+#include "half_bounds.hpp"
 #include "lbvh.hpp"
 #include "lbvh_device.hpp"
 
@@ -213,6 +214,12 @@ __global__ __launch_bounds__(256) void k_refit_levels(const ShapeBox *boxes, con
                                                       BVHNodeGPU *btn, BVHNodeGPU *btl, TNode *tnodes, Prim *prims) {
     refit_levels_body<LEAF>(boxes, sorted, n, s0, levels, in_bounds, out_bounds, btn, btl, tnodes, prims, TNODES,
                             blockIdx.x);
+}
+
+// by one wave
+__global__ __launch_bounds__(kWave) void k_blurs(const TNode *nodes, int nnodes, unsigned *out) {
+    const bool b = half_blurs(nodes, nnodes);
+    if (threadIdx.x == 0) *out = b ? 1u : 0u;
 }
 
 template <bool LEAVES>
@@ -426,7 +433,7 @@ static int clbvh_sort(ptgpu_clbvh *h) {
 
 namespace ptgpu {
 // The Morton-keyed tree's height is known on the device after the refit; the traversal stack is
-// sized from it, so the first use after a build reads it back (one 4-byte copy).
+// sized from it, so the first use after a build reads it back, and with it whether binary16 bounds blur the tree.
 int clbvh_prepare_traversal(ptgpu_clbvh *h, bool recording, bool exact, bool wide) {
     const int known = h->known_height[h->optimized ? 1 : 0];
     const bool no_readback = recording || h->ctx->capturing || (h->speculate && known > 0);
@@ -444,16 +451,25 @@ int clbvh_prepare_traversal(ptgpu_clbvh *h, bool recording, bool exact, bool wid
             bound = kRecordedHeightDefault;
         h->acc.depth = bound;
         h->acc.height_check = misc_counters(h) + 9;
-    } else if (h->height_pending) {
-        unsigned w[3] = {0, 0, 0};   // error word, -, height
+    } else if (h->height_pending || (h->blurs_pending && exact && !recording && !h->ctx->capturing)) {
+        unsigned w[3] = {0, 0, 0};   // error word, blurs, height
+        if (h->blurs_pending) {
+            hipLaunchKernelGGL(k_blurs, dim3(1), dim3(kWave), 0, h->ctx->stream, (const TNode *)h->acc.nodes, h->acc.nnodes,
+                               misc_counters(h) + 10);
+            PT_HIP(hipGetLastError());
+        }
         PT_HIP(hipMemcpyAsync(w, misc_counters(h) + 9, 12, hipMemcpyDeviceToHost, h->ctx->stream));
         PT_HIP(hipStreamSynchronize(h->ctx->stream));
         PT_CHECK(w[0] == 0, PTGPU_ERR_HIP, "LBVH build failed (error word %u: 1 sort look-back spin limit, 2 "
                  "traversal-tree list overflow)", w[0]);
-        h->acc.depth = (int)w[2];
-        h->acc.height_check = nullptr;
-        h->known_height[h->optimized ? 1 : 0] = (int)w[2];
-        h->height_pending = false;
+        if (h->blurs_pending) h->acc.blurs = (int)w[1];
+        h->blurs_pending = false;
+        if (h->height_pending) {
+            h->acc.depth = (int)w[2];
+            h->acc.height_check = nullptr;
+            h->known_height[h->optimized ? 1 : 0] = (int)w[2];
+            h->height_pending = false;
+        }
     }
     if (h->wide_pending && wide) {
         PT_TRY(build_wide(h->ctx, &h->acc, h->tnodes4));
@@ -517,6 +533,7 @@ void ptgpu::clbvh_mark_built(ptgpu_clbvh *h) {
         h->acc.depth = 0;
     }
     h->height_pending = h->trav_topology == 1 && n >= 2;
+    h->blurs_pending = n >= 2;
 }
 
 extern "C" {

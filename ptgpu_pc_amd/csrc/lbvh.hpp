@@ -54,6 +54,7 @@ struct ptgpu_clbvh {
     bool export_pending = false;             // btn/btl still describe the tree before optimize
     int trav_topology = 1;    // traversal tree: 0 = the exported index-keyed tree, 1 = Morton-keyed LBVH
     bool height_pending = false;
+    bool blurs_pending = false;   // acc.blurs is the previous build's
     int known_height[2] = {0, 0};   // last heights read back: [0] plain build, [1] after optimize
     bool speculate = false;         // no read-back once a height is known: a bound, checked on the device
     unsigned *sorted = nullptr;
@@ -61,7 +62,7 @@ struct ptgpu_clbvh {
     ptgpu::DevAccel acc;
     std::vector<BVHNodeGPU> h_btn, h_btl;
     // misc: [0..5] scene centroid bounds, words 8.. counters ([0] unused, [1..8] sort
-    // tile counters, [9] build error word, [10] unused, [11] traversal-tree height),
+    // tile counters, [9] build error word, [10] binary16 bounds blur the tree, [11] traversal-tree height),
     // floats 64.. per-block bound partials
     float *scene6() const { return misc.as<float>(); }
     unsigned *counters() const { return misc.as<unsigned>() + 8; }

@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "device_util.hpp"
+#include "half_bounds.hpp"
 #include "lbvh.hpp"
 #include "lbvh_device.hpp"
 
@@ -146,11 +147,14 @@ __global__ __launch_bounds__(LEAVES ? kWave : kMThreads) void kb_mtree(const Bui
                        S.ms.counts[k & 1], S.tnodes, S.ctr + 11, S.ctr + 9, blockIdx.x - starts[s]);
 }
 
-// heights[s] = traversal-tree height, errs[s] = build error word
-__global__ __launch_bounds__(256) void kb_gather(const BuildSeg *g, int ns, unsigned *out) {
-    for (int s = threadIdx.x; s < ns; s += 256) {
+// Scene by scene: traversal-tree height, build error word, whether binary16 bounds blur the tree.
+__global__ __launch_bounds__(kWave) void kb_gather(const BuildSeg *g, int ns, unsigned *out) {
+    const int s = blockIdx.x;
+    const bool b = half_blurs(g[s].tnodes, g[s].n - 1);
+    if (threadIdx.x == 0) {
         out[s] = g[s].ctr[11];
         out[ns + s] = g[s].ctr[9];
+        out[2 * ns + s] = b ? 1u : 0u;
     }
 }
 
@@ -231,7 +235,7 @@ int build_batch(ptgpu_ctx *ctx, ptgpu_clbvh *const *hs, int ns) {
     const size_t upload = align16(o_fstarts + (size_t)(nf + 1) * sizeof(int));
     const size_t o_ctr = upload;
     const size_t o_out = o_ctr + 64;
-    const size_t dev_bytes = o_out + (size_t)2 * ns * sizeof(unsigned);
+    const size_t dev_bytes = o_out + (size_t)3 * ns * sizeof(unsigned);
     BuildStaging &B = ctx->build_staging;
     const bool recording = ctx->capturing;
     std::vector<char> img;   // recorded: the tables' image, staged by record_stage
@@ -321,10 +325,10 @@ int build_batch(ptgpu_ctx *ctx, ptgpu_clbvh *const *hs, int ns) {
         }
         return PTGPU_OK;
     }
-    hipLaunchKernelGGL(kb_gather, dim3(1), dim3(256), 0, st, d_segs, ns, d_out);
+    hipLaunchKernelGGL(kb_gather, dim3((unsigned)ns), dim3(kWave), 0, st, d_segs, ns, d_out);
     PT_HIP(hipGetLastError());
     unsigned *h_out = reinterpret_cast<unsigned *>(hp + o_out);
-    PT_HIP(hipMemcpyAsync(h_out, d_out, (size_t)2 * ns * sizeof(unsigned), hipMemcpyDeviceToHost, st));
+    PT_HIP(hipMemcpyAsync(h_out, d_out, (size_t)3 * ns * sizeof(unsigned), hipMemcpyDeviceToHost, st));
     PT_HIP(hipStreamSynchronize(st));
 
     bool sort_err = false;
@@ -338,6 +342,10 @@ int build_batch(ptgpu_ctx *ctx, ptgpu_clbvh *const *hs, int ns) {
             h->acc.depth = (int)h_out[s];
             h->known_height[0] = (int)h_out[s];
             h->height_pending = false;
+        }
+        if (h->blurs_pending && h_out[ns + s] == 0) {
+            h->acc.blurs = (int)h_out[2 * ns + s];
+            h->blurs_pending = false;
         }
         sort_err |= h_out[ns + s] != 0;
     }

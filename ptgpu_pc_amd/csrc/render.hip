@@ -929,59 +929,6 @@ __global__ __launch_bounds__(256) void k_trace(DevAccel A, const Ray *rays, cons
     }
 }
 
-// binary16 bounds rounded outward: the nearest binary16 (round to nearest even), stepped one
-// binary16 ulp down (lo) or up (hi) when it lies on the wrong side of x.  A NaN bound becomes the
-// infinity on its own side; values beyond the binary16 range round to +-65504 or the infinity.
-__device__ __forceinline__ unsigned short half_down(float x) {
-    if (x != x) return 0xFC00u;   // -inf
-    const _Float16 h = (_Float16)x;
-    unsigned short b = __builtin_bit_cast(unsigned short, h);
-    if ((float)h > x) {
-        if (b == 0x0000u || b == 0x8000u) b = 0x8001u;   // +-0 -> the largest negative subnormal
-        else if (b & 0x8000u) b = (unsigned short)(b + 1u);   // negative: away from zero
-        else b = (unsigned short)(b - 1u);                    // positive: toward zero
-    }
-    return b;
-}
-__device__ __forceinline__ unsigned short half_up(float x) {
-    if (x != x) return 0x7C00u;   // +inf
-    const _Float16 h = (_Float16)x;
-    unsigned short b = __builtin_bit_cast(unsigned short, h);
-    if ((float)h < x) {
-        if (b == 0x0000u || b == 0x8000u) b = 0x0001u;   // +-0 -> the smallest positive subnormal
-        else if (b & 0x8000u) b = (unsigned short)(b - 1u);   // negative: toward zero
-        else b = (unsigned short)(b + 1u);                    // positive: away from zero
-    }
-    return b;
-}
-
-// Do binary16 bounds blur this tree?  They are absolute, so a scene far from the origin (or past 65,504) has
-// boxes a binary16 step wide, whatever its shapes' size, and a walk of them visits much of the tree.  Each lane
-// widens the leaf boxes of one node, spread evenly over the tree, and the wave compares the areas' sums:
-// one answer for all waves of a launch.  At a sum over four times the exact one the two walks cost alike (100,000
-// rays; the scene moved by 16: 1,002-shape soup 67 us here against 71 over binary nodes, 327,692-shape mesh 413
-// against 236; by 256: 256 against 73 us, 146 against 0.24 ms).
-__device__ __forceinline__ bool half_blurs(const DevAccel &A) {
-    const int at = (int)((long long)__lane_id() * A.nnodes / kWave);
-    const TNode t = A.nodes[at];
-    float exact = 0.f, wide = 0.f;
-    auto add = [&](int r, float x0, float y0, float z0, float x1, float y1, float z1) {
-        auto area = [](float dx, float dy, float dz) { return dx * dy + dy * dz + dz * dx; };
-        auto lo = [](float v) { return (float)__builtin_bit_cast(_Float16, half_down(v)); };
-        auto hi = [](float v) { return (float)__builtin_bit_cast(_Float16, half_up(v)); };
-        if (r >= 0 || r == kEmptyRef) return;
-        exact += area(x1 - x0, y1 - y0, z1 - z0);
-        wide += area(hi(x1) - lo(x0), hi(y1) - lo(y0), hi(z1) - lo(z0));
-    };
-    add(t.r.x, t.a.x, t.a.y, t.a.z, t.a.w, t.b.x, t.b.y);
-    add(t.r.y, t.b.z, t.b.w, t.c.x, t.c.y, t.c.z, t.c.w);
-    for (int x = 1; x < kWave; x <<= 1) {
-        exact += __shfl_xor(exact, x);
-        wide += __shfl_xor(wide, x);
-    }
-    return __builtin_amdgcn_readfirstlane((int)(wide > 4.f * exact)) != 0;
-}
-
 // The same queries over binary16 four-wide nodes.  A lane whose query ends takes the wave's next ray once eight
 // lanes (or a quarter of those that still have work) have ended, so the wave's steps stay full, where one ray per
 // thread over binary nodes let the longest of 64 hold the others; few rays are spread over all waves, whose idle
@@ -997,22 +944,6 @@ __global__ __launch_bounds__(256, STACK <= 36 ? 4 : 2) void k_trace_half(DevAcce
     const int slack = half_slack(STACK, A);
     __shared__ int s_stack[STACK * 256];
     int *const stk = s_stack + threadIdx.x;
-    if (half_blurs(A)) {
-        // one ray per thread over the binary nodes; every four-wide stack class holds their walk
-        for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
-            const float *rf = reinterpret_cast<const float *>(rays + i);
-            const f3 o = mk(rf[0], rf[1], rf[2]), d = mk(rf[3], rf[4], rf[5]);
-            if (any) {
-                hitout[i] = anyhit<STACK>(A, o, d, maxt[i], stk, nullptr, nullptr) ? 1 : 0;
-            } else {
-                float t;
-                const int id = closest<STACK>(A, o, d, &t, stk, nullptr, nullptr);
-                tout[i] = id >= 0 ? t : 0.f;
-                idout[i] = id;
-            }
-        }
-        return;
-    }
     HalfTree T;
     T.nodes = to_gmem(A.nodes4h);
     T.prims = to_gmem(A.prims);
@@ -1268,11 +1199,19 @@ __global__ void k_ref_parents(const BVHNodeGPU *btn, int n, int *par, unsigned *
 
 // Height of that tree: the longest walk from a leaf up to the root (node 0), in edges, into err[1].
 // A leaf no node points at sets err[0] bit 4; a walk longer than kMaxRefHeight (too deep for the
-// traversal stack, or a cycle) sets bit 8; a leaf whose nShape is not a shape index sets bit 16.
+// traversal stack, or a cycle) sets bit 8; a leaf whose nShape is not a shape index sets bit 16.  Every `every`-th
+// leaf's box goes into the blur sums err[2] and err[3].
 constexpr int kMaxRefHeight = 62;
-__global__ void k_ref_height(const BVHNodeGPU *btl, const int *par, int n, unsigned *err) {
+__global__ void k_ref_height(const BVHNodeGPU *btl, const int *par, int n, int every, unsigned *err) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
+    if (k % every == 0) {
+        const Bound b = load_bound(&btl[k].bound);
+        BlurSums s;
+        s.add(b.min_x, b.min_y, b.min_z, b.max_x, b.max_y, b.max_z);
+        atomicAdd(reinterpret_cast<float *>(err) + 2, s.exact);
+        atomicAdd(reinterpret_cast<float *>(err) + 3, s.wide);
+    }
     if ((unsigned)btl[k].nShape >= (unsigned)n) atomicOr(err, 16u);
     int p = par[n - 1 + k], d = 1;
     while (p > 0 && d <= kMaxRefHeight) {
@@ -1420,13 +1359,13 @@ int convert_bvh_ref_into(ptgpu_ctx *ctx, const Shape *d_shapes, int n, const BVH
         int *par = parents;
         unsigned *err = reinterpret_cast<unsigned *>(par + (2 * n - 1));
         PT_TRY(fill_u32(ctx->stream, par, 0xFFFFFFFFu, (size_t)(2 * n - 1)));
-        PT_TRY(fill_u32(ctx->stream, err, 0u, 2));
+        PT_TRY(fill_u32(ctx->stream, err, 0u, 4));
         hipLaunchKernelGGL(k_ref_parents, dim3((n + 254) / 256), dim3(256), 0, ctx->stream, d_btn, n, par, err);
         PT_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_ref_height, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, d_btl, par, n, err);
+        hipLaunchKernelGGL(k_ref_height, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, d_btl, par, n, (n + 63) / 64, err);
         PT_HIP(hipGetLastError());
-        unsigned h_err[2] = {0, 0};
-        PT_HIP(hipMemcpyAsync(h_err, err, 8, hipMemcpyDeviceToHost, ctx->stream));
+        unsigned h_err[4] = {0, 0, 0, 0};
+        PT_HIP(hipMemcpyAsync(h_err, err, 16, hipMemcpyDeviceToHost, ctx->stream));
         PT_HIP(hipStreamSynchronize(ctx->stream));
         PT_CHECK(!(h_err[0] & 3u), PTGPU_ERR_INVALID, "btn/btl: %s",
                  (h_err[0] & 1u) ? "a child index is out of range" : "a node has two parents (not a tree)");
@@ -1435,6 +1374,9 @@ int convert_bvh_ref_into(ptgpu_ctx *ctx, const Shape *d_shapes, int n, const BVH
         PT_CHECK(!(h_err[0] & 8u), PTGPU_ERR_UNSUPPORTED, "btn/btl: tree deeper than %d levels (or cyclic)",
                  kMaxRefHeight);
         acc->depth = (int)h_err[1];
+        float sums[2];
+        std::memcpy(sums, h_err + 2, 8);
+        acc->blurs = blurred(sums[0], sums[1]) ? 1 : 0;
     } else {
         PT_CHECK(n == 1, PTGPU_ERR_INVALID, "shapeCnt %d < 1", n);
         int ns = -1;
@@ -1560,7 +1502,7 @@ static LaunchShapes launch_shapes(const ptgpu_ctx *ctx, const DevAccel &acc, int
 
 static bool walks_half(const ptgpu_ctx *ctx, const DevAccel &acc) {
     return (ctx->engine == 0 || ctx->engine == 3) && acc.mode != PTGPU_ACCEL_NONE && acc.root >= 0 && ctx->wide == 2 &&
-           acc.nodes4h && stack_for_wide(acc, ctx->stack_min) > 0;
+           acc.nodes4h && !acc.blurs && stack_for_wide(acc, ctx->stack_min) > 0;
 }
 
 bool launch_spreads(const ptgpu_ctx *ctx, const DevAccel &acc, int pixels) {
@@ -1696,7 +1638,7 @@ int launch_trace(ptgpu_ctx *ctx, const DevAccel &acc, unsigned int shapeCnt, con
     if (n <= 0) return PTGPU_OK;
     PT_CHECK(!acc.height_check, PTGPU_ERR_UNSUPPORTED,
              "batch queries cannot be recorded before the tree height was read back");
-    const int sw = acc.nodes4h && acc.root >= 0 && ctx->wide == 2 ? stack_for_wide(acc, ctx->stack_min) : -1;
+    const int sw = acc.nodes4h && !acc.blurs && acc.root >= 0 && ctx->wide == 2 ? stack_for_wide(acc, ctx->stack_min) : -1;
     if (sw > 0) {
         // Few rays are spread as launch_shape spreads few pixels.  Four workgroups of the 32-entry stack on a CU
         // (five would fit: 0.80 against 0.71 ms for 20,000 shapes and a million rays); under the short stack, which
@@ -2133,7 +2075,7 @@ int launch_batch(ptgpu_ctx *ctx, BatchChannel &ch, const ptgpu_render_job *jobs,
     std::vector<unsigned> begin((size_t)njobs + 1, 0u);
     std::vector<int> jst((size_t)njobs, 0);   // each job's traversal-stack class (32, 48 or 64 entries)
     if (!ctx->capturing) PT_TRY(build_wide_many(ctx, jobs, njobs));
-    bool half = ctx->wide == 2;   // binary16 nodes only when every job's tree has them
+    bool half = ctx->wide == 2;   // binary16 nodes only when every job's tree has them and none is blurred by them
     unsigned long long total = 0;
     for (int j = 0; j < njobs; j++) {
         const ptgpu_render_job &J = jobs[j];
@@ -2157,7 +2099,7 @@ int launch_batch(ptgpu_ctx *ctx, BatchChannel &ch, const ptgpu_render_job *jobs,
         const int sw = stack_for_wide(R.acc, ctx->stack_min);
         PT_CHECK(sw > 0, PTGPU_ERR_UNSUPPORTED, "job %d: tree height %d exceeds the traversal stack", j, R.acc.depth);
         jst[(size_t)j] = sw;
-        half = half && R.acc.nodes4h;
+        half = half && R.acc.nodes4h && !R.acc.blurs;
         if (J.bvh) {
             if (J.bvh->lights_for != (int)a->lightCnt) {
                 PT_TRY(build_light_list(ctx, a->shapes, (int)a->shapeCnt, (int)a->lightCnt, J.bvh->lights,

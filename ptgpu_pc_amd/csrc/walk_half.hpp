@@ -7,6 +7,7 @@
 // checked again.
 #pragma once
 
+#include "half_bounds.hpp"
 #include "render_device.hpp"
 
 namespace ptgpu {
