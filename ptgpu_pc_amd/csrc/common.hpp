@@ -157,10 +157,11 @@ struct BatchChannel {
     size_t pinned_bytes = 0;
     hipEvent_t copied = nullptr;   // the last table upload from `pinned` has finished
     hipEvent_t ready = nullptr;    // scene preparation on the context's stream, waited on by `stream`
-    // jobs are rendered in one launch per traversal-stack class; the classes after the first run on
-    // these streams, forked from and joined back into `stream` (default priority, created on first use)
-    hipStream_t sub[2] = {nullptr, nullptr};
-    hipEvent_t fork = nullptr, join[2] = {nullptr, nullptr};
+    // the trees of the deepest traversal-stack class are rendered in a launch of their own; where there are others
+    // too, their launch runs on this stream, forked from and joined back into `stream` (default priority, created
+    // on first use)
+    hipStream_t sub = nullptr;
+    hipEvent_t fork = nullptr, join = nullptr;
     void release();
 };
 }  // namespace ptgpu
@@ -200,11 +201,11 @@ struct ptgpu_ctx {
     int quad = 16;      // per-lane-state megakernel, binary16 nodes: traversing lanes at or below which four lanes share a query
     int batch_regroup = 40;
     int blocks_per_cu = ptgpu::kBlocksPerCu;   // single-frame renders
-    bool blocks_auto = true;      // "blocks_per_cu" 0, the default: the launch picks (launch_shape, render.hip)
+    bool blocks_auto = true;      // "blocks_per_cu" 0, the default: the launch picks (launch_shapes, render.hip)
     int batch_blocks_per_cu = 3;  // batched renders: throughput-bound, more waves per SIMD
     int wide = 2;        // per-lane-state megakernel: 0 binary nodes, 1 four-wide, 2 four-wide binary16 (when they exist)
-    int stack_min = 0;
-    int short_stack = 1;  // 48-entry binary16 walks on the 36-entry class (0 off; 2 every binary16 walk on 8 entries, a test)   // smallest traversal stack class a render or query launch uses (0: the tree's height decides)
+    int stack_min = 0;    // smallest traversal stack class a render or query launch uses (0: the tree's height decides)
+    int short_stack = 1;  // 48-entry binary16 walks on the 36-entry class (0 off; 2 every binary16 walk on 8 entries, a test)
     void *wf_workspace = nullptr;
     // scratch for raw-layout renders and light lists
     ptgpu::DevBuf tmp_nodes, tmp_nodes4, tmp_prims, tmp_lights, tmp_scan, tmp_counter;

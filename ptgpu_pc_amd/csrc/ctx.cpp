@@ -51,14 +51,11 @@ void BatchChannel::release() {
     if (copied) (void)hipEventDestroy(copied);
     if (ready) (void)hipEventDestroy(ready);
     copied = ready = nullptr;
-    for (int i = 0; i < 2; i++) {
-        if (sub[i]) (void)hipStreamDestroy(sub[i]);
-        if (join[i]) (void)hipEventDestroy(join[i]);
-        sub[i] = nullptr;
-        join[i] = nullptr;
-    }
+    if (sub) (void)hipStreamDestroy(sub);
+    if (join) (void)hipEventDestroy(join);
     if (fork) (void)hipEventDestroy(fork);
-    fork = nullptr;
+    sub = nullptr;
+    fork = join = nullptr;
 }
 
 }  // namespace ptgpu

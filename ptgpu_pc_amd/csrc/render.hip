@@ -40,7 +40,7 @@ struct RenderJob {
     unsigned *pixels;
 };
 
-// A single-frame launch's shape (launch_shape): workgroups that work, lanes of a wave that take pixels; the others help
+// A single-frame launch's shape (launch_shapes): workgroups that work, lanes of a wave that take pixels; the others help
 // in the sparse phase.
 struct LaunchShape {
     int blocks, lanes;
@@ -437,7 +437,6 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
         __syncthreads();
     }
     // frame fields: the launch's own, or (batch) the lane's job's
-#define JF(field) to_gmem(MULTI ? P.jobs[jb].field : P.field)
     int jb = 0;
     // batch: the lane's job's fields that every shading pass reads, kept in registers from the pixel
     // claim on (a field read through the job table is one more dependent load)
@@ -447,8 +446,6 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
     // and those every new sample reads
     const gmem<const Camera> *j_camera = to_gmem(P.camera);
     int j_width = P.width, j_height = P.height, j_spp = P.spp, j_currentSample = P.currentSample;
-#define JSHAPES (MULTI ? from_gmem(j_shapes) : P.shapes)
-#define JFR(field) (MULTI ? j_##field : P.field)
     // the tree of the lane's current query (uniform for a single frame)
     const gmem<const TNode> *t_nodes = to_gmem(P.acc.nodes);
     const gmem<const TNode4> *t_nodes4 = to_gmem(P.acc.nodes4);
@@ -537,7 +534,7 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
         rad = add3(rad, Ld);
         rd = nl;
         depth++;
-        if (depth > JFR(max_depth)) {
+        if (depth > (MULTI ? j_max_depth : P.max_depth)) {
             st = kEnded;
         } else {
             n_closest++;
@@ -768,8 +765,8 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
                         s1 = to_gmem(MULTI ? P.jobs[jb].seeds : args->seeds)[2 * gid + 1];
                         k = 0;
                         if ((MULTI ? j_currentSample : args->currentSample) > 0) {
-                            const gmem<const float> *cv =
-                                reinterpret_cast<const gmem<const float> *>(to_gmem(MULTI ? P.jobs[jb].colors : args->colors) + (H - y - 1) * W + x);
+                            const gmem<const float> *cv = reinterpret_cast<const gmem<const float> *>(
+                                to_gmem(MULTI ? P.jobs[jb].colors : args->colors) + (H - y - 1) * W + x);
                             col = mk(cv[0], cv[1], cv[2]);
                         }
                         camera_ray(MULTI ? from_gmem(j_camera) : &s_cam, s0, s1, W, H, x, y, ro, rd);
@@ -824,8 +821,9 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
                     const bool sh = !MULTI && li < n_lds_lights
                                         ? sample_light_words(s_lights + 16 * li, s_lights[16 * li + 13], s0, s1, ro,
                                                              nl, &sd, &len, &con)
-                                        : sample_light((MULTI ? from_gmem(j_shapes) : args->shapes) + (MULTI ? from_gmem(j_lights) : args->lights)[li], s0, s1, ro, nl, &sd, &len,
-                                                       &con);
+                                        : sample_light((MULTI ? from_gmem(j_shapes) : args->shapes) +
+                                                           (MULTI ? from_gmem(j_lights) : args->lights)[li],
+                                                       s0, s1, ro, nl, &sd, &len, &con);
                     li++;
                     if (!sh) continue;
                     if (shoot) {
@@ -859,7 +857,8 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
                     rad = mk(0.f, 0.f, 0.f); thr = mk(1.f, 1.f, 1.f); spec = true; depth = 0;
                     st = kSeg;
                 } else {
-                    gmem<float> *cp = reinterpret_cast<gmem<float> *>(to_gmem(MULTI ? P.jobs[jb].colors : args->colors) + (H - y - 1) * W + x);
+                    gmem<float> *cp = reinterpret_cast<gmem<float> *>(
+                        to_gmem(MULTI ? P.jobs[jb].colors : args->colors) + (H - y - 1) * W + x);
                     cp[0] = col.x; cp[1] = col.y; cp[2] = col.z;
                     gmem<unsigned> *px = to_gmem(MULTI ? P.jobs[jb].pixels : args->pixels);
                     if (px) px[y * W + x] = pack_rgba_tab(col, s_pack);
@@ -899,9 +898,6 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
             atomicAdd(args->trav_stats + 1, b);
         }
     }
-#undef JF
-#undef JSHAPES
-#undef JFR
 }
 
 // Batch queries (Intersect / IntersectP on arbitrary rays).
@@ -1640,7 +1636,7 @@ int launch_trace(ptgpu_ctx *ctx, const DevAccel &acc, unsigned int shapeCnt, con
              "batch queries cannot be recorded before the tree height was read back");
     const int sw = acc.nodes4h && !acc.blurs && acc.root >= 0 && ctx->wide == 2 ? stack_for_wide(acc, ctx->stack_min) : -1;
     if (sw > 0) {
-        // Few rays are spread as launch_shape spreads few pixels.  Four workgroups of the 32-entry stack on a CU
+        // Few rays are spread as launch_shapes spreads few pixels.  Four workgroups of the 32-entry stack on a CU
         // (five would fit: 0.80 against 0.71 ms for 20,000 shapes and a million rays); under the short stack, which
         // trees past 32 entries take, three for a batch that fills all lanes (0.64 against 0.72 ms for 65,538
         // shapes) and four for one that is spread (30,000 rays: 111 against 137 us).
@@ -2072,7 +2068,6 @@ static int build_wide_many(ptgpu_ctx *ctx, const ptgpu_render_job *jobs, int njo
 int launch_batch(ptgpu_ctx *ctx, BatchChannel &ch, const ptgpu_render_job *jobs, int njobs,
                  unsigned long long *d_ray_counter) {
     std::vector<RenderJob> table((size_t)njobs);
-    std::vector<unsigned> begin((size_t)njobs + 1, 0u);
     std::vector<int> jst((size_t)njobs, 0);   // each job's traversal-stack class (32, 48 or 64 entries)
     if (!ctx->capturing) PT_TRY(build_wide_many(ctx, jobs, njobs));
     bool half = ctx->wide == 2;   // binary16 nodes only when every job's tree has them and none is blurred by them
@@ -2121,11 +2116,9 @@ int launch_batch(ptgpu_ctx *ctx, BatchChannel &ch, const ptgpu_render_job *jobs,
         R.spp = a->spp;
         R.max_depth = a->max_depth;
         R.pixels = a->pixels;
-        begin[(size_t)j] = (unsigned)total;
         total += (unsigned long long)a->width * (unsigned long long)a->height;
         PT_CHECK(total < (1ull << 31), PTGPU_ERR_UNSUPPORTED, "batch of more than 2^31 pixels");
     }
-    begin[(size_t)njobs] = (unsigned)total;
     // At most two launches, run at once on the channel's stream and one forked from it.  The kernel's
     // registers allow three workgroups per CU and so does a 48-entry stack (50 KB), so every tree but the
     // deepest shares one launch sized for the deepest of them; trees that need 64 entries (two workgroups per
@@ -2220,9 +2213,9 @@ int launch_batch(ptgpu_ctx *ctx, BatchChannel &ch, const ptgpu_render_job *jobs,
         const Cls &K = cls[(size_t)k];
         hipStream_t s = stream;
         if (k > 0) {
-            if (!ch.sub[k - 1]) PT_HIP(hipStreamCreateWithFlags(&ch.sub[k - 1], hipStreamNonBlocking));
-            if (!ch.join[k - 1]) PT_HIP(hipEventCreateWithFlags(&ch.join[k - 1], hipEventDisableTiming));
-            s = ch.sub[k - 1];
+            if (!ch.sub) PT_HIP(hipStreamCreateWithFlags(&ch.sub, hipStreamNonBlocking));
+            if (!ch.join) PT_HIP(hipEventCreateWithFlags(&ch.join, hipEventDisableTiming));
+            s = ch.sub;
             PT_HIP(hipStreamWaitEvent(s, ch.fork, 0));
         }
         RenderParams P;
@@ -2238,7 +2231,7 @@ int launch_batch(ptgpu_ctx *ctx, BatchChannel &ch, const ptgpu_render_job *jobs,
         P.jobs = reinterpret_cast<const RenderJob *>(static_cast<char *>(d_table) + K.jo);
         P.job_begin = reinterpret_cast<const unsigned *>(static_cast<char *>(d_table) + K.bo);
         P.njobs = (int)K.jobs.size();
-            P.launch.inside.lanes = kWave;
+        P.launch.inside.lanes = kWave;
         P.depth_cap = wide_depth_cap(K.st);
         P.status = K.checks ? ctx->rec_status.as<unsigned>() : nullptr;
         const long long all = (long long)ctx->cu_count * ctx->batch_blocks_per_cu;
@@ -2260,8 +2253,8 @@ int launch_batch(ptgpu_ctx *ctx, BatchChannel &ch, const ptgpu_render_job *jobs,
 #undef PT_BATCH
         PT_HIP(hipGetLastError());
         if (k > 0) {
-            PT_HIP(hipEventRecord(ch.join[k - 1], s));
-            PT_HIP(hipStreamWaitEvent(stream, ch.join[k - 1], 0));
+            PT_HIP(hipEventRecord(ch.join, s));
+            PT_HIP(hipStreamWaitEvent(stream, ch.join, 0));
         }
     }
     return PTGPU_OK;

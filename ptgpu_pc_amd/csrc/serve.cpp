@@ -410,25 +410,17 @@ int ptgpu_server_tick(ptgpu_server *s, int *n_active, int *n_queued) {
         }
     }
     if (!s->jobs.empty()) {
-        // lanes take pixels in job order: the longest per-pixel chains (most samples this launch, then the
-        // largest frames) go first, so the launch does not end waiting on a long chain started late
-        std::vector<size_t> order(s->jobs.size());
-        for (size_t i = 0; i < order.size(); i++) order[i] = i;
-        std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) {
-            const ptgpu_render_args &x = s->jobs[a].args, &y = s->jobs[b].args;
-            if (x.spp != y.spp) return x.spp > y.spp;
-            return (long long)x.width * x.height > (long long)y.width * y.height;
+        // the order in which the launch's frames are reported when it ends (launch_batch orders their pixels itself):
+        // most samples first, then the largest
+        s->flight[c] = s->job_slots;
+        std::stable_sort(s->flight[c].begin(), s->flight[c].end(), [](const Slot *a, const Slot *b) {
+            if (a->step != b->step) return a->step > b->step;
+            return (long long)a->r.width * a->r.height > (long long)b->r.width * b->r.height;
         });
-        std::vector<ptgpu_render_job> sorted;
-        sorted.reserve(order.size());
-        for (size_t i : order) {
-            sorted.push_back(s->jobs[i]);
-            s->flight[c].push_back(s->job_slots[i]);
-            s->job_slots[i]->in_flight = true;
-        }
+        for (Slot *sl : s->flight[c]) sl->in_flight = true;
         if (!s->ch[c].stream) PT_HIP(hipStreamCreateWithFlags(&s->ch[c].stream, hipStreamNonBlocking));
         if (!s->done[c]) PT_HIP(hipEventCreateWithFlags(&s->done[c], hipEventDisableTiming));
-        PT_TRY(launch_batch(s->ctx, s->ch[c], sorted.data(), (int)sorted.size(), s->rays.as<unsigned long long>()));
+        PT_TRY(launch_batch(s->ctx, s->ch[c], s->jobs.data(), (int)s->jobs.size(), s->rays.as<unsigned long long>()));
         PT_HIP(hipEventRecord(s->done[c], s->ch[c].stream));
         s->launched_at[c] = ++s->launches;
     } else {
