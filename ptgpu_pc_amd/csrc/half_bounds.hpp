@@ -33,8 +33,7 @@ __device__ __forceinline__ unsigned short half_up(float x) {
 
 // Do binary16 bounds blur this tree?  They are absolute, so a scene far from the origin (or past 65,504) has
 // boxes a binary16 step wide, whatever its shapes' size, and a walk of them visits much of the tree.  Each lane
-// widens the leaf boxes of one node, spread evenly over the tree, and the wave compares the areas' sums (BlurSums
-// takes one leaf box; several waves may add theirs).  At a sum over four times the exact one the walks of binary16
+// widens the leaf boxes of one node, spread evenly over the tree, and the wave compares the areas' sums.  At a sum over four times the exact one the walks of binary16
 // and binary32 boxes cost alike (100,000 rays; the scene moved by 16: 1,002-shape soup 67 us here against 71 over binary
 // nodes, 327,692-shape mesh 413 against 236; by 256: 256 against 73 us, 146 against 0.24 ms; a 256x256 frame of a
 // 20,002-shape soup moved by 16, binary16 / binary32 four-wide nodes: 0.73 / 0.69 ms, by 256: 21.2 / 0.75).
@@ -49,6 +48,14 @@ struct BlurSums {
     }
 };
 __host__ __device__ inline bool blurred(float exact, float wide) { return wide > 4.f * exact; }
+// of a wave's sums
+__device__ __forceinline__ bool half_blurs(BlurSums s) {
+    for (int x = 1; x < kWave; x <<= 1) {
+        s.exact += __shfl_xor(s.exact, x);
+        s.wide += __shfl_xor(s.wide, x);
+    }
+    return blurred(s.exact, s.wide);
+}
 // by one wave
 __device__ __forceinline__ bool half_blurs(const TNode *nodes, int nnodes) {
     BlurSums s;
@@ -57,11 +64,7 @@ __device__ __forceinline__ bool half_blurs(const TNode *nodes, int nnodes) {
         if (t.r.x < 0 && t.r.x != kEmptyRef) s.add(t.a.x, t.a.y, t.a.z, t.a.w, t.b.x, t.b.y);
         if (t.r.y < 0 && t.r.y != kEmptyRef) s.add(t.b.z, t.b.w, t.c.x, t.c.y, t.c.z, t.c.w);
     }
-    for (int x = 1; x < kWave; x <<= 1) {
-        s.exact += __shfl_xor(s.exact, x);
-        s.wide += __shfl_xor(s.wide, x);
-    }
-    return blurred(s.exact, s.wide);
+    return half_blurs(s);
 }
 
 }  // namespace ptgpu

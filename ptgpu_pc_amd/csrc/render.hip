@@ -144,7 +144,7 @@ __device__ __forceinline__ int claimed_pixel(const RenderParams &P, unsigned m) 
 // The kernel's arguments, to be read where they are used: the shading pass of the per-lane-state kernel reads some
 // forty words of them, which the compiler would load once and keep, and then has no scalar register left for
 // the traversal loop (32 of them were spilled to lanes of a vector register, and 12 vector registers to scratch;
-// now 11 and 7).  1024x768x16 of the 327,692-shape mesh 18.2 -> 17.75 ms, 640x480 of the 65,538-shape soup by
+// so read, 7 and 8).  1024x768x16 of the 327,692-shape mesh 18.2 -> 17.75 ms, 640x480 of the 65,538-shape soup by
 // RadianceGPU 2.25 -> 2.09, 97x61 of a 332-shape mesh 0.265 -> 0.250.
 __device__ __forceinline__ cmem<RenderParams> *launch_args() {
     auto *p = (cmem<RenderParams> *)__builtin_amdgcn_kernarg_segment_ptr();
@@ -1195,19 +1195,19 @@ __global__ void k_ref_parents(const BVHNodeGPU *btn, int n, int *par, unsigned *
 
 // Height of that tree: the longest walk from a leaf up to the root (node 0), in edges, into err[1].
 // A leaf no node points at sets err[0] bit 4; a walk longer than kMaxRefHeight (too deep for the
-// traversal stack, or a cycle) sets bit 8; a leaf whose nShape is not a shape index sets bit 16.  Every `every`-th
-// leaf's box goes into the blur sums err[2] and err[3].
+// traversal stack, or a cycle) sets bit 8; a leaf whose nShape is not a shape index sets bit 16.  err[2]: whether
+// binary16 bounds blur the tree, from 64 leaves spread over it (half_blurs).
 constexpr int kMaxRefHeight = 62;
-__global__ void k_ref_height(const BVHNodeGPU *btl, const int *par, int n, int every, unsigned *err) {
+__global__ __launch_bounds__(256) void k_ref_height(const BVHNodeGPU *btl, const int *par, int n, unsigned *err) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    if (k % every == 0) {
-        const Bound b = load_bound(&btl[k].bound);
+    if (k < kWave) {
+        const Bound b = load_bound(&btl[(int)((long long)k * n / kWave)].bound);
         BlurSums s;
         s.add(b.min_x, b.min_y, b.min_z, b.max_x, b.max_y, b.max_z);
-        atomicAdd(reinterpret_cast<float *>(err) + 2, s.exact);
-        atomicAdd(reinterpret_cast<float *>(err) + 3, s.wide);
+        const bool blurs = half_blurs(s);
+        if (k == 0) err[2] = blurs ? 1u : 0u;
     }
+    if (k >= n) return;
     if ((unsigned)btl[k].nShape >= (unsigned)n) atomicOr(err, 16u);
     int p = par[n - 1 + k], d = 1;
     while (p > 0 && d <= kMaxRefHeight) {
@@ -1355,13 +1355,13 @@ int convert_bvh_ref_into(ptgpu_ctx *ctx, const Shape *d_shapes, int n, const BVH
         int *par = parents;
         unsigned *err = reinterpret_cast<unsigned *>(par + (2 * n - 1));
         PT_TRY(fill_u32(ctx->stream, par, 0xFFFFFFFFu, (size_t)(2 * n - 1)));
-        PT_TRY(fill_u32(ctx->stream, err, 0u, 4));
+        PT_TRY(fill_u32(ctx->stream, err, 0u, 2));
         hipLaunchKernelGGL(k_ref_parents, dim3((n + 254) / 256), dim3(256), 0, ctx->stream, d_btn, n, par, err);
         PT_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_ref_height, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, d_btl, par, n, (n + 63) / 64, err);
+        hipLaunchKernelGGL(k_ref_height, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, d_btl, par, n, err);
         PT_HIP(hipGetLastError());
-        unsigned h_err[4] = {0, 0, 0, 0};
-        PT_HIP(hipMemcpyAsync(h_err, err, 16, hipMemcpyDeviceToHost, ctx->stream));
+        unsigned h_err[3] = {0, 0, 0};
+        PT_HIP(hipMemcpyAsync(h_err, err, 12, hipMemcpyDeviceToHost, ctx->stream));
         PT_HIP(hipStreamSynchronize(ctx->stream));
         PT_CHECK(!(h_err[0] & 3u), PTGPU_ERR_INVALID, "btn/btl: %s",
                  (h_err[0] & 1u) ? "a child index is out of range" : "a node has two parents (not a tree)");
@@ -1370,9 +1370,7 @@ int convert_bvh_ref_into(ptgpu_ctx *ctx, const Shape *d_shapes, int n, const BVH
         PT_CHECK(!(h_err[0] & 8u), PTGPU_ERR_UNSUPPORTED, "btn/btl: tree deeper than %d levels (or cyclic)",
                  kMaxRefHeight);
         acc->depth = (int)h_err[1];
-        float sums[2];
-        std::memcpy(sums, h_err + 2, 8);
-        acc->blurs = blurred(sums[0], sums[1]) ? 1 : 0;
+        acc->blurs = (int)h_err[2];
     } else {
         PT_CHECK(n == 1, PTGPU_ERR_INVALID, "shapeCnt %d < 1", n);
         int ns = -1;
@@ -1471,12 +1469,17 @@ static int stack_for(const DevAccel &acc, int least) {
 //     on four per CU: 443, 161 / 411, 185 / 428, 296; 180x180 of it, 64 / eight on four per CU: 452, 167 / 479, 353;
 //     150x150 of the 20,492-shape mesh, 64 / eight: 487, 184 / 367, 201; 100x100, eight / four: 329, 126 / 306, 136.
 //   * Larger frames get four workgroups per CU (what the registers and the stack leave room for), but a
-//     frame of fewer than two pixels a lane whose camera is outside the scene's box keeps two.
-//     Seen from inside, every pixel's path is long and more waves
-//     keep the SIMDs busy: 1024x768x16 of the 327,692-shape mesh, two / four a CU: 28.8 / 18.5 ms.  From
-//     outside, much of the frame is background and the few long paths decide: on two a CU they run with
-//     fewer neighbours and lanes whose pixel was background take another (512x512x8 of the 65,538-shape
-//     soup, two / four: 5.1 / 5.7 ms; at 1024x1024x4, 6.9 / 5.0 ms).
+//     frame of fewer than two pixels a lane (524,288 on 256 CUs) whose camera is outside the scene's box keeps
+//     two.  Seen from inside, every pixel's path is long and more waves keep the SIMDs busy: 1024x768x16 of the
+//     327,692-shape mesh, two / four a CU: 28.8 / 18.5 ms.  From outside, four are faster for a frame alone and
+//     two for frames in flight, where another frame fills the drain and a build finds room, and the more so the
+//     smaller the frame: the line lies where what the one loses is about what the other wins.  Two / four a CU,
+//     8 spp, alone and three in flight (ms): 65,538-shape soup at 512x512 5.09 / 4.97 and 2.86 / 3.57, 720x720
+//     6.93 / 6.51 and 4.15 / 5.50, above the line 800x800 8.04 / 6.78 and 4.91 / 6.16, 1024x1024 12.1 / 8.8 and
+//     7.54 / 8.16; seen from further off, 512x512 7.36 / 6.00 and 4.43 / 5.38, 1024x768 16.4 / 11.4 and 10.4 / 11.1;
+//     the 20,482-shape mesh from outside, 512x512 1.90 / 1.74 and 1.05 / 1.10, 720x720 2.93 / 2.59 and 1.69 / 1.79,
+//     800x800 3.55 / 2.93 and 2.06 / 2.11; a 1,282-shape one at 512x512 1.49 / 1.29 and 0.82 / 0.81.  A caller who
+//     keeps frames in flight sets two, at any size (900x600 of the soup: 3.2 against 4.8 ms).
 static LaunchShapes launch_shapes(const ptgpu_ctx *ctx, const DevAccel &acc, int total, bool automatic, bool share) {
     const int cus = ctx->cu_count;
     const bool deep = stack_for_wide(acc, 0) != 32;

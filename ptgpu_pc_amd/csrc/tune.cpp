@@ -150,9 +150,9 @@ int autotune_frame(ptgpu_ctx *ctx, ptgpu_clbvh *h, const ptgpu_render_args *a, i
     float best_render = 1e30f;
     int bb = 0, br = ctx->regroup, bw = ctx->wide;
     // With frames in flight (frames_per_build 0) the next frame's render and the next tree's build start while this one
-    // runs: more than two workgroups per CU leave the build no room (it takes 0.27 ms beside two and ends with the
-    // frame beside four) and hardly speed up the frames (two in flight, two / four per CU: 512x512x8 of the
-    // 65,538-shape soup 2.98 / 3.23 ms a frame, 640x480x2 of the 20,492-shape mesh 1.13 / 1.19).  The automatic shape is
+    // runs: more than two workgroups per CU leave the build no room (it takes 0.25 ms beside two and ends with the
+    // frame beside four, which hold every register) and slow the frames down (three in flight, two / four per CU:
+    // 512x512x8 of the 65,538-shape soup 2.86 / 3.57 ms a frame, 1024x768x8 4.71 / 5.97).  The automatic shape is
     // tried there only where it spreads the frame, whose workgroups then end with their pixels.
     const int bpc_max = frames_per_build == 0 ? 2 : 4;
     const bool automatic = frames_per_build > 0 || launch_spreads(ctx, h->acc, (int)(a->width * a->height));
