@@ -272,8 +272,8 @@ def render_version() -> str:
 
 def measured_counters():
     """Counter figures of the render kernel from the committed rocprofv3 summary of this workload (or
-    None where they are another version's): HBM bytes per launch (calibrated FETCH_SIZE + WRITE_SIZE), the profile's average duration, L2
-    hit rate, VALU busy fraction and VALU lane utilisation."""
+    None where they are another version's): HBM bytes per launch (calibrated FETCH_SIZE + WRITE_SIZE), the
+    profile's average duration, L2 hit rate, VALU busy fraction and VALU lane utilisation."""
     try:
         t = json.loads(TRAFFIC_FILE.read_text())
     except (OSError, ValueError):
@@ -300,17 +300,20 @@ BUILD_BYTES_PER_PRIM = sum(STAGE_BYTES.values())   # 328 B per primitive with 8-
 TRAV_TREE_BYTES = 4 + 24 + 64
 
 
-def render_roofline(alg_bytes, avg_ms, box_tests, prim_tests, box_bytes, measured=True, kernel=None, step_ms=None):
-    """Roofline object of a render launch.  The path-tracing kernel is bound neither by HBM nor by VALU:
-    its time is the longest per-pixel chain of dependent node fetches (samples of a pixel run in order,
-    each query a chain of node visits), so `bound` says "latency"; `achieved` / `frac` price the
-    algorithmic bytes against the HBM peak as the contract asks, and `measured` gives what the counters
-    say the kernel actually moves (calibrated HBM traffic, L2 hit rate, VALU busy and lane use)."""
+def render_roofline(alg_bytes, avg_ms, box_tests, prim_tests, box_bytes, measured=True, kernel=None, step_ms=None,
+                    bound="latency", limiter="per-pixel chains of dependent node fetches (the samples of a pixel run "
+                                             "in order)"):
+    """Roofline object of a render launch.  The path-tracing kernel is not bound by HBM: an open scene's frame
+    takes as long as its longest per-pixel chain of dependent node fetches (samples of a pixel run in order,
+    each query a chain of node visits), so `bound` says "latency"; a closed scene's large frame keeps the vector
+    units busy ("vector issue").  `achieved` / `frac` price the algorithmic bytes, most of which the caches serve,
+    against the HBM peak, and `measured` gives what the counters say the kernel actually moves (calibrated HBM
+    traffic, L2 hit rate, VALU busy and lane use)."""
     achieved = alg_bytes / (avg_ms * 1e-3) / 1e9
-    out = {"bound": "latency", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+    out = {"bound": bound, "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
            "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
            "kernel": kernel or f"{RENDER_KERNEL} (path-tracing megakernel, per-lane states)",
-           "limiter": "per-pixel chains of dependent node fetches (the samples of a pixel run in order)",
+           "limiter": limiter,
            "per_launch": {"box_tests": box_tests, "prim_tests": prim_tests, "bytes_per_box_test": box_bytes,
                           "alg_bytes": alg_bytes, "avg_ms": round(avg_ms, 4)}}
     if step_ms:
@@ -1004,7 +1007,8 @@ def c3_compare(steps: int = 3, tune: bool = True, cpu: bool = False):
                   width=W3, height=H3, currentSample=0, spp=SPP3, max_depth=D3, pixels=d_pix, trav_stats=d_stats)
         box, prim = (int(x) for x in d_stats.download(np.uint64)[:2])
         alg = box_bytes * box + 36 * prim + W3 * H3 * (24 + 16 + 4)
-        return render_roofline(alg, ms, box, prim, box_bytes, measured=False)
+        return render_roofline(alg, ms, box, prim, box_bytes, measured=False, bound="vector issue",
+                               limiter="instructions of the walk's steps: every pixel of the closed box is a path")
 
     def render(bvh, kd):
         best, rays = 1e9, 0
@@ -1047,7 +1051,7 @@ def c3_compare(steps: int = 3, tune: bool = True, cpu: bool = False):
         out[name] = {"build_ms_host": round(build_ms, 1), "render_ms": round(ms, 2),
                      "mrays_s": round(rays / ms / 1e3, 1), "rays": rays,
                      "pixels_identical": pix.tobytes() == out["_pix"].tobytes(), **kd.stats(),
-                     "roofline": roofline_of(None, kd, ms, 32)}   # KD leaves share primitives: fp32 four-wide nodes
+                     "roofline": roofline_of(None, kd, ms, 16)}
         kd.close()
     out.pop("_pix")
     tuning = None
