@@ -374,9 +374,9 @@ __global__ __launch_bounds__(256) void k_render(RenderParams P) {
 //     shadow ray starts the next query between passes;
 //   * divisions and roots are correctly rounded in three and five instructions (rcp_exact, sqrt_exact);
 //   * a wave with few queries left shares them among its lanes (half_sparse).
-// Times before and after, one frame: 512x512x8 spp of the 65,538-shape soup 7.75 -> 5.2 ms; 1024x768x16 of the
-// 327,692-shape mesh 36.0 -> 17.6 ms; 640x480x4 of a 20,492-shape SAH KD tree 5.0 -> 2.7 ms; 97x61x1 of a
-// 332-shape mesh 0.57 -> 0.25 ms.
+// Times before and after, one frame: 512x512x8 spp of the 65,538-shape soup 7.75 -> 5.1 ms; 1024x768x16 of the
+// 327,692-shape mesh 36.0 -> 17.5 ms; 640x480x4 of a 20,492-shape SAH KD tree 5.0 -> 2.7 ms; 97x61x1 of a
+// 332-shape mesh 0.57 -> 0.22 ms.
 enum : int {
     kNeed = 0,    // wants a pixel
     kTrav = 1,    // traversing
@@ -1042,7 +1042,7 @@ __global__ __launch_bounds__(256) void k_light_count(const Shape *shapes, int n,
 }
 // The list itself and its length; a block starts after the emitters of the blocks before it (a single one needs no
 // counts).  What bounds it for one frame's scene is its launch and two round trips: with the flags loaded one
-// by one, a scan kernel between and the length read back, the nine shapes of a 256x256x4 frame took 42 of its 192 us for the list.
+// by one, a scan kernel between and the length read back, the nine shapes of a 256x256x4 frame took 42 of its then 192 us for the list.
 __global__ __launch_bounds__(256) void k_light_write(const Shape *shapes, int n, const unsigned *counts, int cap,
                                                      int *out, unsigned *total) {
     __shared__ unsigned s_w[4][16], s_run;

@@ -393,8 +393,9 @@ __device__ bool brute_any(const Prim *prims, int n, f3 o, f3 d, float maxt, unsi
 // The same for up to kBrutePrims primitives held in LDS, four tests at a time.  A frame of 256x256 pixels is one
 // wave per SIMD, so what bounds it is each test's chain of a load, a root and branches; four spheres tested
 // without a branch share one wait and fill each other's latencies.  256x256x4 spp of nine spheres, the whole
-// call: 242 -> 192 us (one scalar load a test: 223 us).  256 triangles: 1.33 -> 1.26 ms; past 256 the scalar
-// loop is as fast (257: 1.26 ms).
+// call: 242 -> 192 us (one scalar load a test: 223 us); later, with the light list in one launch, 150, and with
+// the last group's empty places at -infinity, which the four-wide test misses by itself, 134.  256 triangles:
+// 1.33 -> 1.26 ms; past 256 the scalar loop is as fast (257: 1.26 ms).
 constexpr int kBrutePrims = 256;
 template <int CAP>
 struct BruteScene {
