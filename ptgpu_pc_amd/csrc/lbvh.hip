@@ -451,7 +451,8 @@ int clbvh_prepare_traversal(ptgpu_clbvh *h, bool recording, bool exact, bool wid
             bound = kRecordedHeightDefault;
         h->acc.depth = bound;
         h->acc.height_check = misc_counters(h) + 9;
-    } else if (h->height_pending || (h->blurs_pending && exact && !recording && !h->ctx->capturing)) {
+    } else if (h->height_pending || (h->blurs_pending && !recording && !h->ctx->capturing &&
+                                     (exact || h->blurs_age < 0 || (!h->speculate && h->blurs_age >= kBlursAge)))) {
         unsigned w[3] = {0, 0, 0};   // error word, blurs, height
         if (h->blurs_pending) {
             hipLaunchKernelGGL(k_blurs, dim3(1), dim3(kWave), 0, h->ctx->stream, (const TNode *)h->acc.nodes, h->acc.nnodes,
@@ -464,6 +465,7 @@ int clbvh_prepare_traversal(ptgpu_clbvh *h, bool recording, bool exact, bool wid
                  "traversal-tree list overflow)", w[0]);
         if (h->blurs_pending) h->acc.blurs = (int)w[1];
         h->blurs_pending = false;
+        h->blurs_age = 0;
         if (h->height_pending) {
             h->acc.depth = (int)w[2];
             h->acc.height_check = nullptr;
@@ -534,6 +536,7 @@ void ptgpu::clbvh_mark_built(ptgpu_clbvh *h) {
     }
     h->height_pending = h->trav_topology == 1 && n >= 2;
     h->blurs_pending = n >= 2;
+    if (h->blurs_age >= 0) h->blurs_age++;
 }
 
 extern "C" {

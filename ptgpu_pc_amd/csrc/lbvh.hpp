@@ -13,6 +13,10 @@ namespace ptgpu {
 int clbvh_prepare_traversal(ptgpu_clbvh *h, bool recording = false, bool exact = false, bool wide = true);
 // Height bound of a traversal recorded before the height could be read back: the height last read
 // for a build of the same kind (plain or optimised) plus this margin, or the default without one.
+// An index-keyed tree's height is known without a read-back, so its frames wait for whether binary16 bounds blur it at the
+// first build and at every 64th only (waiting at each costs a 97x61 frame with its rebuild 40 of 214 us); others take
+// the last answer.  A handle set to skip the read-back waits for the first alone.
+constexpr int kBlursAge = 64;
 constexpr int kRecordedHeightMargin = 4;
 constexpr int kRecordedHeightDefault = 41;   // the deepest tree the 64-entry four-wide stack walks
 int clbvh_export_optimized(ptgpu_clbvh *h);
@@ -55,6 +59,7 @@ struct ptgpu_clbvh {
     int trav_topology = 1;    // traversal tree: 0 = the exported index-keyed tree, 1 = Morton-keyed LBVH
     bool height_pending = false;
     bool blurs_pending = false;   // acc.blurs is the previous build's
+    int blurs_age = -1;           // builds since an answer was read (-1: none was)
     int known_height[2] = {0, 0};   // last heights read back: [0] plain build, [1] after optimize
     bool speculate = false;         // no read-back once a height is known: a bound, checked on the device
     unsigned *sorted = nullptr;

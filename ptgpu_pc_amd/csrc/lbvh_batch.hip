@@ -346,6 +346,7 @@ int build_batch(ptgpu_ctx *ctx, ptgpu_clbvh *const *hs, int ns) {
         if (h->blurs_pending && h_out[ns + s] == 0) {
             h->acc.blurs = (int)h_out[2 * ns + s];
             h->blurs_pending = false;
+            h->blurs_age = 0;
         }
         sort_err |= h_out[ns + s] != 0;
     }
