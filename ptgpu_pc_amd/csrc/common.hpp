@@ -99,6 +99,8 @@ struct DevAccel {
     int mode = PTGPU_ACCEL_NONE;
     int blurs = 0;         // 1: binary16 bounds blur the tree (half_bounds.hpp): its walks take binary32 boxes.  A tree whose
                            // first walk could not wait for the answer keeps that of the build before it.
+    int long_walks = 0;    // 1: a KD tree, an index-keyed LBVH or a caller's tree, whose queries have more steps or shapes
+                           // than a Morton-keyed LBVH's (launch_shapes)
     int leaf_runs = 0;     // 1: every leaf range is disjoint and its last Prim carries kLastInLeaf
     // A traversal recorded into a graph right after a build, before its height could be read back:
     // `depth` is then a bound, and the build's status words (error word, -, height) are checked

@@ -379,6 +379,7 @@ int upload_device(ptgpu_kdtree *T) {
     A.leaf_runs = 1;
     A.blurs = half_blurs_kd(T->nodes) ? 1 : 0;
     A.mode = PTGPU_ACCEL_KD;
+    A.long_walks = 1;
     const KNode &root = T->nodes[0];
     if (root.leaf) {
         A.root = ~root.start;

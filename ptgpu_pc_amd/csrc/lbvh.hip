@@ -534,6 +534,7 @@ void ptgpu::clbvh_mark_built(ptgpu_clbvh *h) {
         h->acc.root_cnt = 1;
         h->acc.depth = 0;
     }
+    h->acc.long_walks = h->trav_topology == 0 && !h->optimized;
     h->height_pending = h->trav_topology == 1 && n >= 2;
     h->blurs_pending = n >= 2;
     if (h->blurs_age >= 0) h->blurs_age++;

@@ -1371,6 +1371,7 @@ int convert_bvh_ref_into(ptgpu_ctx *ctx, const Shape *d_shapes, int n, const BVH
                  kMaxRefHeight);
         acc->depth = (int)h_err[1];
         acc->blurs = (int)h_err[2];
+        acc->long_walks = 1;
     } else {
         PT_CHECK(n == 1, PTGPU_ERR_INVALID, "shapeCnt %d < 1", n);
         int ns = -1;
@@ -1463,11 +1464,13 @@ static int stack_for(const DevAccel &acc, int least) {
 //     From outside much of a frame is background, so it is spread over all the waves that four workgroups per CU
 //     hold, up to 8 pixels each (16 waves per CU: 32,768 pixels on 256 CUs): 180x180 of the 65,538-shape soup, 64
 //     pixels a wave / eight: 831, 311 / 466, 213; at 256x256 eight halve the rate of a 20,482-shape mesh in flight.
-//     Inside, every path is long and frames in flight need the room: up to three workgroups per CU for one and two
-//     pixels a wave, two for four and eight, where deep trees (many steps to save) may have three.  97x61 of the
-//     332-shape mesh, 64 / two: 399, 140 / 236, 118; 128x128 of the 5,132-shape mesh, 64 / eight on two per CU / four
-//     on four per CU: 443, 161 / 411, 185 / 428, 296; 180x180 of it, 64 / eight on four per CU: 452, 167 / 479, 353;
-//     150x150 of the 20,492-shape mesh, 64 / eight: 487, 184 / 367, 201; 100x100, eight / four: 329, 126 / 306, 136.
+//     Inside, every path is long.  Deep trees, KD trees and index-keyed or callers' trees, whose queries have many
+//     steps or shapes to share, are spread alike; where walks are short (Morton-keyed trees of the 32-entry stack)
+//     sharing saves one frame little and costs frames in flight much, so four pixels a wave end at 12,288 and eight
+//     at 20,480.  64 pixels a wave / the share chosen: 6,592 pixels of a 332-shape mesh 399, 144 / 243, 141; 16,384 of a 5,132-shape
+//     one 438, 170 / 413, 203, above the line 22,500 439, 174 (eight: 431, 265); 28,224 of a 20,492-shape one, deep,
+//     490, 193 / 369, 255; 22,500 of the 5,132-shape one index-keyed 644, 259 / 496, 298, as a SAH KD tree
+//     494, 188 / 356, 208, as a mean-split one 719, 269 / 379, 218.
 //   * Larger frames get four workgroups per CU (what the registers and the stack leave room for), but a
 //     frame of fewer than two pixels a lane (524,288 on 256 CUs) whose camera is outside the scene's box keeps
 //     two.  Seen from inside, every pixel's path is long and more waves keep the SIMDs busy: 1024x768x16 of the
@@ -1493,8 +1496,11 @@ static LaunchShapes launch_shapes(const ptgpu_ctx *ctx, const DevAccel &acc, int
     }
     int in = kWave, out = kWave;
     if (share) {
-        in = total <= 12 * cus ? 1 : total <= 24 * cus ? 2 : total <= (deep ? 48 : 32) * cus ? 4 : total <= (deep ? 96 : 64) * cus ? 8 : kWave;
-        out = total <= 16 * cus ? 1 : total <= 32 * cus ? 2 : total <= 64 * cus ? 4 : total <= 128 * cus ? 8 : kWave;
+        auto lanes = [&](int four, int eight) {
+            return total <= 16 * cus ? 1 : total <= 32 * cus ? 2 : total <= four * cus ? 4 : total <= eight * cus ? 8 : kWave;
+        };
+        out = lanes(64, 128);
+        in = acc.long_walks || deep ? out : lanes(48, 80);
     }
     return LaunchShapes{shape(in, 4), shape(out, out == kWave && total < 2 * 4 * 256 * cus ? 2 : 4)};
 }

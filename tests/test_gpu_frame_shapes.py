@@ -78,10 +78,10 @@ class _Frames:
             ctx.close()
 
 
-# around the limits of each share on 256 CUs: 3072, 6144, 8192 and 12288, 16384 and 24576 pixels inside, 4096 .. 32768
-# outside
+# around the limits of each share on 256 CUs: 4096, 8192, 16384 and 32768 pixels, inside 12288 and 20480 for "mesh"
 @pytest.mark.parametrize("w,h", [(1, 3), (64, 48), (439, 7), (64, 64), (241, 17), (96, 64), (1229, 5), (2731, 3), (3277, 5), (96, 128), (4097, 3),
-                                 (192, 128), (3511, 7), (182, 180), (331, 99)])
+                                 (192, 128), (3511, 7), (182, 180), (331, 99), (128, 64), (128, 128), (160, 128),
+                                 (10241, 2), (256, 128)])
 @pytest.mark.parametrize("kind", ["mesh", "deep", "soup"])
 def test_shapes_same_bits(kind, w, h):
     say("case frame shapes", kind, w, h)
@@ -109,3 +109,43 @@ def test_spread_leaves_room(kind, w, h, contexts):
     say(f"  default {default:.4f} ms, 64 pixels a wave {fixed:.4f} ms")
     f.close()
     assert default < 1.3 * fixed
+
+
+@pytest.mark.parametrize("accel,most", [("kd", 0.75), ("kd_sah", 0.9), ("index", 0.9)])
+@pytest.mark.parametrize("w,h", [(64, 112), (129, 64), (128, 112), (260, 75), (182, 180), (331, 99)])
+def test_long_walks_share(accel, most, w, h):
+    """KD trees and index-keyed ones, seen from inside: shared up to 32,768 pixels, with the bits of 64 pixels a wave (their
+    times, 22,500 pixels of the 5,132-shape mesh: 379 against 719 us, SAH 356 / 494, index-keyed 496 / 644)."""
+    say("case long walks", accel, w, h)
+    s, lc, cam = scenes.icosphere_in_box(4, seed=3, width=w, height=h)
+    pt.update_camera(cam)
+    with pt.Context(0) as ctx:
+        d_sh = ctx.to_device(s)
+        bvh = kd = None
+        if accel == "index":
+            bvh = pt.CLBVH(ctx, d_sh, traversal="reference")
+            bvh.buildRadixTree()
+            bvh.buildBVHTree()
+        else:
+            kd = pt.KDTree(ctx, s, sah=accel == "kd_sah", max_depth=24, max_leaf=4) if accel == "kd_sah" else pt.KDTree(ctx, s)
+        seeds = ctx.to_device(default_seeds(w, h))
+        col, sd = ctx.alloc(w * h * 12, F32).zero(), ctx.alloc(w * h * 8, np.uint32)
+        args = dict(colors=col, seeds=sd, camera=ctx.to_device(cam), shapes=d_sh, shapeCnt=len(s), lightCnt=lc, width=w,
+                    height=h, spp=1, max_depth=5)
+
+        def best():
+            ms = []
+            for _ in range(12):
+                sd.copy_from(seeds)
+                ctx.record(0)
+                pt.render(ctx, bvh, kd, **args)
+                ctx.record(1)
+                ms.append(ctx.elapsed_ms(0, 1))
+            return min(ms[2:]), col.download(np.uint32).tobytes() + sd.download(np.uint32).tobytes()
+
+        default, bits = best()
+        ctx.set_tuning("blocks_per_cu", 4)
+        fixed, same = best()
+        say(f"  default {default:.4f} ms, 64 pixels a wave {fixed:.4f} ms")
+        assert bits == same
+        assert default < (most if w * h <= 32768 else 1.05) * fixed
