@@ -71,6 +71,8 @@ struct RenderParams {
     int njobs;
     const int2 *tiles;            // tiled launches (RadianceBoxGPU): tile origins; NULL renders the whole frame
     int tile_w, tile_h;
+    int slack;                    // half_slack of a tree whose height is known, for the classes that hold its walk.  (Computed in
+                                  // the kernel it made KD frames 1 to 3% slower.)
     LaunchShapes launch;
     int depth_cap;                // deepest tree the launch's stack holds (checked when acc.height_check is set)
     const float *pack_tab;        // to_int_tab's table
@@ -455,7 +457,9 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
     T.nprims = P.acc.nprims;
     T.skip = P.acc.nshapes - 1;
     int t_nnodes = P.acc.nnodes, t_root = P.acc.root;
-    int t_slack = HALF && !MULTI ? half_slack(STACK, P.acc) : 0;
+    int t_slack = P.slack;
+    if (HALF && !MULTI && (kIsShort<STACK> || P.acc.height_check))
+        t_slack = __builtin_amdgcn_readfirstlane(half_slack(STACK, P.acc));
 
     int st = (int)__lane_id() < shape.lanes ? kNeed : kIdle;
     bool drained = false;
@@ -937,7 +941,7 @@ template <int STACK, bool WAIT>
 __global__ __launch_bounds__(256, STACK <= 36 ? 4 : 2) void k_trace_half(DevAccel A, const Ray *rays, const float *maxt,
                                                                          int n, float *tout, int *idout, int *hitout,
                                                                          int any, int lanes, int regroup_max, int quad) {
-    const int slack = half_slack(STACK, A);
+    const int slack = __builtin_amdgcn_readfirstlane(half_slack(STACK, A));
     __shared__ int s_stack[STACK * 256];
     int *const stk = s_stack + threadIdx.x;
     HalfTree T;
@@ -1564,6 +1568,7 @@ int launch_render(ptgpu_ctx *ctx, const DevAccel &acc, const RenderLaunch &L) {
     P.tiles = L.tiles;
     P.tile_w = L.tile_w;
     P.tile_h = L.tile_h;
+    P.slack = 0;
     P.depth_cap = binary_depth_cap(st);
     P.status = nullptr;
     if (acc.height_check) {
@@ -1587,6 +1592,7 @@ int launch_render(ptgpu_ctx *ctx, const DevAccel &acc, const RenderLaunch &L) {
         // allocation-free entry does not ask the runtime for.
         const bool tiny = half && sw > 0 && ctx->short_stack == 2 && !L.no_alloc;
         const bool shortst = half && sw == 48 && ctx->short_stack == 1 && !L.no_alloc;
+        P.slack = sw - 3 * ((acc.depth + 2) / 2);
 #define PT_LANES(ST, STATS_, WIDE_, HALF_)                                                                      \
     hipLaunchKernelGGL((k_render_lanes<ST, STATS_, WIDE_, false, HALF_>), dim3(blocks), dim3(256), 0, ctx->stream, P)
 #define PT_LANES_W(ST, STATS_) \
