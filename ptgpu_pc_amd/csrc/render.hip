@@ -457,7 +457,7 @@ __global__ __launch_bounds__(256, HALF && !MULTI && STACK <= 36 ? 4 : HALF && ST
     T.nprims = P.acc.nprims;
     T.skip = P.acc.nshapes - 1;
     int t_nnodes = P.acc.nnodes, t_root = P.acc.root;
-    int t_slack = P.slack;
+    int t_slack = HALF && !MULTI ? P.slack : 0;   // (a batch's lanes take their job's)
     if (HALF && !MULTI && (kIsShort<STACK> || P.acc.height_check))
         t_slack = __builtin_amdgcn_readfirstlane(half_slack(STACK, P.acc));
 
